@@ -14,7 +14,7 @@ Three kinds, each through the package's public entry points:
 The systems are water boxes at the density of 32 molecules in 9.86 A, four
 states per molecule, 30 to 70 Ry, on the smallest grid with compiled transforms
 that holds the density sphere.  A real minimisation takes a few hundred steps;
-a pass runs a few dozen so that it stays short.
+a pass runs 25 to 100 so that it stays short.
 
 Results of mixed precision contexts come out of single precision transforms
 and are returned at single precision; all others are double.
@@ -51,9 +51,9 @@ def listed():
           scf=False, resid=True, monitor=True, steps=40),
         # the benchmark's system and options, both precisions
         m(name="water32-mixed", nmol=32, ecut=70.0, precision="mixed", opt="sd", scf=True,
-          autotune=True, steps=60),
+          autotune=True, steps=100),
         m(name="water32-fp64", nmol=32, ecut=70.0, precision="fp64", opt="sd", scf=True,
-          autotune=True, steps=50),
+          autotune=True, steps=80),
         # ragged state count, with the non-local projectors
         m(name="water21-fp64-kb-cg", nmol=21, ecut=60.0, precision="fp64", opt="cg", scf=True,
           nonlocal_kb=True, monitor=True, steps=30),
@@ -62,12 +62,12 @@ def listed():
           opt="sd", scf=True, steps=40),
         # the largest requests of the request loop, a ragged and a full one
         m(name="water45-mixed-cg", nmol=45, ecut=60.0, precision="mixed", opt="cg", scf=True,
-          steps=20),
+          steps=32),
         m(name="water64-fp64-cg", nmol=64, ecut=70.0, precision="fp64", opt="cg", scf=True,
-          steps=16),
+          steps=24),
         # the largest system
         m(name="water128-mixed", nmol=128, ecut=70.0, precision="mixed", opt="sd", scf=True,
-          steps=16),
+          steps=32),
         # the request loop: six sizes at once, half of them in mixed precision
         dict(name="serve-6", kind="serve", first=4, last=36, count=6, ecut=60.0, steps=25),
     ]
