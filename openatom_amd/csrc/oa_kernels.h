@@ -11,6 +11,26 @@ hipError_t grant_lds(const void* fn, size_t bytes);
 // compute units of the current device (read once per device; thread-safe)
 int cu_count();
 
+// V(r) in the lane order of the row-class R->G pass (oa_plane4.h): pairs of
+// rows (y, y + n/2), [nz][m][n/x1][n/(2m) x1] of them, float or double.
+// p == nullptr: the context's plane passes have no row classes.
+struct VPerm {
+  void* p;
+  int n, m, x1, f32;
+  __device__ __forceinline__ void put(int z, int y, int x, double v) const {
+    const int h = 2 * y >= n ? 1 : 0, r = y - h * (n >> 1);
+    const int q = r / m, cl = r - q * m, t = x / x1, j = x - t * x1, nq = n / (2 * m);
+    const size_t e = (((size_t)(z * m + cl) * (n / x1) + t) * (nq * x1) + j * nq + q) * 2 + h;
+    if (f32) ((float*)p)[e] = (float)v;
+    else ((double*)p)[e] = v;
+  }
+};
+// vp <- v ([nz][n][n])
+hipError_t vperm_set(const VPerm& vp, const double* v, int nz, hipStream_t st);
+// zero the rows y = ny/2 of every plane column of zbuf (pruned planes read them
+// in place of unpopulated frequencies): ncol columns of ny complex values
+hipError_t zero_rows(void* zbuf, size_t ncol, int ny, bool fp32, hipStream_t st);
+
 // Everything the FFT chain needs for one system (device pointers).
 struct FftCtx {
   Geom g;
@@ -55,6 +75,7 @@ struct FftCtx {
   // pass, [nst][nz][plane3_kper] complex T in the x pass's lane order; null:
   // the R->G pass recomputes psi(r) from zbuf
   void* psk;
+  void* vperm;            // V(r) as VPerm describes, for the row-class R->G pass
 };
 
 // two-factor register FFT engine (oa_fft2_*.hip): kind 0 z fwd, 1 y fwd,
@@ -63,15 +84,20 @@ struct FftCtx {
 hipError_t fft2_launch(int kind, int n, bool fp32, const FftCtx& c, hipStream_t st);
 int fft2_ntr(int n);  // transforms per workgroup for length n, 0 if not compiled
 
-// fused y+x plane passes on the two-factor engine (oa_plane3.h), square
-// planes nx == ny == n: kind 0 G->R + rho partials, 1 R->G (V psi, x and
+// fused y+x plane passes on the two-factor engine, square planes nx == ny == n
+// (oa_plane4.h by row class where c.prune is set and the length has classes,
+// else oa_plane3.h): kind 0 G->R + rho partials, 1 R->G (V psi, x and
 // y back to zout), 2 G->R writing psi(r) of c.psir_state, 3 R->G that also
 // leaves the rho partials of its c.nchunk_r chunks (V independent of rho)
 hipError_t plane3_launch(int kind, int n, bool fp32, const FftCtx& c, hipStream_t st);
 size_t plane3_smem(int n, int nplane_x, bool fp32);  // 0 if n is not compiled
 // complex elements per state and z-plane of the kept psi(r) (FftCtx::psk)
-size_t plane3_kper(int n, int nplane_x, bool fp32);  // 0 if n is not compiled
-// row parts of the G->R grid and resident workgroups per CU of both passes
+size_t plane3_kper(int n, int nplane_x, bool fp32, bool prune);  // 0 if n is not compiled
+// row classes of pruned planes of n x n points and the x factor of their lane
+// order (VPerm); 0: none
+int plane_classes(int n, bool fp32, int* x1);
+// workgroups per plane of the G->R grid and resident workgroups per CU of both
+// passes; *rho_ok: those of the R->G pass with rho, 0 if it is not compiled
 hipError_t plane3_info(int n, int nplane_x, bool fp32, bool prune, int* rowparts, int* occ_g2r,
                        int* occ_r2g, int* rho_ok);
 
@@ -137,6 +163,7 @@ struct VksArgs {
   double vol, ecut4;       // Omega; density cutoff 4 ecut_ry on |G|^2
   const double* rho;       // [nz][ny][nx]
   double* v;               // [nz][ny][nx] out: V_KS
+  VPerm vp;                // ... and in the R->G pass's order (vp.p may be null)
   double2* hx;             // [nz][nkx][ny] after the x pass
   double2* hl;             // [nz][nkx][nky] after the y pass
   const double2* vloc;     // [nkx][nky][nz] V_loc(G), zero off the sphere

@@ -720,9 +720,16 @@ hipError_t plane3_info_l(int npx, int* rowparts, int* occ_g2r, int* occ_r2g, int
   const void* g = wide ? (const void*)k3_g2r<T, X1, X2, Y1, Y2, NT, S::ROUNDS, false, L>
                        : (const void*)k3_g2r<T, X1, X2, Y1, Y2, NT, row_rounds<T, L>(), false, L>;
   const void* r = (const void*)k3_r2g<T, X1, X2, Y1, Y2, NT, VREG, false, L>;
-  // the R->G pass with rho accumulators spills at 512 threads
-  *rho_ok = r2g_rho_ok<X1, X2, NT>() && NT == kPlaneThreads ? 1 : 0;
   hipError_t e;
+  *rho_ok = 0;
+  // the R->G pass with rho accumulators spills at 512 threads
+  if constexpr (r2g_rho_ok<X1, X2, NT>() && NT == kPlaneThreads) {
+    const void* h = (const void*)k3_r2g<T, X1, X2, Y1, Y2, NT, VREG, true, L>;
+    if ((e = oa::grant_lds(h, smem)) != hipSuccess ||
+        (e = hipOccupancyMaxActiveBlocksPerMultiprocessor(rho_ok, h, NT, smem)) != hipSuccess)
+      return e;
+    *rho_ok = *rho_ok > 1 ? *rho_ok : 1;
+  }
   if ((e = oa::grant_lds(g, smem)) != hipSuccess || (e = oa::grant_lds(r, smem)) != hipSuccess)
     return e;
   if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(occ_g2r, g, NT, smem)) != hipSuccess)
@@ -808,11 +815,14 @@ hipError_t plane3_info_pr(int npx, int* rowparts, int* occ_g2r, int* occ_r2g, in
                                                                    rho_ok);
 }
 
-template <typename T, int X1, int X2, int Y1, int Y2>
+// PRUNED: pruned variants exist (lengths without row classes, oa_plane4.h)
+template <typename T, int X1, int X2, int Y1, int Y2, bool PRUNED>
 hipError_t plane3_info(int npx, bool prune, int* rowparts, int* occ_g2r, int* occ_r2g,
                        int* rho_ok) {
-  return prune ? plane3_info_pr<T, X1, X2, Y1, Y2, true>(npx, rowparts, occ_g2r, occ_r2g, rho_ok)
-               : plane3_info_pr<T, X1, X2, Y1, Y2, false>(npx, rowparts, occ_g2r, occ_r2g, rho_ok);
+  if constexpr (PRUNED)
+    if (prune)
+      return plane3_info_pr<T, X1, X2, Y1, Y2, true>(npx, rowparts, occ_g2r, occ_r2g, rho_ok);
+  return plane3_info_pr<T, X1, X2, Y1, Y2, false>(npx, rowparts, occ_g2r, occ_r2g, rho_ok);
 }
 
 template <typename T, int X1, int X2, int Y1, int Y2, bool PR>
@@ -830,10 +840,11 @@ hipError_t launch_plane3_pr(int kind, const FftCtx& c, hipStream_t st) {
 
 // c.prune (set by the host when every populated |kx|, |ky| <= (N - 1) / 4)
 // selects the variants pruned to the sphere
-template <typename T, int X1, int X2, int Y1, int Y2>
+template <typename T, int X1, int X2, int Y1, int Y2, bool PRUNED>
 hipError_t launch_plane3(int kind, const FftCtx& c, hipStream_t st) {
-  return c.prune ? launch_plane3_pr<T, X1, X2, Y1, Y2, true>(kind, c, st)
-                 : launch_plane3_pr<T, X1, X2, Y1, Y2, false>(kind, c, st);
+  if constexpr (PRUNED)
+    if (c.prune) return launch_plane3_pr<T, X1, X2, Y1, Y2, true>(kind, c, st);
+  return launch_plane3_pr<T, X1, X2, Y1, Y2, false>(kind, c, st);
 }
 
 }  // namespace oa3

@@ -6,8 +6,9 @@
 //                 CP_State_GSpacePlane.C:2646-2671)
 //   k_red_sync : redundant kx=0 points <- conj(partner)
 //                (CP_State_GSpacePlane.C:2862-3061)
-//   k_reduce_to, k_dot, k_resid, k_fill_zero: deterministic reductions and
-//   graph-safe zero fill.
+//   k_vperm    : V(r) into the lane order of the row-class R->G pass
+//   k_reduce_to, k_dot, k_resid, k_fill_zero, k_zero_rows: deterministic
+//   reductions and graph-safe zero fills.
 #include <algorithm>
 
 #include "oa_common.h"
@@ -211,6 +212,39 @@ __global__ void k_resid(const double* __restrict__ S, int n, StepDev* res) {
 
 hipError_t resid_stats(const double* S, int n, StepDev* res, hipStream_t st) {
   hipLaunchKernelGGL(k_resid, dim3(1), dim3(1024), 0, st, S, n, res);
+  return hipGetLastError();
+}
+
+__global__ void k_vperm(VPerm vp, const double* __restrict__ v, int nz) {
+  const size_t tot = (size_t)nz * vp.n * vp.n;
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot;
+       e += (size_t)gridDim.x * blockDim.x) {
+    const size_t r = e / vp.n;
+    const int x = (int)(e - r * vp.n), z = (int)(r / vp.n), y = (int)(r - (size_t)z * vp.n);
+    vp.put(z, y, x, v[e]);
+  }
+}
+
+hipError_t vperm_set(const VPerm& vp, const double* v, int nz, hipStream_t st) {
+  if (!vp.p) return hipSuccess;
+  hipLaunchKernelGGL(k_vperm, dim3(1024), dim3(256), 0, st, vp, v, nz);
+  return hipGetLastError();
+}
+
+template <typename T>
+__global__ void k_zero_rows(cpx<T>* __restrict__ z, size_t ncol, int ny) {
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < ncol;
+       e += (size_t)gridDim.x * blockDim.x)
+    z[e * ny + ny / 2] = {(T)0, (T)0};
+}
+
+hipError_t zero_rows(void* zbuf, size_t ncol, int ny, bool fp32, hipStream_t st) {
+  if (fp32)
+    hipLaunchKernelGGL(k_zero_rows<float>, dim3(1024), dim3(256), 0, st, (cpx<float>*)zbuf, ncol,
+                       ny);
+  else
+    hipLaunchKernelGGL(k_zero_rows<double>, dim3(1024), dim3(256), 0, st, (cpx<double>*)zbuf,
+                       ncol, ny);
   return hipGetLastError();
 }
 

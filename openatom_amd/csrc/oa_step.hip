@@ -154,6 +154,7 @@ struct oa_ctx {
   double2 *twx = nullptr, *twy = nullptr, *twz = nullptr;
   double *g2 = nullptr, *occ = nullptr, *dtm = nullptr, *vks = nullptr, *rho = nullptr;
   void *zbuf = nullptr, *xbuf = nullptr, *psir = nullptr, *zout = nullptr;
+  oa::VPerm vperm{};    // plane engine with row classes: V(r) for the R->G pass
   void* psk = nullptr;  // plane engine, opt.psir_keep: psi(r) between the plane passes
   double* eke_part = nullptr;
   int nblk = 0;
@@ -305,20 +306,27 @@ std::vector<double2> twiddles(int n) {
   return t;
 }
 
-// States per chunk for a grid of units x nchunk workgroups of which `slots`
-// are resident at once: minimise rounds * (states per workgroup + 1), the
-// +1 standing for a workgroup's fixed start-up cost; ties go to fewer
-// chunks.  At most max_chunks chunks.
-void pick_chunks(int units, int slots, int nst, int max_chunks, int& cs, int& nchunk) {
+// States per chunk for a grid of units x nchunk workgroups, occ resident per
+// CU.  A state costs a CU that holds k workgroups k + 1.5 units of time (fitted
+// to the plane passes: 5.6, 6.8, 8.6 us with 1, 2, 3 workgroups in FP32 at
+// 100^3; between none and 2.7 over the sizes), a workgroup half a state to
+// start; the last round runs with what is left of the grid, and a grid of few
+// rounds ends less evenly (6 % at one).  per_chunk: what a chunk costs besides
+// (its rho partial).  Within 4 % of the fastest count at 80^3 to 160^3, where
+// counting whole rounds was up to 15 % off.  At most max_chunks chunks.
+void pick_chunks(int units, int occ, int ncu, int nst, int max_chunks, double per_chunk, int& cs,
+                 int& nchunk) {
   double best = 1e300;
+  const long slots = (long)occ * ncu;
   cs = nst;
   nchunk = 1;
   for (int nc = 1; nc <= std::min(nst, std::max(1, max_chunks)); nc++) {
     const int s = (nst + nc - 1) / nc, ncr = (nst + s - 1) / s;
     if (ncr != nc) continue;
-    const long wg = (long)units * ncr;
-    const long rounds = (wg + slots - 1) / slots;
-    const double cost = (double)rounds * (s + 1);
+    const long wg = (long)units * ncr, full = wg / slots, rem = wg % slots;
+    const double rounds = full * (occ + 1.5) + (rem ? (rem + ncu - 1) / ncu + 1.5 : 0.0);
+    const double cost = (s + 0.5) * rounds * (1.0 + 0.06 / std::max(1.0, (double)wg / slots)) +
+                        per_chunk * nc;
     if (cost < best) {
       best = cost;
       cs = s;
@@ -473,9 +481,13 @@ oa_status build_layout(oa_ctx* c) {
     // chunk count is bounded like the G->R one's
     c->fuse_rho = rho_ok && !c->opt.vks_from_rho;
     const int max_r = c->fuse_rho ? std::min(c->nst, kMaxRhoChunks) : c->nst;
-    pick_chunks(c->nz * rowparts, std::max(1, occ_g) * ncu, c->nst, kMaxRhoChunks, f.cs,
+    // a rho partial is written and read back: 3.3 us at 100^3, where a unit of
+    // the G->R pass is about 1 us; both scale with the points of a plane
+    const double part = 3e-6 * (double)c->nx * c->ny * c->nz;
+    pick_chunks(c->nz * rowparts, std::max(1, occ_g), ncu, c->nst, kMaxRhoChunks, part, f.cs,
                 f.nchunk);
-    pick_chunks(c->nz, std::max(1, occ_r) * ncu, c->nst, max_r, f.cs_r, f.nchunk_r);
+    pick_chunks(c->nz, std::max(1, c->fuse_rho ? rho_ok : occ_r), ncu, c->nst, max_r,
+                c->fuse_rho ? part : 0.0, f.cs_r, f.nchunk_r);
     c->nzblk = (c->nlines + oa::fft2_ntr(c->nz) - 1) / oa::fft2_ntr(c->nz);
     if (c->opt.autotune) {
       c->tune_nchunk = chunk_candidates(c->nst, f.nchunk, kMaxRhoChunks);
@@ -659,8 +671,14 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
     // run separately and opt.psir_keep asks to keep it between them
     TRY(dalloc(c, &c->zout, zsz));
     TRY(dalloc(c, &c->psir, N * rsz));
+    if (c->fc.prune) {
+      c->vperm.m = oa::plane_classes(c->nx, c->fp32, &c->vperm.x1);
+      c->vperm.n = c->nx;
+      c->vperm.f32 = c->fp32 ? 1 : 0;
+      if (c->vperm.m > 0) TRY(dalloc(c, &c->vperm.p, N * rsz));
+    }
     if (c->opt.psir_keep && !c->fuse_rho) {
-      const size_t kper = oa::plane3_kper(c->nx, c->nplane_x, c->fp32);
+      const size_t kper = oa::plane3_kper(c->nx, c->nplane_x, c->fp32, c->fc.prune != 0);
       if (kper == 0) return fail(c, OA_EINVAL, "plane size not compiled");
       TRY(dalloc(c, &c->psk, (size_t)c->nst * c->nz * kper * csz));
     }
@@ -766,6 +784,11 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
   HIPCHK(oa::fill_zero(c->psi2, gsz, c->stream));
   HIPCHK(oa::fill_zero(c->force, gsz, c->stream));
   HIPCHK(oa::fill_zero(c->vks, N * sizeof(double), c->stream));
+  if (c->vperm.p) {
+    HIPCHK(oa::fill_zero(c->vperm.p, N * rsz, c->stream));
+    HIPCHK(oa::zero_rows(c->zbuf, (size_t)c->nst * c->nz * c->nplane_x, c->ny, c->fp32,
+                         c->stream));
+  }
   HIPCHK(oa::fill_zero(c->res, sizeof(StepDev), c->stream));
   if (c->vloc)
     HIPCHK(oa::fill_zero(c->vloc, (size_t)c->va.nkx * c->va.nky * c->nz * sizeof(double2),
@@ -793,6 +816,7 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
   f.xbuf = c->xbuf;
   f.psir = c->psir;
   f.psk = c->psk;
+  f.vperm = c->vperm.p;
   f.rho = c->rho;
   f.eke_part = c->eke_part;
   f.lines = c->lines;
@@ -822,7 +846,8 @@ FftCtx range_ctx(oa_ctx* c, int s0, int ns) {
   f.zout = static_cast<unsigned char*>(c->zout) + (size_t)s0 * zst;
   if (c->psk)
     f.psk = static_cast<unsigned char*>(c->psk) +
-            (size_t)s0 * c->nz * oa::plane3_kper(c->nx, c->nplane_x, c->fp32) * (c->fp32 ? 8 : 16);
+            (size_t)s0 * c->nz * oa::plane3_kper(c->nx, c->nplane_x, c->fp32, c->fc.prune != 0) *
+                (c->fp32 ? 8 : 16);
   f.occ = c->occ + s0;
   f.eke_part = c->eke_part + (size_t)s0 * c->nzblk;
   f.nchunk = (ns + f.cs - 1) / f.cs;
@@ -861,6 +886,7 @@ oa_status st_vks(oa_ctx* c) {
   oa::VksArgs a = c->va;
   a.rho = c->rho;
   a.v = c->vks;
+  a.vp = c->vperm;
   a.twx = c->twx;
   a.twy = c->twy;
   a.twz = c->twz;
@@ -1387,8 +1413,10 @@ oa_status autotune(oa_ctx* c) {
   HIPCHK(hipStreamSynchronize(c->stream));
   // leave no state from the trial runs behind
   HIPCHK(oa::fill_zero(c->res, sizeof(StepDev), c->stream));
-  if (c->opt.vks_from_rho)  // V_KS of the trials' (zero) density
+  if (c->opt.vks_from_rho) {  // V_KS of the trials' (zero) density
     HIPCHK(oa::fill_zero(c->vks, (size_t)c->nx * c->ny * c->nz * sizeof(double), c->stream));
+    HIPCHK(oa::vperm_set(c->vperm, c->vks, c->nz, c->stream));
+  }
   c->have_S = c->have_T = false;
   HIPCHK(hipStreamSynchronize(c->stream));
   return OA_OK;
@@ -1641,6 +1669,7 @@ oa_status oa_vks_set(oa_ctx* c, const double* v) {
     return fail(c, OA_ESTATE, "this context builds V from rho (vks_from_rho)");
   HIPCHK(hipSetDevice(c->device));
   TRY(upload(c, c->vks, v, (size_t)c->nx * c->ny * c->nz * sizeof(double)));
+  HIPCHK(oa::vperm_set(c->vperm, c->vks, c->nz, c->stream));
   c->have_v = true;
   return OA_OK;
 }
