@@ -470,98 +470,165 @@ hipError_t gram_reduce_f32(const float* part, int nslice, int n, int nb, int sym
 // ================================================================== rotate
 // Y[j][k] = beta Y[j][k] + s(k) sum_{i < ni} M[i][j] X[i][k] as D = M^T X: the
 // output tile rows are j and its columns k, so the stores run along k.
-// Workgroup: 64 columns k x 128 rows j; wave w owns j tiles 2w, 2w+1 of the
-// block.  The i loop runs in chunks of 16 with the next chunk's operands
-// loaded while the current chunk's 32 MFMAs issue.
 constexpr int kRK = 64;
 
-__global__ __launch_bounds__(256, 2) void k_rotate(RotArgs a) {
+// n or ni > 128.  Workgroup: 64 columns k, W waves of JT 16-row tiles j each;
+// wave: 16 JT x 64 outputs, so a step of four i costs JT + 2 loads per lane for
+// 4 JT MFMAs.  A lane's B values are four consecutive k (two 16-byte loads; the
+// output column l16 of tile y is k = kb + 4 l16 + y, any assignment works as long
+// as the stores follow it), so a row of Y is read and written 32 bytes per lane.
+// The loads of a step are issued kRwRing steps ahead into a register ring (two
+// ahead: 20 % slower, four: the same), two waves per SIMD (one: 10 % slower).
+// Bound by the matrix pipe, and below 400 states by the start and end of a
+// block.  Y = M^T X (and Y += ...): 512 states x 260,992 reals 68 (62) TFLOP/s,
+// 256 x 131,824 50 (47), 180 x 73,600 45 (46); 50 (50), 45 (40), 32 (32) before,
+// with 32 x 64 outputs per wave, 1.5 times the loads per MFMA and Y accessed in
+// 8-byte pieces.  A library product of the first two shapes reaches 71 and 49.
+constexpr int kRwRing = 3;
+
+template <int JT>
+struct RwStep {
+  double a[JT];
+  double4 b;
+};
+
+template <int JT, bool USE_Y>
+__global__ __launch_bounds__(256, 2) void k_rotate_w(RotArgs a) {
   __shared__ double red[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int l16 = lane & 15, g = lane >> 4;
   const int kb = blockIdx.x * kRK;
-  const int jb = blockIdx.y * 128 + wave * 32;
-  // operand columns clamped into range: columns past n or K are computed
-  // from duplicated data and never stored
-  int jc[2], kc[4];
-#pragma unroll
-  for (int x = 0; x < 2; x++) jc[x] = min(jb + 16 * x + l16, a.n - 1);
-#pragma unroll
-  for (int y = 0; y < 4; y++) kc[y] = min(kb + 16 * y + l16, a.K - 1);
-  v4d acc[2][4];
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 4; y++) acc[x][y] = vzero();
-  if (jb < a.n) {
-    double am0[4][2], bx0[4][4], am1[4][2], bx1[4][4];
-    // branch-free: rows past ni are clamped and their M values zeroed (a
-    // load that only some lanes issue is waited for on its own)
-    auto load = [&](int i0, double (&am)[4][2], double (&bx)[4][4]) {
-#pragma unroll
-      for (int s = 0; s < 4; s++) {
-        const int i = i0 + 4 * s + g, ic = min(i, a.ni - 1);
-        const bool vi = i < a.ni;
-#pragma unroll
-        for (int x = 0; x < 2; x++) {
-          const double m = a.M[(size_t)ic * a.n + jc[x]];
-          am[s][x] = vi ? m : 0.0;
-        }
-#pragma unroll
-        for (int y = 0; y < 4; y++) bx[s][y] = a.X[(size_t)ic * a.ldx + kc[y]];
-      }
-    };
-    auto mma = [&](const double (&am)[4][2], const double (&bx)[4][4]) {
-#pragma unroll
-      for (int s = 0; s < 4; s++)
-#pragma unroll
-        for (int x = 0; x < 2; x++)
-#pragma unroll
-          for (int y = 0; y < 4; y++) acc[x][y] = mfma16(am[s][x], bx[s][y], acc[x][y]);
-    };
-    int i0 = 0;
-    load(0, am0, bx0);
-    while (i0 < a.ni) {
-      if (i0 + 16 < a.ni) load(i0 + 16, am1, bx1);
-      mma(am0, bx0);
-      i0 += 16;
-      if (i0 >= a.ni) break;
-      if (i0 + 16 < a.ni) load(i0 + 16, am0, bx0);
-      mma(am1, bx1);
-      i0 += 16;
-    }
-  }
-  // fused steepest descent: every read of X (= sd_psi) in this workgroup
-  // precedes the updates below; no other workgroup reads these columns
-  if (a.sd_psi) __syncthreads();
+  const int jb = (blockIdx.y * nw + wave) * 16 * JT;
   double fn = 0.0;
+  if (jb < a.n) {
+    v4d acc[JT][4];
 #pragma unroll
-  for (int x = 0; x < 2; x++)
+    for (int x = 0; x < JT; x++)
 #pragma unroll
-    for (int y = 0; y < 4; y++)
+      for (int y = 0; y < 4; y++) acc[x][y] = vzero();
+    // byte offsets of the lane inside a step's four rows; rows j past n are
+    // computed from duplicated data and never stored
+    unsigned mo[JT];
+#pragma unroll
+    for (int x = 0; x < JT; x++)
+      mo[x] = (unsigned)((g * a.n + min(jb + 16 * x + l16, a.n - 1)) * sizeof(double));
+    const unsigned xo = (unsigned)((g * a.ldx + kb + 4 * l16) * sizeof(double));
+    const int nfull = a.ni >> 2;
+    auto load = [&](int st, RwStep<JT>& d) __attribute__((always_inline)) {
+      const char* mp = (const char*)(a.M + (size_t)st * 4 * a.n);
+      const char* xp = (const char*)(a.X + (size_t)st * 4 * a.ldx);
+#pragma unroll
+      for (int x = 0; x < JT; x++) d.a[x] = *(const double*)(mp + mo[x]);
+      d.b = *(const double4*)(xp + xo);
+    };
+    auto mma = [&](const RwStep<JT>& d) __attribute__((always_inline)) {
+      const double bv[4] = {d.b.x, d.b.y, d.b.z, d.b.w};
+#pragma unroll
+      for (int x = 0; x < JT; x++)
+#pragma unroll
+        for (int y = 0; y < 4; y++) acc[x][y] = mfma16(d.a[x], bv[y], acc[x][y]);
+    };
+    if (nfull > 0) {
+      RwStep<JT> ring[kRwRing];
+      static_for<0, kRwRing>([&](auto dc) __attribute__((always_inline)) {
+        constexpr int d = decltype(dc)::value;
+        load(min(d, nfull - 1), ring[d]);
+      });
+      // every load is issued on every path (past the end: the last step again)
+      for (int st = 0; st < nfull; st += kRwRing) {
+        static_for<0, kRwRing>([&](auto dc) __attribute__((always_inline)) {
+          constexpr int d = decltype(dc)::value;
+          if (st + d < nfull) mma(ring[d]);
+          load(min(st + d + kRwRing, nfull - 1), ring[d]);
+        });
+      }
+    }
+    if (a.ni & 3) {  // the last, partial step: rows past ni clamped, their M zeroed
+      RwStep<JT> d;
+      const int i = 4 * nfull + g, ic = min(i, a.ni - 1);
+#pragma unroll
+      for (int x = 0; x < JT; x++) {
+        const double m = a.M[(size_t)ic * a.n + min(jb + 16 * x + l16, a.n - 1)];
+        d.a[x] = i < a.ni ? m : 0.0;
+      }
+      d.b = *(const double4*)(a.X + (size_t)ic * a.ldx + kb + 4 * l16);
+      mma(d);
+    }
+    const int k0 = kb + 4 * l16;
+    double s[4];
+#pragma unroll
+    for (int y = 0; y < 4; y++) s[y] = k0 + y < a.k_lo ? a.s_lo : a.s_hi;
+#pragma unroll
+    for (int x = 0; x < JT; x++) {
+      double4 yo[4];
+      if (USE_Y) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const int j = min(jb + 16 * x + g + 4 * v, a.n - 1);
+          yo[v] = *(const double4*)(a.Y + (size_t)j * a.ldx + k0);
+        }
+      }
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int j = jb + 16 * x + g + 4 * v;
-        const int k = kb + 16 * y + l16;  // unclamped: each output once
-        if (j < a.n && k < a.K) {
-          const double s = (k < a.k_lo) ? a.s_lo : a.s_hi;
-          double* yp = a.Y + (size_t)j * a.ldx + k;
-          double val = s * acc[x][y][v];
-          if (a.beta != 0.0) val = a.beta * (*yp) + val;
-          *yp = val;
-          if (a.sd_psi) {
-            a.sd_psi[(size_t)j * a.ldx + k] += a.dtm[k >> 1] * val;
-            fn += val * val;
+        double o[4];
+#pragma unroll
+        for (int y = 0; y < 4; y++) o[y] = s[y] * acc[x][y][v];
+        if (USE_Y) {
+          o[0] = a.beta * yo[v].x + o[0];
+          o[1] = a.beta * yo[v].y + o[1];
+          o[2] = a.beta * yo[v].z + o[2];
+          o[3] = a.beta * yo[v].w + o[3];
+        }
+        if (j < a.n) {
+          double* yp = a.Y + (size_t)j * a.ldx + k0;
+          if (k0 + 3 < a.K) {
+            *(double4*)yp = make_double4(o[0], o[1], o[2], o[3]);
+            fn += (o[0] * o[0] + o[1] * o[1]) + (o[2] * o[2] + o[3] * o[3]);
+          } else {
+#pragma unroll
+            for (int y = 0; y < 4; y++)
+              if (k0 + y < a.K) {
+                yp[y] = o[y];
+                fn += o[y] * o[y];
+              }
           }
         }
       }
-  if (a.sd_psi) {
+    }
+  }
+  if (a.fpart) {
     for (int o = 32; o > 0; o >>= 1) fn += __shfl_down(fn, o, 64);
     if (lane == 0) red[wave] = fn;
     __syncthreads();
-    if (tid == 0)
-      a.fpart[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    if (threadIdx.x == 0) {
+      double t = 0.0;
+      for (int w = 0; w < nw; w++) t += red[w];
+      a.fpart[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = t;
+    }
   }
+}
+
+// Waves per workgroup and 16-row tiles per wave for n output rows: the pair
+// that computes the fewest rows past n (9 tiles: 3 x 3, 12: 4 x 3, 16: 4 x 4),
+// then the larger tile per wave; four waves before three, which leave two SIMDs
+// with half the work unless an even number of workgroups shares the CU.
+struct RwShape {
+  int waves, jt, blocks;
+};
+static RwShape rw_shape(int n) {
+  const int nt = (n + 15) / 16;
+  RwShape best{4, 4, (nt + 15) / 16};
+  int waste = best.blocks * 16;
+  const int cand[3][2] = {{4, 3}, {3, 3}, {4, 2}};
+  for (const auto& c : cand) {
+    const int per = c[0] * c[1], blocks = (nt + per - 1) / per;
+    if (blocks * per < waste) {
+      waste = blocks * per;
+      best = {c[0], c[1], blocks};
+    }
+  }
+  return best;
 }
 
 // n, ni <= 128: persistent workgroups of 8 waves (two per SIMD).  M is staged
@@ -742,13 +809,14 @@ static int rotate_pgrid(int K) {
 }
 
 int rotate_nwg(int n, int K) {
-  return n <= 128 ? rotate_pgrid(K) : ((K + kRK - 1) / kRK) * ((n + 127) / 128);
+  return n <= 128 ? rotate_pgrid(K) : ((K + kRK - 1) / kRK) * rw_shape(n).blocks;
 }
 
 hipError_t rotate_f64(const RotArgs& args, hipStream_t st) {
   RotArgs a = args;
   if (a.ni <= 0) a.ni = a.n;
-  if ((a.sd_psi || a.fpart) && (a.n > 128 || a.ni > 128)) return hipErrorInvalidValue;
+  if (a.sd_psi && (a.n > 128 || a.ni > 128)) return hipErrorInvalidValue;
+  if (a.fpart && a.n <= 128 && a.ni > 128) return hipErrorInvalidValue;
   if (a.sd_psi && (a.sd_psi != a.X || !a.dtm || !a.fpart || a.ni != a.n))
     return hipErrorInvalidValue;
   if (a.n <= 128 && a.ni <= 128) {
@@ -764,8 +832,13 @@ hipError_t rotate_f64(const RotArgs& args, hipStream_t st) {
     hipLaunchKernelGGL(fns[v], dim3(rotate_pgrid(a.K)), dim3(kRotThreads), kRotSmem, st, a);
     return hipGetLastError();
   }
-  dim3 grid((a.K + kRK - 1) / kRK, (a.n + 127) / 128);
-  hipLaunchKernelGGL(k_rotate, grid, dim3(256), 0, st, a);
+  if (a.ldx % kRK) return hipErrorInvalidValue;  // whole 64-column blocks inside a row
+  const RwShape sh = rw_shape(a.n);
+  const bool y = a.beta != 0.0;
+  void (*const fn)(RotArgs) = sh.jt == 4   ? (y ? k_rotate_w<4, true> : k_rotate_w<4, false>)
+                              : sh.jt == 3 ? (y ? k_rotate_w<3, true> : k_rotate_w<3, false>)
+                                           : (y ? k_rotate_w<2, true> : k_rotate_w<2, false>);
+  hipLaunchKernelGGL(fn, dim3((a.K + kRK - 1) / kRK, sh.blocks), dim3(64 * sh.waves), 0, st, a);
   return hipGetLastError();
 }
 

@@ -1035,7 +1035,7 @@ oa_status st_gram(oa_ctx* c, const double2* A, const double2* B, bool sym, doubl
 }
 
 // sd: also apply psi += dt/m F to X (= psi) in the same pass (n <= 128)
-// fnorm: also leave per-workgroup partials of sum Y^2 in fpart (n <= 128)
+// fnorm: also leave per-workgroup partials of sum Y^2 in fpart
 // split: the split-BF16 kernel (no SD epilogue; split_rotate_ok);
 // update: Y = X + X (M - I) (split only)
 oa_status st_rotate(oa_ctx* c, const double2* X, const double* M, double2* Y, double beta,
@@ -1099,18 +1099,10 @@ oa_status st_sd_finish(oa_ctx* c) {
 // Lambda projection, then the CG direction and update: |F|^2 (fovlap) must
 // be complete before gamma, so the update is a pass of its own
 oa_status st_lambda_cg(oa_ctx* c) {
-  const size_t N2 = (size_t)2 * c->nst * c->ld;  // reals in F, zero padding included
   TRY(st_gram(c, c->psi, c->force, false, 1.0, 1.0, c->lam, split_on(c, kSplitLambda)));
-  if (c->nst <= 128) {
-    TRY(st_rotate(c, c->psi, c->lam, c->force, 1.0, -0.5, -1.0, false, true,
-                  split_on(c, kSplitProj) && split_rotate_ok(c)));
-    HIPCHK(oa::reduce_to(c->fpart, lambda_nwg(c), 1.0, &c->res->fnorm2, c->stream));
-  } else {
-    TRY(st_rotate(c, c->psi, c->lam, c->force, 1.0, -0.5, -1.0));
-    const double* fr = reinterpret_cast<const double*>(c->force);
-    HIPCHK(oa::dot_parts(fr, fr, N2, c->fpart, c->nfpart, c->stream));
-    HIPCHK(oa::reduce_to(c->fpart, c->nfpart, 1.0, &c->res->fnorm2, c->stream));
-  }
+  TRY(st_rotate(c, c->psi, c->lam, c->force, 1.0, -0.5, -1.0, false, true,
+                split_on(c, kSplitProj) && split_rotate_ok(c)));
+  HIPCHK(oa::reduce_to(c->fpart, lambda_nwg(c), 1.0, &c->res->fnorm2, c->stream));
   HIPCHK(oa::cg_gamma(c->res, c->cgs, c->stream));
   HIPCHK(oa::cg_update(c->psi, c->cgdir, c->force, c->dtm, c->g2, c->ecut_ry, c->nst, c->npts,
                        c->ld, c->cgs, c->stream));
