@@ -16,9 +16,8 @@
 // vector instructions, which bound the gram).
 //
 //   gram_bf16   : C = sum_k w(k) A[i][k] B[j][k] (Lambda = Re Psi^H F, and S on
-//                 request): one workgroup per 128 x 128 output block and K
-//                 slice, wave (wr, wc) the 64 x 64 quadrant, operands loaded
-//                 from HBM straight into registers and split there;
+//                 request): one workgroup per output block (128 or 256 square)
+//                 and K slice, operands split once per workgroup into LDS;
 //   rotate_bf16 : Y = beta Y + s(k) M^T X (+ X) for n, ni <= 128 (F -= w Psi
 //                 Lambda, and Psi T on request in the form Psi + Psi (T - I)):
 //                 persistent workgroups over 64-column blocks of K; the
@@ -32,6 +31,8 @@
 // Within one MFMA the assignment of k to (lane group, element) is free as
 // long as A and B agree.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "oa_common.h"
 #include "oa_gemm_common.h"
@@ -88,102 +89,154 @@ __device__ __forceinline__ f16v mma6(const Split& a, const Split& b, f16v acc) {
   return mfma32(a.h, b.h, acc);
 }
 
-// x[e] = X[row][kk + e], two 32-byte loads (kk a multiple of 8 inside the
-// row's allocation; lda a multiple of 16)
-__device__ __forceinline__ void load8(const double* __restrict__ X, int lda, int row, int kk,
-                                      double (&x)[8]) {
-  const double4* p = reinterpret_cast<const double4*>(X + (size_t)row * lda + kk);
-  const double4 u = p[0], v = p[1];
-  x[0] = u.x;
-  x[1] = u.y;
-  x[2] = u.z;
-  x[3] = u.w;
-  x[4] = v.x;
-  x[5] = v.y;
-  x[6] = v.z;
-  x[7] = v.w;
-}
-
-__device__ __forceinline__ void mask8(int kk, int rs, int re, double (&x)[8]) {
-#pragma unroll
-  for (int e = 0; e < 8; e++) x[e] = (kk + e >= rs && kk + e < re) ? x[e] : 0.0;
-}
-
-struct GFrag {
-  double a[2][8];  // two 32-row tiles of A
-  double b[2][8];  // two 32-row tiles of B
-};
-
 }  // namespace
 
-// grid (output blocks nbe x nbe_b, K slices); every block is computed whole
-// (a symmetric product's lower half is mirrored by the reduction)
-__global__ __launch_bounds__(256) void k_gram_bf16(GramArgs a, float* __restrict__ part,
-                                                   int nbe_b, int nlo) {
-  const int bi = blockIdx.x / nbe_b, bj = blockIdx.x - (blockIdx.x / nbe_b) * nbe_b;
-  const int sp = blockIdx.y;
+// ------------------------------------------------------------------ gram
+// Blocks of 64 RT x 64 RT outputs (every block whole: a symmetric product's
+// lower half is mirrored by the reduction), operands split once per workgroup.
+// A workgroup of four waves (wave: RT x RT tiles of 32 x 32) owns a block and a
+// K slice.  Per 16 k values every thread loads pairs of its rows (a row's 128
+// bytes by eight lanes), splits them and puts the three terms into LDS in the
+// operand layout; the MFMAs of the current chunk, the split of the next one and
+// the loads of the one after overlap (double-buffered LDS, one barrier per
+// chunk).  A split in every wave that uses an operand, from registers, took
+// each value through the conversions up to eight times and bound the product:
+// us for 128 x 65,922 reals 42 -> 27, 180 x 73,600 150 -> 65, 256 x 131,824
+// 284 -> 133, 512 x 260,992 2533 -> 878 (conversions and MFMAs alternate in one
+// wave per SIMD there; the bytes take 420 at the rate of a copy).
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+
+template <int RT>
+constexpr size_t gram_bf16_lds() {
+  return (size_t)2 * 2 * 3 * (2 * RT) * 64 * sizeof(bf8);
+}
+
+// Workgroups go to the 8 XCDs round-robin: all output blocks of one K slice read
+// the same operand columns, so they are put on one XCD (one L2) where the slice
+// count allows.
+__device__ __forceinline__ void slice_block(int& b, int& sp) {
+  b = blockIdx.x;
+  sp = blockIdx.y;
+  if (gridDim.y % 8 == 0) {
+    const int id = blockIdx.x + gridDim.x * blockIdx.y, k = id >> 3;
+    b = k % gridDim.x;
+    sp = (k / gridDim.x) * 8 + (id & 7);
+  }
+}
+
+template <int RT>
+__global__ __launch_bounds__(256, RT == 4 ? 1 : 2) void k_gram_bf16(GramArgs a,
+                                                                     float* __restrict__ part,
+                                                                     int nbe_b, int nlo) {
+  constexpr int TT = 2 * RT;                   // 32-row tiles per operand
+  constexpr int TERM = TT * 64, OPER = 3 * TERM, BUF = 2 * OPER;  // in bf8
+  extern __shared__ __align__(16) unsigned char gb_smem[];
+  bf8* L = reinterpret_cast<bf8*>(gb_smem);    // [buffer][operand][term][tile][lane]
+  int blk, sp;
+  slice_block(blk, sp);
+  const int bi = blk / nbe_b, bj = blk - bi * nbe_b;
   const GSlice s = gram_slice(a, sp, nlo);
   const double* __restrict__ B = a.sym ? a.A : a.B;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int l32 = lane & 31, g = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wr = wave >> 1, wc = wave & 1;
-  const int rbase = bi * 128 + wr * 64, cbase = bj * 128 + wc * 64;
-  if (rbase >= a.n || cbase >= a.nb) return;
-  int ra[2], rb[2];
-#pragma unroll
-  for (int x = 0; x < 2; x++) {  // rows past the matrices: outputs not stored
-    const int r = rbase + 32 * x + l32, q = cbase + 32 * x + l32;
-    ra[x] = r < a.n ? r : 0;
-    rb[x] = q < a.nb ? q : 0;
-  }
-  f16v acc[2][2];
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++) acc[x][y] = fzero16();
-  auto mfmas = [&](const GFrag& f) __attribute__((always_inline)) {
-    Split sa[2], sb[2];
-#pragma unroll
-    for (int x = 0; x < 2; x++) {
-      sa[x] = split3(f.a[x]);
-      sb[x] = split3(f.b[x]);
-    }
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-      for (int y = 0; y < 2; y++) acc[x][y] = mma6(sa[x], sb[y], acc[x][y]);
+  const int l32 = lane & 31, g = lane >> 5;
+  // staging: thread (r0, kp) takes the pair of k values 2 kp, 2 kp + 1 of row r0
+  // of every tile; rows past the matrices repeat the last (outputs not stored)
+  const int kp = tid & 7, r0 = tid >> 3;
+  unsigned* const stage = reinterpret_cast<unsigned*>(L) + (r0 + 32 * (kp >> 2)) * 4 + (kp & 3);
+  double2 raw[2 * TT];
+  auto load = [&](int u, int c) __attribute__((always_inline)) {
+    const bool isb = u >= TT;
+    const int n = isb ? a.nb : a.n;
+    const int tb = min((isb ? bj : bi) * 64 * RT + 32 * (isb ? u - TT : u), n - 1);
+    const double* p = (isb ? B : a.A) + (size_t)tb * a.lda + s.base + 16 * c;
+    raw[u] = *reinterpret_cast<const double2*>(p + (size_t)min(r0, n - 1 - tb) * a.lda + 2 * kp);
   };
-  GFrag ring[2];
-  chunk_ring(
-      s.c0, s.c1, ring,
-      [&](int c, GFrag& d) __attribute__((always_inline)) {
-        const int kk = s.base + 16 * c + 8 * g;
+  // split tile u of chunk c into buffer buf; edge: elements outside the region
+  // [rs, re) are zeroed (only a slice's first and last chunk reach past it;
+  // padding past K may hold anything)
+  auto split = [&](auto edge, int u, int c, int buf) __attribute__((always_inline)) {
+    double2 x = raw[u];
+    if constexpr (decltype(edge)::value) {
+      const int kk = s.base + 16 * c + 2 * kp;
+      x.x = kk >= s.rs && kk < s.re ? x.x : 0.0;
+      x.y = kk + 1 >= s.rs && kk + 1 < s.re ? x.y : 0.0;
+    }
+    f2 r = {(float)x.x, (float)x.y};
+    // the FP32 values as such: rounding the doubles to BF16 directly, as the
+    // compiler otherwise does for the first term, takes ten instructions more
+    asm("" : "+v"(r.x), "+v"(r.y));
+    unsigned* out = stage + (size_t)(buf * BUF + (u >= TT ? OPER : 0) + (u % TT) * 64) * 4;
 #pragma unroll
-        for (int x = 0; x < 2; x++) {
-          load8(a.A, a.lda, ra[x], kk, d.a[x]);
-          load8(B, a.lda, rb[x], kk, d.b[x]);
-        }
-      },
-      [&](int c, const GFrag& d) __attribute__((always_inline)) {
-        const int k0 = s.base + 16 * c;
-        if (k0 >= s.rs && k0 + 16 <= s.re) {
-          mfmas(d);
-        } else {  // a chunk at the region's edge (padding past K may hold anything)
-          GFrag m = d;
+    for (int t = 0; t < 3; t++) {
+      const bf2 h = {(__bf16)r.x, (__bf16)r.y};
+      out[(size_t)t * TERM * 4] = __builtin_bit_cast(unsigned, h);
+      r.x -= (float)h.x;
+      r.y -= (float)h.y;
+    }
+  };
+  f16v acc[RT][RT];
 #pragma unroll
-          for (int x = 0; x < 2; x++) {
-            mask8(k0 + 8 * g, s.rs, s.re, m.a[x]);
-            mask8(k0 + 8 * g, s.rs, s.re, m.b[x]);
-          }
-          mfmas(m);
-        }
-      });
+  for (int x = 0; x < RT; x++)
+#pragma unroll
+    for (int y = 0; y < RT; y++) acc[x][y] = fzero16();
+  // the products of chunk c0 + i, and the split of the next one
+  auto chunk = [&](auto edge, int i) __attribute__((always_inline)) {
+    const bf8* Ab = L + (i & 1) * BUF + wr * RT * 64 + lane;
+    const bf8* Bb = L + (i & 1) * BUF + OPER + wc * RT * 64 + lane;
+    const int cn = min(s.c0 + i + 1, s.c1 - 1), cl = min(s.c0 + i + 2, s.c1 - 1);
+    Split sb[RT];
+#pragma unroll
+    for (int y = 0; y < RT; y++)
+      sb[y] = {Bb[y * 64], Bb[TERM + y * 64], Bb[2 * TERM + y * 64]};
+#pragma unroll
+    for (int x = 0; x < RT; x++) {
+      const Split sa = {Ab[x * 64], Ab[TERM + x * 64], Ab[2 * TERM + x * 64]};
+      // the six term products, small terms first, over independent tiles
+#pragma unroll
+      for (int y = 0; y < RT; y++) acc[x][y] = mfma32(sa.l, sb[y].h, acc[x][y]);
+#pragma unroll
+      for (int y = 0; y < RT; y++) acc[x][y] = mfma32(sa.m, sb[y].m, acc[x][y]);
+#pragma unroll
+      for (int y = 0; y < RT; y++) acc[x][y] = mfma32(sa.h, sb[y].l, acc[x][y]);
+#pragma unroll
+      for (int y = 0; y < RT; y++) acc[x][y] = mfma32(sa.m, sb[y].h, acc[x][y]);
+#pragma unroll
+      for (int y = 0; y < RT; y++) acc[x][y] = mfma32(sa.h, sb[y].m, acc[x][y]);
+#pragma unroll
+      for (int y = 0; y < RT; y++) acc[x][y] = mfma32(sa.h, sb[y].h, acc[x][y]);
+      // four tiles of the next chunk between the products; a tile's loads for
+      // the chunk after it follow at once and are in flight for a whole chunk
+#pragma unroll
+      for (int u = 4 * x; u < 4 * x + 4; u++) {
+        split(edge, u, cn, (i + 1) & 1);
+        load(u, cl);
+      }
+    }
+    __syncthreads();
+  };
+  const int nc = s.c1 - s.c0;
+  if (nc > 0) {
+#pragma unroll
+    for (int u = 0; u < 2 * TT; u++) load(u, s.c0);
+#pragma unroll
+    for (int u = 0; u < 2 * TT; u++) {
+      split(std::true_type{}, u, s.c0, 0);
+      load(u, min(s.c0 + 1, s.c1 - 1));
+    }
+    __syncthreads();
+    int i = 0;
+    for (; i < nc - 2; i++) chunk(std::false_type{}, i);
+    for (; i < nc; i++) chunk(std::true_type{}, i);
+  }
   float* out = part + (size_t)sp * a.n * a.nb;
   const float w = (float)s.w;  // 1 or 2: exact
+  const int rbase = bi * 64 * RT + wr * 32 * RT, cbase = bj * 64 * RT + wc * 32 * RT;
 #pragma unroll
-  for (int x = 0; x < 2; x++)
+  for (int x = 0; x < RT; x++)
 #pragma unroll
-    for (int y = 0; y < 2; y++)
+    for (int y = 0; y < RT; y++)
 #pragma unroll
       for (int v = 0; v < 16; v++) {
         const int r = rbase + 32 * x + 8 * (v >> 2) + 4 * g + (v & 3);
@@ -192,12 +245,31 @@ __global__ __launch_bounds__(256) void k_gram_bf16(GramArgs a, float* __restrict
       }
 }
 
+// Block edge in units of 64 rows: 256 rows where that pads a matrix of more
+// than one block no more than 128 rows do (512 states: 878 us against 1088;
+// 256: 155 against 133, 300: 233 against 142), else 128.
+static int gram_bf16_rt(int n, int nb) {
+  const int m = std::max(n, nb);
+  return m > 256 && (m + 255) / 256 * 2 == (m + 127) / 128 ? 4 : 2;
+}
+
+// one workgroup per CU for a single block or blocks of 256 rows, else two
+int gram_bf16_slices(int n, int K, int target) {
+  const int rt = gram_bf16_rt(n, n), nb = (n + 64 * rt - 1) / (64 * rt);
+  const int ns = std::max(2, target * (nb > 1 && rt == 2 ? 2 : 1) / (nb * nb));
+  return std::min(ns, std::max(2, K / 64));  // at least four chunks per slice
+}
+
 hipError_t gram_bf16(const GramArgs& a, float* part, hipStream_t st) {
   if (a.nslice < 1 || (a.k_lo > 0 && a.k_lo < a.K && a.nslice < 2) || (a.lda & 15) ||
       a.n < 1 || a.nb < 1 || (a.sym && a.nb != a.n) || !part)
     return hipErrorInvalidValue;
-  const int nbe = (a.n + 127) / 128, nbe_b = (a.nb + 127) / 128;
-  hipLaunchKernelGGL(k_gram_bf16, dim3(nbe * nbe_b, a.nslice), dim3(256), 0, st, a, part, nbe_b,
+  const int rt = gram_bf16_rt(a.n, a.nb), edge = 64 * rt;
+  const int nbe = (a.n + edge - 1) / edge, nbe_b = (a.nb + edge - 1) / edge;
+  void (*const fn)(GramArgs, float*, int, int) = rt == 4 ? k_gram_bf16<4> : k_gram_bf16<2>;
+  const size_t lds = rt == 4 ? gram_bf16_lds<4>() : gram_bf16_lds<2>();
+  if (const hipError_t e = grant_lds((const void*)fn, lds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(nbe * nbe_b, a.nslice), dim3(256), lds, st, a, part, nbe_b,
                      gram_nlo(a));
   return hipGetLastError();
 }

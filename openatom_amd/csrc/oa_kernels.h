@@ -243,6 +243,8 @@ int rotate_nwg(int n, int K);  // workgroups of a rotate launch (fpart entries)
 // (every block whole, also when sym), summed by gram_reduce_f32.
 hipError_t gram_bf16(const GramArgs& a, float* part, hipStream_t st);
 hipError_t gram_reduce_f32(const float* part, int nslice, int n, int nb, int sym, double alpha,
+// K slices of an n x n product on `target` CUs
+int gram_bf16_slices(int n, int K, int target);
                            double* C, hipStream_t st);
 // rotate_bf16: the product of rotate_f64 for n, ni <= 128 and ldx a multiple
 // of 64 (no SD epilogue); fpart, if set, gets per-workgroup sums of Ynew^2

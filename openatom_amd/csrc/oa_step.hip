@@ -306,6 +306,12 @@ std::vector<double2> twiddles(int n) {
   return t;
 }
 
+// Split-BF16 products of a mixed-precision context (opt.gemm_split bits):
+// the Lambda gram, S, Psi T, the Lambda projection F -= w Psi Lambda.  The
+// projection and the rotation have a split kernel up to 128 states.
+constexpr int kSplitLambda = 1, kSplitS = 2, kSplitRot = 4, kSplitProj = 8;
+bool split_on(const oa_ctx* c, int bit) { return c->fp32 && (c->opt.gemm_split & bit) != 0; }
+
 // States per chunk for a grid of units x nchunk workgroups, occ resident per
 // CU.  A state costs a CU that holds k workgroups k + 1.5 units of time (fitted
 // to the plane passes: 5.6, 6.8, 8.6 us with 1, 2, 3 workgroups in FP32 at
@@ -697,16 +703,18 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
   TRY(dalloc(c, &c->S2, nn * sizeof(double)));
   TRY(dalloc(c, &c->T, nn * sizeof(double)));
   TRY(dalloc(c, &c->lam, nn * sizeof(double)));
-  // gram: one workgroup per (128 x 128 output block, K slice), about one
-  // workgroup per CU in all; the same slice count serves S and Lambda
+  // gram: one workgroup per (output block, K slice), about one or two
+  // workgroups per CU in all
   const int K = 2 * c->npts;
   int ncu = 0;
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) !=
           hipSuccess || ncu <= 0)
     ncu = 256;
   c->nslice_sym = oa::gram_slices(n, K, 2 * c->nkx0, 1, ncu);
-  c->nslice_full = oa::gram_slices(n, K, 2 * c->nkx0, 0, ncu);
-  int max_slice = std::max(c->nslice_sym, c->nslice_full);
+  const bool split_lam = split_on(c, kSplitLambda);
+  c->nslice_full = split_lam ? oa::gram_bf16_slices(n, K, ncu)
+                             : oa::gram_slices(n, K, 2 * c->nkx0, 0, ncu);
+  int max_sym = c->nslice_sym, max_full = c->nslice_full;
   if (c->opt.autotune) {
     // K slices: half, the heuristic and twice it (at least 2, at most K/64)
     auto cands = [&](int h) {
@@ -718,9 +726,13 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
     };
     c->tune_nslice_sym = cands(c->nslice_sym);
     c->tune_nslice_full = cands(c->nslice_full);
-    max_slice = std::max({max_slice, c->tune_nslice_sym.back(), c->tune_nslice_full.back()});
+    max_sym = std::max(max_sym, c->tune_nslice_sym.back());
+    max_full = std::max(max_full, c->tune_nslice_full.back());
   }
-  TRY(dalloc(c, &c->gpart, (size_t)max_slice * nn * sizeof(double)));
+  // the split product's partials are FP32
+  TRY(dalloc(c, &c->gpart,
+             nn * std::max(max_sym * sizeof(double),
+                           max_full * (split_lam ? sizeof(float) : sizeof(double)))));
   TRY(dalloc(c, &c->nsX0, nn * sizeof(double)));
   TRY(dalloc(c, &c->nsX1, nn * sizeof(double)));
   TRY(dalloc(c, &c->nsT0, nn * sizeof(double)));
@@ -1001,11 +1013,6 @@ oa_status st_r2g(oa_ctx* c, int ev0 = -1) {
   return st_energies(c);
 }
 
-// Split-BF16 products of a mixed-precision context (opt.gemm_split bits):
-// the Lambda gram, S, Psi T, the Lambda projection F -= w Psi Lambda.  The
-// projection and the rotation have a split kernel up to 128 states.
-constexpr int kSplitLambda = 1, kSplitS = 2, kSplitRot = 4, kSplitProj = 8;
-bool split_on(const oa_ctx* c, int bit) { return c->fp32 && (c->opt.gemm_split & bit) != 0; }
 bool split_rotate_ok(const oa_ctx* c) { return c->nst <= 128 && (2 * c->ld) % 64 == 0; }
 
 oa_status st_gram(oa_ctx* c, const double2* A, const double2* B, bool sym, double wlo, double whi,
