@@ -97,7 +97,8 @@ size_t plane3_kper(int n, int nplane_x, bool fp32, bool prune);  // 0 if n is no
 // order (VPerm); 0: none
 int plane_classes(int n, bool fp32, int* x1);
 // workgroups per plane of the G->R grid and resident workgroups per CU of both
-// passes; *rho_ok: those of the R->G pass with rho, 0 if it is not compiled
+// passes; *rho_ok, if not 0 on entry: those of the R->G pass with rho (0 if it
+// is not compiled)
 hipError_t plane3_info(int n, int nplane_x, bool fp32, bool prune, int* rowparts, int* occ_g2r,
                        int* occ_r2g, int* rho_ok);
 

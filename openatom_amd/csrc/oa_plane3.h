@@ -721,14 +721,17 @@ hipError_t plane3_info_l(int npx, int* rowparts, int* occ_g2r, int* occ_r2g, int
                        : (const void*)k3_g2r<T, X1, X2, Y1, Y2, NT, row_rounds<T, L>(), false, L>;
   const void* r = (const void*)k3_r2g<T, X1, X2, Y1, Y2, NT, VREG, false, L>;
   hipError_t e;
+  const bool want = *rho_ok != 0;
   *rho_ok = 0;
   // the R->G pass with rho accumulators spills at 512 threads
   if constexpr (r2g_rho_ok<X1, X2, NT>() && NT == kPlaneThreads) {
-    const void* h = (const void*)k3_r2g<T, X1, X2, Y1, Y2, NT, VREG, true, L>;
-    if ((e = oa::grant_lds(h, smem)) != hipSuccess ||
-        (e = hipOccupancyMaxActiveBlocksPerMultiprocessor(rho_ok, h, NT, smem)) != hipSuccess)
-      return e;
-    *rho_ok = *rho_ok > 1 ? *rho_ok : 1;
+    if (want) {
+      const void* h = (const void*)k3_r2g<T, X1, X2, Y1, Y2, NT, VREG, true, L>;
+      if ((e = oa::grant_lds(h, smem)) != hipSuccess ||
+          (e = hipOccupancyMaxActiveBlocksPerMultiprocessor(rho_ok, h, NT, smem)) != hipSuccess)
+        return e;
+      *rho_ok = *rho_ok > 1 ? *rho_ok : 1;
+    }
   }
   if ((e = oa::grant_lds(g, smem)) != hipSuccess || (e = oa::grant_lds(r, smem)) != hipSuccess)
     return e;

@@ -716,6 +716,7 @@ hipError_t plane4_info(int* rowparts, int* occ_g2r, int* occ_r2g, int* rho_ok) {
   using R = typename H::R;
   constexpr size_t sg = smem4<T, G>(), sr = smem4<T, R>();
   *rowparts = G::M;
+  const bool want = *rho_ok != 0;
   *rho_ok = 0;
   const void* g = (const void*)k4_g2r<T, G, false, false, H::WG>;
   const void* r = (const void*)k4_r2g<T, R, H::VREG, false, false, H::WR>;
@@ -723,11 +724,13 @@ hipError_t plane4_info(int* rowparts, int* occ_g2r, int* occ_r2g, int* rho_ok) {
   if ((e = oa::grant_lds(g, sg)) != hipSuccess || (e = oa::grant_lds(r, sr)) != hipSuccess)
     return e;
   if constexpr (rho_ok4<T, X1, X2>()) {
-    const void* h = (const void*)k4_r2g<T, R, H::VREG, true, false, 1>;
-    if ((e = oa::grant_lds(h, sr)) != hipSuccess ||
-        (e = hipOccupancyMaxActiveBlocksPerMultiprocessor(rho_ok, h, R::NT, sr)) != hipSuccess)
-      return e;
-    *rho_ok = *rho_ok > 1 ? *rho_ok : 1;
+    if (want) {
+      const void* h = (const void*)k4_r2g<T, R, H::VREG, true, false, 1>;
+      if ((e = oa::grant_lds(h, sr)) != hipSuccess ||
+          (e = hipOccupancyMaxActiveBlocksPerMultiprocessor(rho_ok, h, R::NT, sr)) != hipSuccess)
+        return e;
+      *rho_ok = *rho_ok > 1 ? *rho_ok : 1;
+    }
   }
   if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(occ_g2r, g, G::NT, sg)) != hipSuccess)
     return e;

@@ -485,7 +485,7 @@ oa_status build_layout(oa_ctx* c) {
       ncu = 256;
     // fused rho: every R->G chunk then writes one rho partial too, so its
     // chunk count is bounded like the G->R one's
-    c->fuse_rho = rho_ok && !c->opt.vks_from_rho;
+    c->fuse_rho = rho_ok > 0;
     const int max_r = c->fuse_rho ? std::min(c->nst, kMaxRhoChunks) : c->nst;
     // a rho partial is written and read back: 3.3 us at 100^3, where a unit of
     // the G->R pass is about 1 us; both scale with the points of a plane
@@ -1111,9 +1111,8 @@ oa_status st_lambda_cg(oa_ctx* c) {
                 split_on(c, kSplitProj) && split_rotate_ok(c)));
   HIPCHK(oa::reduce_to(c->fpart, lambda_nwg(c), 1.0, &c->res->fnorm2, c->stream));
   HIPCHK(oa::cg_gamma(c->res, c->cgs, c->stream));
-  HIPCHK(oa::cg_update(c->psi, c->cgdir, c->force, c->dtm, c->g2, c->ecut_ry, c->nst, c->npts,
-                       c->ld, c->cgs, c->stream));
-  HIPCHK(oa::red_sync(c->psi, c->red, c->partner, c->nred, c->nst, c->ld, c->stream));
+  HIPCHK(oa::cg_update(c->psi, c->cgdir, c->force, c->dtm, c->g2, c->sd_twin, c->ecut_ry, c->nst,
+                       c->npts, c->ld, c->cgs, c->stream));
   return OA_OK;
 }
 
