@@ -243,9 +243,9 @@ int rotate_nwg(int n, int K);  // workgroups of a rotate launch (fpart entries)
 // gram_bf16: the product of gram_f64 with FP32 partials part[nslice][n][nb]
 // (every block whole, also when sym), summed by gram_reduce_f32.
 hipError_t gram_bf16(const GramArgs& a, float* part, hipStream_t st);
-hipError_t gram_reduce_f32(const float* part, int nslice, int n, int nb, int sym, double alpha,
 // K slices of an n x n product on `target` CUs
 int gram_bf16_slices(int n, int K, int target);
+hipError_t gram_reduce_f32(const float* part, int nslice, int n, int nb, int sym, double alpha,
                            double* C, hipStream_t st);
 // rotate_bf16: the product of rotate_f64 for n, ni <= 128 and ldx a multiple
 // of 64 (no SD epilogue); fpart, if set, gets per-workgroup sums of Ynew^2
@@ -305,8 +305,8 @@ struct CgDev {
 hipError_t cg_gamma(const StepDev* res, CgDev* cg, hipStream_t st);
 // cg = gamma cg + F where g2 <= ecut; psi += dtm cg (cp_min_CG.C:55-105)
 hipError_t cg_update(double2* psi, double2* cgdir, const double2* f, const double* dtm,
-                     const double* g2, double ecut, int nst, int npts, int ld, const CgDev* cg,
-                     hipStream_t st);
+                     const double* g2, const int* twin, double ecut, int nst, int npts, int ld,
+                     const CgDev* cg, hipStream_t st);
 // psi += dtm[p] * F (cp_min_std.C:56-86); accumulates |F|^2 partials.
 // twin[p] (may be null): -1, or -2 for a redundant kx=0 point (not
 // written), or the redundant twin of p, which receives conj(new psi[p])

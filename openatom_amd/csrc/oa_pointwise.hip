@@ -87,39 +87,55 @@ hipError_t cg_gamma(const StepDev* res, CgDev* cg, hipStream_t st) {
   return hipGetLastError();
 }
 
-// cg = gamma cg + F where g2 <= ecut; psi += dt/m cg (cp_min_CG.C:55-105)
-__global__ void k_cg_update(double2* __restrict__ psi, double2* __restrict__ cgd,
-                            const double2* __restrict__ f, const double* __restrict__ dtm,
-                            const double* __restrict__ g2, double ecut, int nst, int npts, int ld,
-                            const CgDev* __restrict__ cg) {
+// cg = gamma cg + F where g2 <= ecut; psi += dt/m cg (cp_min_CG.C:55-105), and
+// the redundant kx=0 points from their partners (twin: -1, -2 for a redundant
+// point, or the index of the redundant twin, as in k_sd).  Block (b, s): 1024
+// points of state s, four per thread with every load issued before the first
+// use: five streams of 16 bytes per point at the rate of a copy (256 states x
+// 65,912 points 264 -> 132 us; one point per iteration and a division for its
+// state left too few bytes in flight).
+constexpr int kCgPer = 4;
+__global__ __launch_bounds__(256) void k_cg_update(
+    double2* __restrict__ psi, double2* __restrict__ cgd, const double2* __restrict__ f,
+    const double* __restrict__ dtm, const double* __restrict__ g2, const int* __restrict__ twin,
+    double ecut, int npts, int ld, const CgDev* __restrict__ cg) {
   const double gamma = cg->gamma;
-  const size_t tot = (size_t)nst * npts;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot;
-       e += (size_t)gridDim.x * blockDim.x) {
-    const int s = (int)(e / npts), p = (int)(e - (size_t)s * npts);
-    const size_t o = (size_t)s * ld + p;
-    double2 d = cgd[o];
-    if (g2[p] <= ecut) {
-      const double2 fv = f[o];
-      d.x = d.x * gamma + fv.x;
-      d.y = d.y * gamma + fv.y;
-      cgd[o] = d;
+  const size_t row = (size_t)blockIdx.y * ld;
+  const int p0 = blockIdx.x * (256 * kCgPer) + threadIdx.x;
+  double2 d[kCgPer], fv[kCgPer], c[kCgPer];
+  double m[kCgPer], gg[kCgPer];
+  int tw[kCgPer];
+#pragma unroll
+  for (int u = 0; u < kCgPer; u++) {
+    const int p = min(p0 + 256 * u, npts - 1);
+    d[u] = cgd[row + p];
+    fv[u] = f[row + p];
+    c[u] = psi[row + p];
+    m[u] = dtm[p];
+    gg[u] = g2[p];
+    tw[u] = twin[p];
+  }
+#pragma unroll
+  for (int u = 0; u < kCgPer; u++) {
+    const int p = p0 + 256 * u;
+    if (p >= npts) continue;
+    if (gg[u] <= ecut) {
+      d[u].x = d[u].x * gamma + fv[u].x;
+      d[u].y = d[u].y * gamma + fv[u].y;
+      cgd[row + p] = d[u];
     }
-    const double m = dtm[p];
-    double2 c = psi[o];
-    c.x += d.x * m;
-    c.y += d.y * m;
-    psi[o] = c;
+    c[u].x += d[u].x * m[u];
+    c[u].y += d[u].y * m[u];
+    if (tw[u] != -2) psi[row + p] = c[u];
+    if (tw[u] >= 0) psi[row + tw[u]] = make_double2(c[u].x, -c[u].y);
   }
 }
 
 hipError_t cg_update(double2* psi, double2* cgdir, const double2* f, const double* dtm,
-                     const double* g2, double ecut, int nst, int npts, int ld, const CgDev* cg,
-                     hipStream_t st) {
-  const size_t tot = (size_t)nst * npts;
-  int blocks = (int)std::min<size_t>((tot + 255) / 256, 4096);
-  hipLaunchKernelGGL(k_cg_update, dim3(blocks), dim3(256), 0, st, psi, cgdir, f, dtm, g2, ecut,
-                     nst, npts, ld, cg);
+                     const double* g2, const int* twin, double ecut, int nst, int npts, int ld,
+                     const CgDev* cg, hipStream_t st) {
+  hipLaunchKernelGGL(k_cg_update, dim3((npts + 256 * kCgPer - 1) / (256 * kCgPer), nst),
+                     dim3(256), 0, st, psi, cgdir, f, dtm, g2, twin, ecut, npts, ld, cg);
   return hipGetLastError();
 }
 

@@ -475,7 +475,8 @@ oa_status build_layout(oa_ctx* c) {
   if (c->engine == kEngPlane) {
     // State chunks of both plane passes from the resident-workgroup count
     // (every G->R chunk also writes one rho partial of N doubles)
-    int rowparts = 1, occ_g = 1, occ_r = 1, rho_ok = 0, ncu = 0;
+    // the R->G pass with rho is only for a V that does not depend on rho
+    int rowparts = 1, occ_g = 1, occ_r = 1, rho_ok = c->opt.vks_from_rho ? 0 : 1, ncu = 0;
     if (oa::plane3_info(c->nx, c->nplane_x, c->fp32, f.prune != 0, &rowparts, &occ_g, &occ_r,
                         &rho_ok) !=
         hipSuccess)
