@@ -83,23 +83,23 @@ typedef struct {
                           the second call; the Newton-Schulz launch stays outside); stage
                           timings then read: [0] everything before Newton-Schulz, [8]
                           Newton-Schulz, [9] Psi T (+ residual), [12] whole step */
-  int ns_mode;         /* 0: one cooperative launch when all workgroups fit (default; the
-                          autotuner picks among the forms below that fit),
+  int ns_mode;         /* 0: plain launches (default): one workgroup for n <= 64, above it
+                          two launches per iteration for the iterations expected and one
+                          that runs any others,
                           1: two launches per iteration with a device-side early exit,
                           2: one cooperative launch over 32 x 32 tiles,
                           3, 4, 5: one cooperative launch over 16-row blocks, each split
                           over 1, 2 or 4 workgroups by 16-column tiles (4 and 5 need
                           n > 16 and n > 48); 2..5 give OA_EINVAL where they do not fit;
-                          6: no cooperative launch: one plain launch of one workgroup for
-                          n <= 64, else as 1 (for contexts that share the device) */
+                          6: as 0 (no cooperative launch, for contexts that share the
+                          device) */
   int vks_from_rho;    /* 1: each step builds V(r) = V_KS[rho] from its own density
                           (PZ-LDA exchange-correlation, Hartree, local pseudopotential of
                           oa_local_pseudo_set) between rho and V psi, as the density chares
                           do; 0 (default): V(r) is the input of oa_vks_set */
   int autotune;        /* 1: oa_create times candidate launch shapes on the device and keeps
                           the fastest: state chunks of the two plane passes, K slices of
-                          the S and Lambda products, Newton-Schulz as one cooperative launch
-                          or two launches per iteration.  Chunking changes the order of the
+                          the S and Lambda products.  Chunking changes the order of the
                           rho sums (rounding only).  0 (default): fixed heuristics */
   int gemm_split;      /* mixed precision only: products run as split-BF16 matrix-core
                           products (each FP64 operand rounded to FP32 and split exactly into

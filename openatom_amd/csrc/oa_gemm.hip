@@ -1036,58 +1036,109 @@ __global__ __launch_bounds__(256) void k_ns_coop(NsArgs a) {
   }
 }
 
-// One workgroup for the whole iteration, a plain launch (n <= kNsOneMax):
-// the recurrence of k_ns_coop with the workgroup visiting every 32 x 32 tile
-// in turn and workgroup barriers in place of the grid barriers.  For the
-// small matrices of small requests this replaces 2 max_iter + 2 launches per
-// step (most of them early exits) by one, with no cooperative launch.
-__global__ __launch_bounds__(256) void k_ns_one(NsArgs a) {
+// One workgroup for the whole iteration, a plain launch (n <= kNsOneMax): X, T
+// and C stay in LDS (zero past n, odd row stride), a wave computes 16 x 16 tiles;
+// the new X = C X / 2 and T = C T / 2 (X, T and C commute, so C X = X C up to
+// rounding) wait in registers until every wave has read the old ones.  Bound by
+// the matrix pipe of one CU at n = 64 and by the dependent products and three
+// barriers per iteration below; no operand leaves the CU.  The stage of a step
+// (4 to 5 iterations) takes 15 us at 16 states, and 64 states 37; the cooperative
+// and single-workgroup forms through global memory took 49 and 50.
+__global__ __launch_bounds__(1024) void k_ns_one(NsArgs a) {
+  constexpr int LD = kNsOneMax + 1;
   extern __shared__ __align__(16) double ns_smem[];
-  const int n = a.n, nt = (n + NT - 1) / NT, ntile = nt * nt;
-  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4, wave = threadIdx.x >> 6;
-  const int wr = (wave >> 1) * 16, wc = (wave & 1) * 16;
-  for (int e = threadIdx.x; e < n * n; e += 256) {
-    a.X0[e] = 0.5 * a.S[e];  // B = S/2 (ortho.C:236-239)
-    a.T0[e] = (e / n == e % n) ? 1.0 : 0.0;
+  __shared__ double red[16];
+  double *X = ns_smem, *T = X + kNsOneMax * LD, *C = T + kNsOneMax * LD;
+  const int n = a.n, nt = (n + 15) >> 4, np = 16 * nt, tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int nw = blockDim.x >> 6;
+  for (int e = tid; e < np * np; e += blockDim.x) {
+    const int r = e / np, c = e - r * np;
+    const bool in = r < n && c < n;
+    X[r * LD + c] = in ? 0.5 * a.S[(size_t)r * n + c] : 0.0;  // B = S/2 (ortho.C:236-239)
+    T[r * LD + c] = in && r == c ? 1.0 : 0.0;
   }
   __syncthreads();
-  double* X[2] = {a.X0, a.X1};
-  double* T[2] = {a.T0, a.T1};
+  // rows 16 ti.. of A times columns 16 tj.. of B
+  auto product = [&](const double* A, const double* B, int ti, int tj) {
+    const double* ap = A + (16 * ti + l16) * LD + g;
+    const double* bp = B + g * LD + 16 * tj + l16;
+    v4d p0 = vzero(), p1 = vzero();
+    for (int k = 0; k < np; k += 16) {  // two accumulator chains
+      p0 = mfma16(ap[k], bp[k * LD], p0);
+      p1 = mfma16(ap[k + 4], bp[(k + 4) * LD], p1);
+      p0 = mfma16(ap[k + 8], bp[(k + 8) * LD], p0);
+      p1 = mfma16(ap[k + 12], bp[(k + 12) * LD], p1);
+    }
+    return p0 + p1;
+  };
   int conv = 0;
   double err = 0.0;
   for (int it = 1; it <= a.max_iter; it++) {
-    const int o = (it - 1) & 1, w = it & 1;
-    v4d p1, p2;
-    for (int t = 0; t < ntile; t++) {  // C = 3I - T X
-      const int r0 = (t / nt) * NT, c0 = (t % nt) * NT;
-      ns_tile2(T[o], X[o], nullptr, nullptr, n, r0, c0, ns_smem, p1, p2);
-      blk_store(a.C, p1, n, r0 + wr, c0 + wc, -1.0, 3.0, nullptr);
+    for (int t = wave; t < nt * nt; t += nw) {  // C = 3I - T X
+      const int ti = t / nt, tj = t - ti * nt;
+      const v4d p = product(T, X, ti, tj);
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int r = 16 * ti + g + 4 * v, c = 16 * tj + l16;
+        C[r * LD + c] = (r == c && r < n ? 3.0 : 0.0) - p[v];
+      }
     }
     __syncthreads();
+    // tiles q = wave and wave + nw of the 2 nt^2: the X tiles, then the T tiles
+    v4d p[2];
     double e = 0.0;
-    for (int t = 0; t < ntile; t++) {  // X' = X C / 2, T' = C T / 2
-      const int r0 = (t / nt) * NT, c0 = (t % nt) * NT;
-      ns_tile2(X[o], a.C, a.C, T[o], n, r0, c0, ns_smem, p1, p2);
-      blk_store(X[w], p1, n, r0 + wr, c0 + wc, 0.5, 0.0, nullptr);
-      e += blk_store(T[w], p2, n, r0 + wr, c0 + wc, 0.5, 0.0, T[o]);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int q = wave + i * nw, t = q < nt * nt ? q : q - nt * nt;
+      if (q >= 2 * nt * nt) continue;
+      const int ti = t / nt, tj = t - ti * nt;
+      const double* D = q < nt * nt ? X : T;
+      p[i] = product(C, D, ti, tj) * 0.5;
+      if (q >= nt * nt)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const double d = T[(16 * ti + g + 4 * v) * LD + 16 * tj + l16] - p[i][v];
+          e += d * d;
+        }
     }
-    err = sqrt(wg_sum(e) / ((double)n * n));  // wg_sum ends with a barrier
+    for (int off = 32; off > 0; off >>= 1) e += __shfl_down(e, off, 64);
+    if (lane == 0) red[wave] = e;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int q = wave + i * nw, t = q < nt * nt ? q : q - nt * nt;
+      if (q >= 2 * nt * nt) continue;
+      const int ti = t / nt, tj = t - ti * nt;
+      double* D = q < nt * nt ? X : T;
+#pragma unroll
+      for (int v = 0; v < 4; v++) D[(16 * ti + g + 4 * v) * LD + 16 * tj + l16] = p[i][v];
+    }
+    double sum = 0.0;
+    for (int w = 0; w < nw; w++) sum += red[w];
+    err = sqrt(sum / ((double)n * n));
+    __syncthreads();
     if (err <= a.tol) {
       conv = it;
       break;
     }
   }
-  const int last = conv ? conv : a.max_iter;
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     a.res->ns_iter = conv ? conv : -a.max_iter;
     a.res->ns_err = err;
   }
-  const double* Tf = T[last & 1];
-  for (int e = threadIdx.x; e < n * n; e += 256) a.Tout[e] = Tf[e];
-  (void)lane;
-  (void)l16;
-  (void)g;
+  for (int e = tid; e < n * n; e += blockDim.x) {
+    const int r = e / n, c = e - r * n;
+    a.Tout[e] = T[r * LD + c];
+  }
 }
+
+// threads of a k_ns_one launch: a wave per two of the 2 nt^2 tiles, at most 16
+static int ns_one_threads(int n) {
+  const int nt = (n + 15) / 16;
+  return 64 * std::min(16, nt * nt);
+}
+constexpr size_t kNsOneSmem = (size_t)3 * kNsOneMax * (kNsOneMax + 1) * sizeof(double);
 
 // ---- fallback: two launches per iteration with a device-side early exit
 
@@ -1657,6 +1708,248 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
   }
 }
 
+// ---- plain launches by tiles, then one that finishes
+//
+// A launch boundary takes the place of the grid barrier: about 3 us against 30 us
+// for entering a cooperative launch and 8 us per barrier.  C = 3I - T X in one
+// launch, X' = C X / 2 and T' = C T / 2 in the next; a workgroup computes one
+// tile of 16 R rows and columns, its eight waves sharing the sum over k (four to
+// a product where there are two), all loads of a wave in flight at once: these
+// products are bound by the latency of reading what the last launch wrote
+// through another XCD's L2.  The first iteration starts from T0 = I and X0 =
+// S/2 (ortho.C:236-239) and needs one launch.  The convergence test (the last
+// iteration's partials, summed in the same order by every workgroup) overlaps
+// the product, and only the stores depend on it.  Iterations after convergence
+// return at once; where the last call's count is known one more than that is
+// launched, and k_nl_tail, one workgroup, runs any others by the same code in the
+// same order, so the result does not depend on how many were launched.  T goes to
+// Tout in every iteration.  The stage takes 70 us at 84, 128 and 180 states, 95 at
+// 256 and 174 at 512 (4 to 6 iterations); the cooperative forms took 103, 91, 186,
+// 280 and, over 32 x 32 tiles, 623.
+constexpr int kNlThreads = 512;
+// iterations launched where no count is known: get_iter_Tmat's limit (cp_lowdin.C:212)
+constexpr int kNlLaunch = 10;
+enum { kNlC, kNlXT, kNlFirst };
+
+struct NlBuf {
+  const double *To, *Xo;
+  double *Tw, *Xw;
+};
+__device__ __forceinline__ NlBuf nl_buf(const NsArgs& a, int it) {  // X_k, T_k in buffer k & 1
+  return (it & 1) ? NlBuf{a.T0, a.X0, a.T1, a.X1} : NlBuf{a.T1, a.X1, a.T0, a.X0};
+}
+
+// Partial sums over this wave's share s of ks of k (chunks of 16) of rows 16 R ti..
+// times columns 16 R tj.. into part[e]; lane group g takes k = 4 g .. 4 g + 3 of a
+// chunk.  A past column n counts as zero, addresses are clamped to the matrix.
+template <int R, bool FIRST>
+__device__ __forceinline__ void nl_product(const double* __restrict__ A,
+                                           const double* __restrict__ B, int n, int ti, int tj,
+                                           int s, int ks, double* __restrict__ part) {
+  constexpr int CB = 4;  // chunks per batch of loads
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int nch = (n + 15) >> 4, q = (nch + ks - 1) / ks, end = min(nch, (s + 1) * q);
+  unsigned ar[R], bc[R];
+  int row[R];
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    row[i] = 16 * (R * ti + i) + l16;
+    ar[i] = (unsigned)min(row[i], n - 1) * (unsigned)n;
+    bc[i] = (unsigned)min(16 * (R * tj + i) + l16, n - 1);
+  }
+  v4d acc[R][R];
+#pragma unroll
+  for (int i = 0; i < R * R; i++) acc[i / R][i % R] = vzero();
+  for (int c0 = s * q; c0 < end; c0 += CB) {
+    double av[R][4 * CB], bv[R][4 * CB];
+#pragma unroll
+    for (int u = 0; u < 4 * CB; u++) {
+      const int k = 16 * (c0 + u / 4) + 4 * g + (u & 3);
+      const unsigned kc = min(k, n - 1);
+#pragma unroll
+      for (int i = 0; i < R; i++) {
+        av[i][u] = A[ar[i] + kc];
+        bv[i][u] = B[kc * (unsigned)n + bc[i]];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4 * CB; u++) {
+      const int k = 16 * (c0 + u / 4) + 4 * g + (u & 3);
+      const bool in = k < n && c0 + u / 4 < end;
+#pragma unroll
+      for (int i = 0; i < R; i++) {
+        if constexpr (FIRST) {  // C = 3I - S/2, X0 = S/2
+          av[i][u] = (row[i] == k ? 3.0 : 0.0) - 0.5 * av[i][u];
+          bv[i][u] = 0.5 * bv[i][u];
+        }
+        av[i][u] = in ? av[i][u] : 0.0;
+      }
+#pragma unroll
+      for (int i = 0; i < R * R; i++)
+        acc[i / R][i % R] = mfma16(av[i / R][u], bv[i % R][u], acc[i / R][i % R]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < R * R; i++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) part[(4 * i + v) * 64 + lane] = acc[i / R][i % R][v];
+}
+
+// Tile (ti, tj) of one launch's work in iteration it.  check: stop where the
+// iteration has converged.  Ends with a barrier when check is off.
+template <int R, int MODE>
+__device__ __forceinline__ void nl_tile(const NsArgs& a, int it, int ti, int tj, int nt,
+                                        bool check, double* part) {
+  __shared__ double red[8];
+  constexpr int NP = MODE == kNlXT ? 2 : 1, KS = 8 / NP, E = 256 * R * R, TP = kNlThreads / NP;
+  constexpr int NE = (E + TP - 1) / TP;
+  const int n = a.n, nwg = nt * nt, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const NlBuf q = nl_buf(a, it);
+  const int m = tid / TP;  // which product's elements this thread finishes
+  int done = 0;
+  double es = 0.0;
+  if (MODE != kNlFirst && check) done = *(const volatile int*)&a.res->ns_iter;
+  if (done != 0) return;  // one more wait, but idle launches take 1.2 us
+  if (MODE == kNlC && check)
+    for (int i = tid; i < nwg; i += kNlThreads) es += a.errpart[(size_t)(it - 1) * nwg + i];
+  int row[NE], col[NE];
+  double old[NE];
+#pragma unroll
+  for (int i = 0; i < NE; i++) {
+    const int e = tid % TP + i * TP, t = e >> 8;
+    row[i] = e < E ? 16 * (R * ti + t / R) + ((e & 63) >> 4) + 4 * ((e >> 6) & 3) : n;
+    col[i] = 16 * (R * tj + t % R) + (e & 15);
+    old[i] = 0.0;
+    if (MODE != kNlC)  // the T element before this iteration (first: of S)
+      old[i] = (MODE == kNlFirst ? a.S : q.To)[(size_t)min(row[i], n - 1) * n + min(col[i], n - 1)];
+  }
+  if constexpr (MODE == kNlFirst)
+    nl_product<R, true>(a.S, a.S, n, ti, tj, wave, KS, part + wave * E);
+  else if constexpr (MODE == kNlC)
+    nl_product<R, false>(q.To, q.Xo, n, ti, tj, wave, KS, part + wave * E);
+  else
+    nl_product<R, false>(a.C, wave < KS ? q.Xo : q.To, n, ti, tj, wave % KS, KS, part + wave * E);
+  if (MODE == kNlC && check) {
+    for (int off = 32; off > 0; off >>= 1) es += __shfl_down(es, off, 64);
+    if (lane == 0) red[wave] = es;
+  }
+  __syncthreads();
+  if (MODE == kNlC && check) {
+    double s = 0.0;
+    for (int w = 0; w < 8; w++) s += red[w];
+    const double err = sqrt(s / ((double)n * n));
+    if (err <= a.tol) {
+      if (ti == 0 && tj == 0 && tid == 0) {
+        a.res->ns_iter = it - 1;
+        a.res->ns_err = err;
+      }
+      return;
+    }
+  }
+  double e2 = 0.0;
+#pragma unroll
+  for (int i = 0; i < NE; i++) {
+    const int e = tid % TP + i * TP;
+    if (row[i] >= n || col[i] >= n) continue;
+    double p = 0.0;
+#pragma unroll
+    for (int s = 0; s < KS; s++) p += part[(m * KS + s) * E + e];
+    const size_t o = (size_t)row[i] * n + col[i];
+    const double one = row[i] == col[i] ? 1.0 : 0.0;
+    if constexpr (MODE == kNlC) {
+      a.C[o] = 3.0 * one - p;
+    } else {
+      double nv = 0.5 * p, before = old[i];
+      if (m == 0) q.Xw[o] = nv;
+      if constexpr (MODE == kNlFirst) {  // T1 = C / 2
+        before = one;
+        nv = 0.5 * (3.0 * one - 0.5 * old[i]);
+      }
+      if (MODE == kNlFirst || m == 1) {
+        q.Tw[o] = nv;
+        a.Tout[o] = nv;
+        e2 += (before - nv) * (before - nv);
+      }
+    }
+  }
+  if constexpr (MODE != kNlC) {
+    for (int off = 32; off > 0; off >>= 1) e2 += __shfl_down(e2, off, 64);
+    if (lane == 0) red[wave] = e2;
+    __syncthreads();
+    if (tid == 0) {
+      double s = 0.0;
+      for (int w = 0; w < 8; w++) s += red[w];
+      a.errpart[(size_t)it * nwg + ti * nt + tj] = s;
+    }
+    if (MODE == kNlFirst && ti == 0 && tj == 0 && tid == 0) {
+      a.res->ns_iter = 0;
+      a.res->ns_err = 0.0;
+    }
+  }
+  if (!check) __syncthreads();
+}
+
+template <int R, int MODE>
+__global__ __launch_bounds__(kNlThreads) void k_nl(NsArgs a, int it) {
+  extern __shared__ __align__(16) double nl_smem[];
+  nl_tile<R, MODE>(a, it, blockIdx.y, blockIdx.x, gridDim.x, true, nl_smem);
+}
+
+// After `launched` iterations: records convergence of the last one, or runs the
+// rest, up to max_iter, in one workgroup
+template <int R>
+__global__ __launch_bounds__(kNlThreads) void k_nl_tail(NsArgs a, int launched, int nt) {
+  extern __shared__ __align__(16) double nl_smem[];
+  __shared__ double part[kNlThreads / 64];
+  const int nwg = nt * nt, tid = threadIdx.x;
+  if (*(const volatile int*)&a.res->ns_iter != 0) return;  // the same in every thread
+  for (int it = launched;; it++) {
+    double es = 0.0;
+    for (int i = tid; i < nwg; i += kNlThreads) es += a.errpart[(size_t)it * nwg + i];
+    for (int off = 32; off > 0; off >>= 1) es += __shfl_down(es, off, 64);
+    __syncthreads();
+    if ((tid & 63) == 0) part[tid >> 6] = es;
+    __syncthreads();
+    es = 0.0;
+    for (int w = 0; w < kNlThreads / 64; w++) es += part[w];
+    const double err = sqrt(es / ((double)a.n * a.n));
+    if (err <= a.tol || it >= a.max_iter) {
+      if (tid == 0) {
+        a.res->ns_iter = err <= a.tol ? it : -a.max_iter;
+        a.res->ns_err = err;
+      }
+      return;
+    }
+    for (int w = 0; w < nwg; w++) nl_tile<R, kNlC>(a, it + 1, w / nt, w % nt, nt, false, nl_smem);
+    __threadfence();
+    __syncthreads();
+    for (int w = 0; w < nwg; w++) nl_tile<R, kNlXT>(a, it + 1, w / nt, w % nt, nt, false, nl_smem);
+    __threadfence();
+    __syncthreads();
+  }
+}
+
+template <int R>
+static hipError_t ns_steps_r(const NsArgs& a, hipStream_t st) {
+  const int nt = (a.n + 16 * R - 1) / (16 * R);
+  const size_t sm = (size_t)8 * 256 * R * R * sizeof(double);
+  for (const void* f : {(const void*)k_nl<R, kNlC>, (const void*)k_nl<R, kNlXT>,
+                        (const void*)k_nl<R, kNlFirst>, (const void*)k_nl_tail<R>})
+    if (const hipError_t e = grant_lds(f, sm); e != hipSuccess) return e;
+  const int count = std::min(a.max_iter, a.hint > 0 ? a.hint + 1 : kNlLaunch);
+  const dim3 grid(nt, nt), thr(kNlThreads);
+  hipLaunchKernelGGL((k_nl<R, kNlFirst>), grid, thr, sm, st, a, 1);
+  for (int it = 2; it <= count; it++) {
+    hipLaunchKernelGGL((k_nl<R, kNlC>), grid, thr, sm, st, a, it);
+    hipLaunchKernelGGL((k_nl<R, kNlXT>), grid, thr, sm, st, a, it);
+  }
+  hipLaunchKernelGGL(k_nl_tail<R>, dim3(1), thr, sm, st, a, count, nt);
+  return hipGetLastError();
+}
+static hipError_t ns_run_steps(const NsArgs& a, hipStream_t st) {
+  return ns_steps_r_of(a.n) == 1 ? ns_steps_r<1>(a, st) : ns_steps_r<2>(a, st);
+}
+
 static const void* nr_kernel(int n) {
   switch (nr_kb(n)) {
     case 8: return (const void*)k_ns_rows<8>;
@@ -1714,11 +2007,12 @@ bool ns_coop_possible(int n, int device) {
 
 hipError_t ns_run(const NsArgs& a, hipStream_t st) {
   if (!a.coop) return ns_run_launches(a, st);
+  if (a.coop == kNsStepsKind) return ns_run_steps(a, st);
   if (a.coop == kNsOneKind) {
     if (a.n > kNsOneMax) return ns_run_launches(a, st);
-    const hipError_t e = grant_lds((const void*)k_ns_one, kNsSmem);
+    const hipError_t e = grant_lds((const void*)k_ns_one, kNsOneSmem);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_ns_one, dim3(1), dim3(256), kNsSmem, st, a);
+    hipLaunchKernelGGL(k_ns_one, dim3(1), dim3(ns_one_threads(a.n)), kNsOneSmem, st, a);
     return hipGetLastError();
   }
   NsArgs args = a;

@@ -268,10 +268,20 @@ struct NsArgs {
              // tiles (two grid barriers per iteration); 2, 3, 4: one cooperative launch
              // over 16-row blocks, each split over 1, 2 or 4 workgroups by column
              // tiles (one barrier per iteration); kNsOneKind: one workgroup, a plain
-             // launch, for n <= kNsOneMax (two launches per iteration above)
+             // launch, for n <= kNsOneMax (two launches per iteration above);
+             // kNsStepsKind: two plain launches per iteration by small tiles for
+             // the iterations expected, one more that runs any others
+  int hint;  // kNsStepsKind: iterations the last call took, 0 if not known
 };
 constexpr int kNsOneKind = 5;
 constexpr int kNsOneMax = 64;
+constexpr int kNsStepsKind = 6;
+// kNsStepsKind: 16-tiles per side of a workgroup's tile, workgroups of a launch
+constexpr int ns_steps_r_of(int n) { return n <= 256 ? 1 : 2; }
+constexpr int ns_steps_wgs(int n) {
+  const int t = 16 * ns_steps_r_of(n), nt = (n + t - 1) / t;
+  return nt * nt;
+}
 hipError_t ns_run(const NsArgs& a, hipStream_t st);
 // FP32 work space of the mixed-precision Newton-Schulz: X and T (double
 // buffered) and C, n x n floats each

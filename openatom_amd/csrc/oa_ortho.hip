@@ -24,14 +24,13 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // Bytes of each part of the work space for n states and max_iter iterations.
 struct NsWork {
   size_t mat;    // one n x n matrix (256-byte granules)
-  size_t err;    // error partials: (max_iter + 2) x the largest workgroup count
+  size_t err;    // error partials: (max_iter + 2) x the workgroup count
   size_t res;    // StepDev
   size_t total;  // 5 mat + err + res
 };
 
 constexpr NsWork ns_work(int n, int max_iter) {
-  const size_t nt = (size_t)(n + 31) / 32, nb = (size_t)(n + 15) / 16;
-  const size_t nwg = std::max(nt * nt, (size_t)oa::kNsRowsMaxSplit * nb);
+  const size_t nwg = oa::ns_steps_wgs(n);
   NsWork w{};
   w.mat = align256((size_t)n * n * sizeof(double));
   w.err = align256((size_t)(max_iter + 2) * nwg * sizeof(double));
@@ -58,15 +57,6 @@ oa::NsArgs ns_args(const double* S, double* T, unsigned char* base, int n, int m
   a.max_iter = max_iter;
   a.tol = tol;
   return a;
-}
-
-// The fastest Newton-Schulz form that fits this device: one cooperative
-// launch over 16-row blocks (split over 4, 2, 1 workgroups), over 32 x 32
-// tiles, else two launches per iteration.
-int ns_kind(int n, int device) {
-  for (int kind = 4; kind >= 2; kind--)
-    if (oa::ns_rows_possible(n, oa::ns_rows_split(kind), device)) return kind;
-  return oa::ns_coop_possible(n, device) ? 1 : 0;
 }
 
 // Iterations used (> 0) or -max_iter, read back after the stream drains.
@@ -140,7 +130,7 @@ oa_status oa_ortho_transform(double* T, const double* S, int n) {
   if (s == OA_OK && hipMemcpyAsync(dS, S, nn, hipMemcpyHostToDevice, st) != hipSuccess) s = OA_EHIP;
   if (s == OA_OK) {
     oa::NsArgs a = ns_args(dS, dT, work, n, max_iter, tol);
-    a.coop = ns_kind(n, dev);
+    a.coop = n <= oa::kNsOneMax ? oa::kNsOneKind : oa::kNsStepsKind;
     if (oa::ns_run(a, st) != hipSuccess) s = OA_EHIP;
     if (s == OA_OK) s = ns_finish(a.res, st, nullptr);
     // T is returned also when the iteration missed its tolerance
@@ -171,7 +161,7 @@ oa_status oa_ortho_transform_noalloc(double* T, const double* S, int n) {
   double* dT = reinterpret_cast<double*>(d.ptr + w.total + kNoAllocMat);
   if (hipMemcpyAsync(dS, S, nn, hipMemcpyHostToDevice, d.st) != hipSuccess) return OA_EHIP;
   oa::NsArgs a = ns_args(dS, dT, d.ptr, n, kOrthoMaxIter, kOrthoTol);
-  a.coop = ns_kind(n, dev);
+  a.coop = n <= oa::kNsOneMax ? oa::kNsOneKind : oa::kNsStepsKind;
   if (oa::ns_run(a, d.st) != hipSuccess) return OA_EHIP;
   oa_status s = ns_finish(a.res, d.st, nullptr);
   if ((s == OA_OK || s == OA_ENOCONV) &&

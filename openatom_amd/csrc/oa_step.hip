@@ -176,10 +176,8 @@ struct oa_ctx {
   std::vector<hipEvent_t> ev;  // [kRing][OA_NTIMINGS] once timing is enabled
   int ev_cur = 0, ev_count = 0;
   bool have_S = false, have_T = false, have_v = false;
-  // Newton-Schulz: 0 two launches per iteration, 1 one cooperative launch
-  // over 32 x 32 tiles, 2 one cooperative launch over 16-row blocks
-  int ns_kind = 0;
-  std::vector<int> ns_kinds;  // the kinds this context can run
+  int ns_kind = 0;  // Newton-Schulz form: NsArgs::coop
+  int ns_seen = 0;  // iterations of the last result fetched (0: none yet)
   bool sd_fused = false;  // SD update inside the Lambda rotate (nst <= 128)
   int engine = 0;     // kEngFft2, kEngSep, kEngFused or kEngPlane
   // plane engine with V fixed during the step: rho partials come from the
@@ -750,25 +748,17 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
   // per-workgroup error partials of either cooperative kind
   TRY(dalloc(c, &c->errpart,
              (size_t)(c->opt.ns_max_iter + 2) *
-                 std::max(nt * nt, oa::kNsRowsMaxSplit * ((n + 15) / 16)) * sizeof(double)));
-  c->ns_kinds.clear();
+                 std::max({nt * nt, oa::kNsRowsMaxSplit * ((n + 15) / 16), oa::ns_steps_wgs(n)}) *
+                 sizeof(double)));
   const int nsm = c->opt.ns_mode;
-  if (nsm == 0) {
-    // row blocks split over 4, 2 or 1 workgroups (kinds 4, 3, 2)
-    for (int kind = 4; kind >= 2; kind--)
-      if (!c->dry && oa::ns_rows_possible(n, oa::ns_rows_split(kind), c->device))
-        c->ns_kinds.push_back(kind);
-    if (!c->dry && oa::ns_coop_possible(n, c->device)) c->ns_kinds.push_back(1);
-    if (n <= oa::kNsOneMax) c->ns_kinds.push_back(oa::kNsOneKind);
-    c->ns_kinds.push_back(0);
+  if (nsm == 0 || nsm == 6) {  // plain launches; faster than every other form at any n
+    c->ns_kind = n <= oa::kNsOneMax ? oa::kNsOneKind : oa::kNsStepsKind;
   } else if (nsm == 1) {
-    c->ns_kinds.push_back(0);
-  } else if (nsm == 6) {  // no cooperative launch
-    c->ns_kinds.push_back(n <= oa::kNsOneMax ? oa::kNsOneKind : 0);
+    c->ns_kind = 0;
   } else if (nsm == 2) {
     if (!c->dry && !oa::ns_coop_possible(n, c->device))
       return fail(c, OA_EINVAL, "ns_mode 2: the 32 x 32 tiles of n do not fit on the device at once");
-    c->ns_kinds.push_back(1);
+    c->ns_kind = 1;
   } else if (nsm >= 3 && nsm <= 5) {
     const int kind = nsm - 1;
     if (!c->dry && !oa::ns_rows_possible(n, oa::ns_rows_split(kind), c->device))
@@ -776,11 +766,10 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
                   "ns_mode " + std::to_string(nsm) +
                       ": the row blocks of n (16 rows each, split over that many workgroups "
                       "by 16-column tiles) do not fit on the device at once");
-    c->ns_kinds.push_back(kind);
+    c->ns_kind = kind;
   } else {
     return fail(c, OA_EINVAL, "ns_mode must be 0..6");
   }
-  c->ns_kind = c->ns_kinds.front();
   c->sd_fused = false;  // measured slower than a separate SD pass (registers)
   // |F|^2 partials: one per workgroup of the SD kernel or of the rotate that
   // applies Lambda and the SD update together
@@ -1196,6 +1185,7 @@ oa_status st_ns(oa_ctx* c, double tol, int max_iter) {
   a.max_iter = max_iter;
   a.tol = tol;
   a.coop = c->ns_kind;
+  a.hint = c->ns_seen;
   if (c->fp32 && c->opt.ns_fp32)
     HIPCHK(oa::ns_run_mixed(a, c->ns32, c->stream));
   else
@@ -1223,6 +1213,7 @@ void drop_graphs(oa_ctx* c) {
 oa_status fetch_result(oa_ctx* c, oa_step_out* out) {
   HIPCHK(hipMemcpyAsync(c->res_host, c->res, sizeof(StepDev), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  c->ns_seen = std::abs(c->res_host->ns_iter);
   if (out) {
     const StepDev& r = *c->res_host;
     out->eke = r.eke;
@@ -1380,19 +1371,6 @@ oa_status autotune(oa_ctx* c) {
       [&]() {
         return st_gram(c, c->psi, c->force, false, 0.5, 1.0, c->lam, split_on(c, kSplitLambda));
       });
-  if (c->ns_kinds.size() > 1) {
-    // S = 2I converges in one iteration: the cost of one iteration either way
-    std::vector<double> two((size_t)c->nst * c->nst, 0.0);
-    for (int i = 0; i < c->nst; i++) two[(size_t)i * c->nst + i] = 2.0;
-    HIPCHK(hipMemcpy(c->S, two.data(), two.size() * sizeof(double), hipMemcpyHostToDevice));
-    tune_knob(
-        c, e0, e1,
-        "Newton-Schulz row blocks split over 4, 2, 1 workgroups (4, 3, 2), cooperative tiles (1), "
-        "one workgroup (5) or launches (0)",
-        c->ns_kinds,
-        c->ns_kind, [&](int v) { c->ns_kind = v; },
-        [&]() { return st_ns(c, c->opt.ns_tol, c->opt.ns_max_iter); });
-  }
   if (c->nst <= 128 && c->opt.use_lambda && !c->opt.use_cg) {
     // F = 0 and psi = 0 at creation: the SD update leaves psi as it is
     tune_knob(
@@ -1641,6 +1619,7 @@ static oa_status copy_g(oa_ctx* c, double2* dev, const double* host, bool in) {
 
 oa_status oa_psi_set(oa_ctx* c, const double* psi) {
   if (!c || !psi) return OA_EINVAL;
+  c->ns_seen = 0;
   if (c->opt.use_cg) {  // a new minimisation: zero direction, iteration 0
     HIPCHK(hipSetDevice(c->device));
     const size_t gsz = (size_t)c->nst * c->ld * sizeof(double2);
