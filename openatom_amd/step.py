@@ -115,7 +115,7 @@ class CPContext:
         self._chk(self._L.oa_psi_set(self.h, ptr(a)))
 
     def get_psi(self):
-        a = np.zeros((self.nst, self.npts), np.complex128)
+        a = np.empty((self.nst, self.npts), np.complex128)
         self._chk(self._L.oa_psi_get(self.h, ptr(a)))
         return a
 
@@ -125,7 +125,7 @@ class CPContext:
         self._chk(self._L.oa_vks_set(self.h, ptr(a)))
 
     def get_force(self):
-        a = np.zeros((self.nst, self.npts), np.complex128)
+        a = np.empty((self.nst, self.npts), np.complex128)
         self._chk(self._L.oa_force_get(self.h, ptr(a)))
         return a
 
