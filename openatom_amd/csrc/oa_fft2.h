@@ -70,6 +70,55 @@ constexpr TwTab<R> make_tw() {
   return t;
 }
 
+// The same for FP32, of the entries W^(n2 k1) that a P x Q split multiplies by.
+// Rounded to nearest, sqrt(1/2), cos(pi/8), sin(pi/8) and sin(pi/3) all come out
+// 1.6 to 3.1e-8 too small, and the results of every pass with them.  Here each entry
+// takes, of the floats on both sides of its parts, the pair that keeps the sum of
+// the moduli's errors so far nearest to zero.  FP32BIAS
+struct Near {
+  double v[2];
+};
+constexpr Near ct_floats(double x) {  // the float nearest to x, the one on its other side
+  const float f = (float)x;
+  if ((double)f == x || f == 0.0f) return {{x, x}};
+  double ulp = 1.0 / (1 << 24);
+  for (double a = f < 0 ? -(double)f : (double)f; a < 0.5; a *= 2) ulp *= 0.5;
+  return {{(double)f, (double)f < x ? (double)f + ulp : (double)f - ulp}};
+}
+template <int P, int Q>
+constexpr TwTab<P * Q> make_tw32() {
+  constexpr int R = P * Q;
+  TwTab<R> t = make_tw<R>();
+  double sum = 0.0;
+  for (int m = 1; m < R; ++m) {
+    int uses = 0;
+    for (int n2 = 1; n2 < Q; ++n2)
+      for (int k1 = 1; k1 < P; ++k1) uses += (n2 * k1) % R == m;
+    const double c = t.c[m], s = t.s[m];
+    const Near nc = ct_floats(c), ns = ct_floats(s);
+    double best = 1.0, err = 0.0;
+    for (int i = 0; i < 4; ++i) {
+      const double a = nc.v[i & 1], b = ns.v[i >> 1];
+      const double e = c * (a - c) + s * (b - s), z = sum + uses * e;
+      if ((z < 0 ? -z : z) < best) {
+        best = z < 0 ? -z : z;
+        err = e;
+        t.c[m] = a;
+        t.s[m] = b;
+      }
+    }
+    sum += uses * err;
+  }
+  return t;
+}
+template <typename T, int P, int Q>
+constexpr TwTab<P * Q> make_tw_for() {
+  if constexpr (sizeof(T) == 4)
+    return make_tw32<P, Q>();
+  else
+    return make_tw<P * Q>();
+}
+
 // ---------------------------------------------------------------- radix DFTs
 template <typename T>
 __device__ __forceinline__ cpx<T> cm(cpx<T> a, cpx<T> b) {
@@ -129,14 +178,16 @@ template <typename T, int S>
 struct Dft<T, 3, S> {
   template <bool ONE>
   static __device__ __forceinline__ void run_tw(cpx<T>* v, const cpx<T>* w) {
+    // FP32: 0.866025388 three times and the next float once (see make_tw32)
     const T h = (T)S * (T)0.86602540378443864676;
+    const T h1 = sizeof(T) == 4 ? (T)S * (T)0.866025447845458984 : h;
     cpx<T> t1, d;
     pair_tw<ONE>(v, w, 1, 2, t1, d);
     const cpx<T> a0 = ONE || w == nullptr ? v[0] : cm(v[0], w[0]);
     const cpx<T> t2 = {fm((T)-0.5, t1.x, a0.x), fm((T)-0.5, t1.y, a0.y)};
     v[0] = {a0.x + t1.x, a0.y + t1.y};
     v[1] = {fm(-h, d.y, t2.x), fm(h, d.x, t2.y)};
-    v[2] = {fm(h, d.y, t2.x), fm(-h, d.x, t2.y)};
+    v[2] = {fm(h, d.y, t2.x), fm(-h1, d.x, t2.y)};
   }
   static __device__ __forceinline__ void run(cpx<T>* v) { run_tw<false>(v, nullptr); }
 };
@@ -197,7 +248,7 @@ struct DftPQ {
   template <bool ONE>
   static __device__ __forceinline__ void run_tw(cpx<T>* v, const cpx<T>* w) {
     constexpr int R = P * Q;
-    constexpr TwTab<R> tw = make_tw<R>();
+    constexpr TwTab<R> tw = make_tw_for<T, P, Q>();
     cpx<T> y[Q][P];
 #pragma unroll
     for (int n2 = 0; n2 < Q; ++n2) {
