@@ -108,4 +108,16 @@ int fft2_ntr(int n) {
   }
 }
 
+int fft2_nrows(int n) {  // XRows in oa_fft2_kernels.h
+  switch (n) {
+#define OA_CASE(nn, r1, r2) \
+  case nn:                  \
+    return 4 * (64 / ((r1) > (r2) ? (r1) : (r2)));
+    OA_FFT2_SIZES(OA_CASE)
+#undef OA_CASE
+    default:
+      return 0;
+  }
+}
+
 }  // namespace oa

@@ -5,9 +5,9 @@
 //
 //   k2_zfwd : sphere gather + z-FFT (FFTW_FORWARD)  psi(G) -> zbuf[s][z][kx][ky]
 //   k2_yfwd : y-FFT (FFTW_FORWARD), transposing     zbuf   -> xbuf[s][z][y][kx]
-//   k2_xc2r : pair-row Hermitian x-FFT, rho         xbuf   -> psir, rho partials
-//   k2_xr2c : V psi occ, pair-row x-FFT             psir,V -> xbuf (conjugated)
-//   k2_ybwd : y-FFT (FFTW_BACKWARD)                 xbuf   -> zbuf
+//   k2_xc2r : pair-row Hermitian x-FFT, rho         xbuf   -> rho partials
+//   k2_xr2c : the same again, V psi occ, x-FFT      xbuf,V -> xout (conjugated)
+//   k2_ybwd : y-FFT (FFTW_BACKWARD)                 xout   -> zbuf
 //   k2_zbwd : z-FFT, pack, -2/N, kinetic force, EKE zbuf   -> F(G)
 // Conventions are those of fftCache.C:460-553, 1099-1319 and
 // CP_State_GSpacePlane.C:1582-1778 (see oa_fft.hip for the restatement).
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(kThreads) void k2_ybwd(FftCtx c) {
   {  // pass 1: lanes along kx (contiguous in xbuf)
     const int tr = tid % NTR, j = tid / NTR;
     if (tr < nk && j < R2) {
-      const cpx<T>* src = (const cpx<T>*)c.xbuf + off + kx0 + tr;
+      const cpx<T>* src = (const cpx<T>*)c.xout + off + kx0 + tr;
       cpx<T> v[R1];
 #pragma unroll
       for (int t = 0; t < R1; t++) v[t] = src[(size_t)(j + t * R2) * npx];
@@ -315,74 +315,150 @@ __global__ __launch_bounds__(kThreads) void k2_ybwd(FftCtx c) {
 // ------------------------------------------------------------------ x passes
 // Workgroup = (block of NTR pair-rows, z, chunk of states); loops over the
 // chunk's states.  Lanes run along x in both passes (rows are contiguous).
-
+// Bound by latency and then memory: the next state's coefficients are loaded while
+// this one's are transformed.  96 states of 72 x 80 x 90 in FP32: G->R 150 -> 51 us,
+// R->G 160 -> 83 us (105 and 210 MB), before with barriers for the whole workgroup
+// between passes and psi(r) written and read.
+// A wave transforms TPW pairs of rows by itself: what one lane leaves in LDS another
+// lane of the same wave reads, in program order, so no barrier stands between the
+// passes of a state or between states, and a wave that waits for memory holds up no
+// other.
 template <typename T, int R1, int R2>
+struct XRows {
+  static constexpr int N = R1 * R2, G = R1 > R2 ? R1 : R2;
+  static constexpr int TPW = 64 / G, NTR = kThreads / 64 * TPW;
+  static constexpr int P1 = R1 | 1;     // odd LDS stride of an R1-long run
+  static constexpr int SZ = R2 * P1;    // >= N
+};
+__device__ __forceinline__ void wave_lds() {  // LDS order within a wave, for the compiler
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The two rows' coefficients of this lane (k = j + t R2): off = byte offset of
+// X1[|k|] in the plane's rows or out of range (buffer loads give zero there), sg
+// the sign that makes X1 +- i X2 or its mirror image of them.
+template <typename T, int R1, int R2>
+struct XIn {
+  unsigned off[R1];
+  T sg[R1];
+  bool two;  // the pair has a second row
+  cpx<T> a[R1], b[R1];
+  __device__ __forceinline__ void init(bool active, int y1, int ny, int npx, int j) {
+    constexpr int N = R1 * R2;
+    two = y1 + 1 < ny;
+#pragma unroll
+    for (int t = 0; t < R1; t++) {
+      const int k = j + t * R2, kk = k < npx ? k : N - k;
+      const bool in = active && j < R2 && kk < npx;
+      off[t] = in ? (unsigned)((y1 * npx + kk) * sizeof(cpx<T>)) : 0x7fffffffu;
+      sg[t] = k == 0 ? (T)0 : k < npx ? (T)1 : (T)-1;
+    }
+  }
+  __device__ __forceinline__ cpx<T> ld(__amdgpu_buffer_rsrc_t r, unsigned o, int so) {
+    if constexpr (sizeof(T) == 4) {
+      typedef unsigned u2 __attribute__((ext_vector_type(2)));
+      return __builtin_bit_cast(cpx<T>, (u2)__builtin_amdgcn_raw_buffer_load_b64(r, o, so, 0));
+    } else {
+      typedef unsigned u4 __attribute__((ext_vector_type(4)));
+      return __builtin_bit_cast(cpx<T>, (u4)__builtin_amdgcn_raw_buffer_load_b128(r, o, so, 0));
+    }
+  }
+  // rows: of one state and z, bytes long
+  __device__ __forceinline__ void load(const cpx<T>* rows, int bytes, int npx) {
+    const __amdgpu_buffer_rsrc_t r =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<cpx<T>*>(rows), (short)0, bytes, 0x00020000);
+#pragma unroll
+    for (int t = 0; t < R1; t++) a[t] = ld(r, off[t], 0);
+#pragma unroll
+    for (int t = 0; t < R1; t++)
+      b[t] = ld(r, two ? off[t] + (unsigned)(npx * sizeof(cpx<T>)) : 0x7fffffffu, 0);
+  }
+  __device__ __forceinline__ void pairs(cpx<T> (&v)[R1]) const {
+#pragma unroll
+    for (int t = 0; t < R1; t++)
+      v[t] = {a[t].x - sg[t] * b[t].y, b[t].x + sg[t] * a[t].y};
+  }
+};
+
+// Second half of the x-FFT to real space: u[t] = the two rows at x = j + t R1
+// (of the lanes j < R1), their coefficients' first pass being in v of the lanes
+// j < R2
+template <typename T, int R1, int R2>
+__device__ __forceinline__ void x_to_real(cpx<T> (&v)[R1], cpx<T> (&u)[R2], cpx<T>* ex,
+                                          const cpx<T> (&w)[R2], bool active, int j) {
+  constexpr int P1 = XRows<T, R1, R2>::P1;
+  Dft<T, R1, -1>::run(v);
+  if (active && j < R2) {
+#pragma unroll
+    for (int t = 0; t < R1; t++) ex[j * P1 + t] = v[t];
+  }
+  wave_lds();
+  if (active && j < R1) {
+#pragma unroll
+    for (int t = 0; t < R2; t++) u[t] = ex[j + t * P1];
+  }
+  wave_lds();
+#pragma unroll
+  for (int t = 1; t < R2; t++) u[t] = cm(u[t], w[t]);
+  Dft<T, R2, -1>::run(u);
+}
+
+// PSIR: psi(r) of state c.psir_state into c.psir instead of rho partials
+template <typename T, int R1, int R2, bool PSIR>
 __global__ __launch_bounds__(kThreads) void k2_xc2r(FftCtx c) {
-  using Sh = Shape<R1, R2>;
-  constexpr int N = Sh::N, G = Sh::G, NTR = Sh::NTR;
-  __shared__ cpx<T> ex[NTR * N];
+  using X = XRows<T, R1, R2>;
+  constexpr int N = X::N, G = X::G, TPW = X::TPW;
+  __shared__ cpx<T> smem[X::NTR * X::SZ];
   const int ny = c.g.ny, npx = c.g.nplane_x;
   const int npairs = (ny + 1) / 2;
-  const int q0 = blockIdx.x * NTR, z = blockIdx.y, chunk = blockIdx.z;
-  const int nq = min(NTR, npairs - q0);
-  const int st0 = chunk * c.cs, st1 = min(c.g.nst, st0 + c.cs);
-  const int tid = threadIdx.x;
-  const int tr = tid / G, j = tid - tr * G;
-  const int y1 = 2 * (q0 + tr), y2 = y1 + 1;
-  const size_t NP = (size_t)N * ny, Ntot = NP * c.g.nz;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int tr = lane / G, j = lane - tr * G;
+  const int q = (blockIdx.x * (kThreads / 64) + wave) * TPW + tr;
+  const int z = blockIdx.y, chunk = blockIdx.z;
+  const bool active = tr < TPW && q < npairs;
+  cpx<T>* ex = smem + (wave * TPW + min(tr, TPW - 1)) * X::SZ;
+  const int st0 = PSIR ? c.psir_state : chunk * c.cs;
+  const int st1 = PSIR ? st0 + 1 : min(c.g.nst, st0 + c.cs);
+  const int y1 = 2 * q, y2 = y1 + 1;
+  const size_t NP = (size_t)N * ny, plane = (size_t)ny * npx;
+  const int bytes = (int)(plane * sizeof(cpx<T>));
+  const cpx<T>* xb = (const cpx<T>*)c.xbuf + z * plane;
+  cpx<T> w[R2];
+#pragma unroll
+  for (int t = 1; t < R2; t++) w[t] = twiddle<T, -1>(c.twx, t * min(j, R1 - 1));
   double acc[2 * R2];
 #pragma unroll
   for (int i = 0; i < 2 * R2; i++) acc[i] = 0.0;
+  XIn<T, R1, R2> in;
+  in.init(active, y1, ny, npx, j);
+  if (st0 < st1) in.load(xb + st0 * plane * c.g.nz, bytes, npx);
   for (int s = st0; s < st1; s++) {
-    if (tr < nq && j < R2) {
-      const cpx<T>* xs = (const cpx<T>*)c.xbuf + ((size_t)s * c.g.nz + z) * ny * npx;
-      cpx<T> v[R1];
+    cpx<T> v[R1], u[R2];
+    in.pairs(v);
+    if (s + 1 < st1) in.load(xb + (s + 1) * plane * c.g.nz, bytes, npx);
+    x_to_real<T, R1, R2>(v, u, ex, w, active, j);
+    if constexpr (PSIR) {
+      if (active && j < R1) {
+        T* pr = (T*)c.psir + (size_t)z * NP;
 #pragma unroll
-      for (int t = 0; t < R1; t++) {
-        const int k = j + t * R2;
-        cpx<T> Z = {(T)0, (T)0};
-        int kk = -1;
-        bool mirror = false;
-        if (k < npx) kk = k;
-        else if (k > N - npx) { kk = N - k; mirror = true; }
-        if (kk >= 0) {
-          const cpx<T> X1 = xs[(size_t)y1 * npx + kk];
-          const cpx<T> X2 = (y2 < ny) ? xs[(size_t)y2 * npx + kk] : cpx<T>{(T)0, (T)0};
-          if (kk == 0) Z = {X1.x, X2.x};
-          else if (!mirror) Z = {X1.x - X2.y, X1.y + X2.x};
-          else Z = {X1.x + X2.y, X2.x - X1.y};
+        for (int t = 0; t < R2; t++) {
+          const int x = j + t * R1;
+          pr[(size_t)y1 * N + x] = u[t].x;
+          if (y2 < ny) pr[(size_t)y2 * N + x] = u[t].y;
         }
-        v[t] = Z;
       }
-      Dft<T, R1, -1>::run(v);
-#pragma unroll
-      for (int t = 0; t < R1; t++) ex[tr * N + j * R1 + t] = v[t];
-    }
-    __syncthreads();
-    if (tr < nq && j < R1) {
-      cpx<T> u[R2];
-#pragma unroll
-      for (int t = 0; t < R2; t++) u[t] = ex[tr * N + j + t * R1];
-#pragma unroll
-      for (int t = 1; t < R2; t++) u[t] = cm(u[t], twiddle<T, -1>(c.twx, t * j));
-      Dft<T, R2, -1>::run(u);
+    } else {
       const double oc = c.occ[s];
-      T* pr = (T*)c.psir + (size_t)s * Ntot + (size_t)z * NP;
 #pragma unroll
       for (int t = 0; t < R2; t++) {
-        const int x = j + t * R1;
-        pr[(size_t)y1 * N + x] = u[t].x;
         acc[2 * t] += oc * (double)u[t].x * (double)u[t].x;
-        if (y2 < ny) {
-          pr[(size_t)y2 * N + x] = u[t].y;
-          acc[2 * t + 1] += oc * (double)u[t].y * (double)u[t].y;
-        }
+        acc[2 * t + 1] += oc * (double)u[t].y * (double)u[t].y;
       }
     }
-    __syncthreads();
   }
-  if (tr < nq && j < R1) {
-    double* rp = c.rho_part + (size_t)chunk * Ntot + (size_t)z * NP;
+  if (!PSIR && active && j < R1) {
+    double* rp = c.rho_part + (size_t)chunk * NP * c.g.nz + (size_t)z * NP;
 #pragma unroll
     for (int t = 0; t < R2; t++) {
       const int x = j + t * R1;
@@ -392,82 +468,90 @@ __global__ __launch_bounds__(kThreads) void k2_xc2r(FftCtx c) {
   }
 }
 
+// psi(r) again from xbuf, V psi, and the x-FFT back of both rows to c.xout, which
+// leaves xbuf to oa_psir_get: reading nplane_x coefficients a row twice moves half
+// the bytes of writing psi(r) and reading it.  The lanes hold x = j + t R1, so the
+// way back takes the factors in the other order.
 template <typename T, int R1, int R2>
 __global__ __launch_bounds__(kThreads) void k2_xr2c(FftCtx c) {
-  using Sh = Shape<R1, R2>;
-  constexpr int N = Sh::N, G = Sh::G, NTR = Sh::NTR;
-  __shared__ cpx<T> ex[NTR * N];
+  using X = XRows<T, R1, R2>;
+  constexpr int N = X::N, G = X::G, TPW = X::TPW, P1 = X::P1;
+  __shared__ cpx<T> smem[X::NTR * X::SZ];
   const int ny = c.g.ny, npx = c.g.nplane_x;
   const int npairs = (ny + 1) / 2;
-  const int q0 = blockIdx.x * NTR, z = blockIdx.y, chunk = blockIdx.z;
-  const int nq = min(NTR, npairs - q0);
-  const int st0 = chunk * c.cs, st1 = min(c.g.nst, st0 + c.cs);
-  const int tid = threadIdx.x;
-  const int tr = tid / G, j = tid - tr * G;
-  const int y1 = 2 * (q0 + tr), y2 = y1 + 1;
-  const size_t NP = (size_t)N * ny, Ntot = NP * c.g.nz;
-  // V at this thread's pass-1 positions, both rows
-  T v1[R1], v2[R1];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int tr = lane / G, j = lane - tr * G;
+  const int q = (blockIdx.x * (kThreads / 64) + wave) * TPW + tr;
+  const int z = blockIdx.y, chunk = blockIdx.z;
+  const bool active = tr < TPW && q < npairs;
+  cpx<T>* ex = smem + (wave * TPW + min(tr, TPW - 1)) * X::SZ;
+  const int st0 = chunk * c.cs_r, st1 = min(c.g.nst, st0 + c.cs_r);
+  const int y1 = 2 * q, y2 = y1 + 1;
+  const size_t NP = (size_t)N * ny, plane = (size_t)ny * npx;
+  const int bytes = (int)(plane * sizeof(cpx<T>));
+  const cpx<T>* xb = (const cpx<T>*)c.xbuf + z * plane;
+  cpx<T>* xo = (cpx<T>*)c.xout + z * plane;
+  cpx<T> w[R2];
 #pragma unroll
-  for (int t = 0; t < R1; t++) {
-    v1[t] = (T)0;
-    v2[t] = (T)0;
-    if (tr < nq && j < R2) {
-      const double* vz = c.vks + (size_t)z * NP;
-      const int x = j + t * R2;
-      v1[t] = (T)vz[(size_t)y1 * N + x];
-      if (y2 < ny) v2[t] = (T)vz[(size_t)y2 * N + x];
-    }
+  for (int t = 1; t < R2; t++) w[t] = twiddle<T, -1>(c.twx, t * min(j, R1 - 1));
+  T v1[R2], v2[R2];  // V at x = j + t R1 of both rows
+#pragma unroll
+  for (int t = 0; t < R2; t++) {
+    const double* vz = c.vks + (size_t)z * NP;
+    const int x = j + t * R1;
+    v1[t] = active && j < R1 ? (T)vz[(size_t)y1 * N + x] : (T)0;
+    v2[t] = active && j < R1 && y2 < ny ? (T)vz[(size_t)y2 * N + x] : (T)0;
   }
+  XIn<T, R1, R2> in;
+  in.init(active, y1, ny, npx, j);
+  if (st0 < st1) in.load(xb + st0 * plane * c.g.nz, bytes, npx);
   for (int s = st0; s < st1; s++) {
-    if (tr < nq && j < R2) {
-      const T oc = (T)c.occ[s];
-      const T* pr = (const T*)c.psir + (size_t)s * Ntot + (size_t)z * NP;
-      cpx<T> v[R1];
+    cpx<T> v[R1], u[R2];
+    in.pairs(v);
+    if (s + 1 < st1) in.load(xb + (s + 1) * plane * c.g.nz, bytes, npx);
+    x_to_real<T, R1, R2>(v, u, ex, w, active, j);
+    const T oc = (T)c.occ[s];
 #pragma unroll
-      for (int t = 0; t < R1; t++) {
-        const int x = j + t * R2;
-        const T f1 = pr[(size_t)y1 * N + x] * (v1[t] * oc);
-        const T f2 = (y2 < ny) ? pr[(size_t)y2 * N + x] * (v2[t] * oc) : (T)0;
-        v[t] = {f1, f2};
-      }
-      Dft<T, R1, -1>::run(v);
+    for (int t = 0; t < R2; t++) u[t] = {u[t].x * (v1[t] * oc), u[t].y * (v2[t] * oc)};
+    Dft<T, R2, -1>::run(u);
 #pragma unroll
-      for (int t = 0; t < R1; t++) ex[tr * N + j * R1 + t] = v[t];
+    for (int t = 1; t < R2; t++) u[t] = cm(u[t], w[t]);
+    if (active && j < R1) {
+#pragma unroll
+      for (int t = 0; t < R2; t++) ex[t * P1 + j] = u[t];
     }
-    __syncthreads();
-    if (tr < nq && j < R1) {
-      cpx<T> u[R2];
+    wave_lds();
+    if (active && j < R2) {
 #pragma unroll
-      for (int t = 0; t < R2; t++) u[t] = ex[tr * N + j + t * R1];
-#pragma unroll
-      for (int t = 1; t < R2; t++) u[t] = cm(u[t], twiddle<T, -1>(c.twx, t * j));
-      Dft<T, R2, -1>::run(u);
-#pragma unroll
-      for (int t = 0; t < R2; t++) ex[tr * N + j + t * R1] = u[t];
+      for (int t = 0; t < R1; t++) v[t] = ex[j * P1 + t];
     }
-    __syncthreads();
+    wave_lds();
+    Dft<T, R1, -1>::run(v);
+    if (active && j < R2) {
+#pragma unroll
+      for (int t = 0; t < R1; t++) ex[j + t * R2] = v[t];
+    }
+    wave_lds();
     // split the two real rows and keep kx < nplane_x, conjugated
-    cpx<T>* xs = (cpx<T>*)c.xbuf + ((size_t)s * c.g.nz + z) * ny * npx;
-    for (int idx = tid; idx < nq * npx; idx += kThreads) {
-      const int q = idx / npx, k = idx - q * npx;
-      const int r1 = 2 * (q0 + q), r2 = r1 + 1;
-      const cpx<T> Zk = ex[q * N + k];
-      const cpx<T> Zm = ex[q * N + (k == 0 ? 0 : N - k)];
-      xs[(size_t)r1 * npx + k] = {(T)0.5 * (Zk.x + Zm.x), -(T)0.5 * (Zk.y - Zm.y)};
-      if (r2 < ny) xs[(size_t)r2 * npx + k] = {(T)0.5 * (Zk.y + Zm.y), (T)0.5 * (Zk.x - Zm.x)};
+    cpx<T>* xs = xo + s * plane * c.g.nz + (size_t)y1 * npx;
+    if (active) {
+      for (int k = j; k < npx; k += G) {
+        const cpx<T> Zk = ex[k], Zm = ex[k == 0 ? 0 : N - k];
+        xs[k] = {(T)0.5 * (Zk.x + Zm.x), -(T)0.5 * (Zk.y - Zm.y)};
+        if (y2 < ny) xs[npx + k] = {(T)0.5 * (Zk.y + Zm.y), (T)0.5 * (Zk.x - Zm.x)};
+      }
     }
-    __syncthreads();
+    wave_lds();
   }
 }
 
 // ------------------------------------------------------------------ launch
 
-enum Kind { ZFWD = 0, YFWD, XC2R, XR2C, YBWD, ZBWD };
+enum Kind { ZFWD = 0, YFWD, XC2R, XR2C, YBWD, ZBWD, XPSIR };
 
 template <typename T, int R1, int R2>
 hipError_t launch(int kind, const FftCtx& c, hipStream_t st) {
-  constexpr int NTR = Shape<R1, R2>::NTR;
+  constexpr int NTR = Shape<R1, R2>::NTR, NX = XRows<T, R1, R2>::NTR;
   const Geom& g = c.g;
   switch (kind) {
     case ZFWD:
@@ -495,14 +579,18 @@ hipError_t launch(int kind, const FftCtx& c, hipStream_t st) {
                          dim3(kThreads), 0, st, c);
       break;
     case XC2R:
-      hipLaunchKernelGGL((k2_xc2r<T, R1, R2>),
-                         dim3(((g.ny + 1) / 2 + NTR - 1) / NTR, g.nz, c.nchunk), dim3(kThreads),
+      hipLaunchKernelGGL((k2_xc2r<T, R1, R2, false>),
+                         dim3(((g.ny + 1) / 2 + NX - 1) / NX, g.nz, c.nchunk), dim3(kThreads),
                          0, st, c);
       break;
     case XR2C:
       hipLaunchKernelGGL((k2_xr2c<T, R1, R2>),
-                         dim3(((g.ny + 1) / 2 + NTR - 1) / NTR, g.nz, c.nchunk), dim3(kThreads),
+                         dim3(((g.ny + 1) / 2 + NX - 1) / NX, g.nz, c.nchunk_r), dim3(kThreads),
                          0, st, c);
+      break;
+    case XPSIR:
+      hipLaunchKernelGGL((k2_xc2r<T, R1, R2, true>),
+                         dim3(((g.ny + 1) / 2 + NX - 1) / NX, g.nz), dim3(kThreads), 0, st, c);
       break;
     default:
       return hipErrorInvalidValue;

@@ -51,6 +51,7 @@ struct FftCtx {
   const double* vks;      // [N] V(r)
   void* zbuf;             // [nst][nz][nplane_x][ny] complex T
   void* xbuf;             // [nst][nz][ny][nplane_x] complex T
+  void* xout;             // the same, of the two-factor passes back
   void* psir;             // [nst][nz][ny][nx] T
   double* rho;            // [N]
   double* eke_part;       // [nst][nblk]
@@ -66,9 +67,9 @@ struct FftCtx {
   const int4* lines;      // [nlines] (first point, length, first kz, kx*ny + ky mod ny)
   // fused two-factor plane passes
   void* zout;             // [nst][nz][nplane_x][ny] complex T: R->G plane output
-  int nchunk_r;           // state chunks of the R->G plane pass ...
+  int nchunk_r;           // state chunks of the R->G plane or x pass ...
   int cs_r;               // ... and states per chunk
-  int psir_state;         // state whose psi(r) the G->R plane pass writes to psir
+  int psir_state;         // state whose psi(r) a G->R pass writes to psir
   int prune;              // plane passes pruned to |kx|, |ky| <= (N - 1) / 4
   int prune_z;            // z passes pruned to |kz| <= (nz - 1) / 4
   // plane engine: psi(r) written by the G->R pass and read back by the R->G
@@ -79,10 +80,12 @@ struct FftCtx {
 };
 
 // two-factor register FFT engine (oa_fft2_*.hip): kind 0 z fwd, 1 y fwd,
-// 2 x c2r + rho partials, 3 V psi + x r2c, 4 y bwd, 5 z bwd + kinetic/EKE;
+// 2 x c2r + rho partials, 3 V psi + x r2c, 4 y bwd, 5 z bwd + kinetic/EKE,
+// 6 x c2r writing psi(r) of c.psir_state;
 // n is the length of the kind's axis
 hipError_t fft2_launch(int kind, int n, bool fp32, const FftCtx& c, hipStream_t st);
 int fft2_ntr(int n);  // transforms per workgroup for length n, 0 if not compiled
+int fft2_nrows(int n);  // row pairs per workgroup of kinds 2, 3 and 6
 
 // fused y+x plane passes on the two-factor engine, square planes nx == ny == n
 // (oa_plane4.h by row class where c.prune is set and the length has classes,
@@ -115,7 +118,7 @@ int plane_threads(int cfg);
 
 // stage: 0 z-gather+FFT, 1 y-FFT fwd, 2 x c2r + rho, 3 V psi + x r2c,
 //        4 y-FFT bwd, 5 z-FFT + pack + kinetic force / EKE partials
-enum { FFT_ZFWD = 0, FFT_YFWD, FFT_XC2R, FFT_XR2C, FFT_YBWD, FFT_ZBWD, FFT_NSTAGE };
+enum { FFT_ZFWD = 0, FFT_YFWD, FFT_XC2R, FFT_XR2C, FFT_YBWD, FFT_ZBWD, FFT_XPSIR };
 hipError_t fft_stage(const FftCtx& c, bool fp32, int stage, hipStream_t st);
 size_t fft_max_smem(const FftCtx& c, bool fp32);
 

@@ -157,7 +157,7 @@ struct oa_ctx {
       *sd_twin = nullptr;  // per point: -1, -2 (redundant kx=0 point) or its redundant twin
   double2 *twx = nullptr, *twy = nullptr, *twz = nullptr;
   double *g2 = nullptr, *occ = nullptr, *dtm = nullptr, *vks = nullptr, *rho = nullptr;
-  void *zbuf = nullptr, *xbuf = nullptr, *psir = nullptr, *zout = nullptr;
+  void *zbuf = nullptr, *xbuf = nullptr, *xout = nullptr, *psir = nullptr, *zout = nullptr;
   oa::VPerm vperm{};    // plane engine with row classes: V(r) for the R->G pass
   void* psk = nullptr;  // plane engine, opt.psir_keep: psi(r) between the plane passes
   double* eke_part = nullptr;
@@ -472,10 +472,14 @@ oa_status build_layout(oa_ctx* c) {
   f.plane_cfg = oa::plane_config_for(c->nx * c->ny);
   if (c->engine == kEngFused && f.plane_cfg < 0) c->engine = kEngSep;
   if (c->engine == kEngFft2) {
-    const int qblk = (npairs_all + oa::fft2_ntr(c->nx) - 1) / oa::fft2_ntr(c->nx);
-    const int nchunk = std::max(1, std::min(c->nst, (1024 + qblk * c->nz - 1) / (qblk * c->nz)));
-    f.cs = (c->nst + nchunk - 1) / nchunk;
-    f.nchunk = (c->nst + f.cs - 1) / f.cs;
+    const int per = ((npairs_all + oa::fft2_nrows(c->nx) - 1) / oa::fft2_nrows(c->nx)) * c->nz;
+    auto chunks = [&](int target, int& cs, int& n) {  // about `target` workgroups
+      n = std::max(1, std::min(c->nst, (target + per - 1) / per));
+      cs = (c->nst + n - 1) / n;
+      n = (c->nst + cs - 1) / cs;
+    };
+    chunks(1024, f.cs, f.nchunk);  // each chunk writes a rho partial
+    chunks(2048, f.cs_r, f.nchunk_r);
     c->nzblk = (c->nlines + oa::fft2_ntr(c->nz) - 1) / oa::fft2_ntr(c->nz);
   }
   if (c->engine == kEngPlane) {
@@ -698,7 +702,12 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
   } else {
     if (c->engine != kEngFused)
       TRY(dalloc(c, &c->xbuf, (size_t)c->nst * c->nz * c->ny * c->nplane_x * csz));
-    TRY(dalloc(c, &c->psir, (size_t)c->nst * N * rsz));
+    if (c->engine == kEngFft2) {  // one state's psi(r), for oa_psir_get
+      TRY(dalloc(c, &c->xout, (size_t)c->nst * c->nz * c->ny * c->nplane_x * csz));
+      TRY(dalloc(c, &c->psir, N * rsz));
+    } else {
+      TRY(dalloc(c, &c->psir, (size_t)c->nst * N * rsz));
+    }
   }
   TRY(dalloc(c, &c->rho, N * sizeof(double)));
   TRY(dalloc(c, &c->vks, N * sizeof(double)));
@@ -824,6 +833,7 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
   f.zbuf = c->zbuf;
   f.zout = c->zout;
   f.xbuf = c->xbuf;
+  f.xout = c->xout;
   f.psir = c->psir;
   f.psk = c->psk;
   f.vperm = c->vperm.p;
@@ -1601,7 +1611,7 @@ oa_status oa_get_config(const oa_ctx* c, int cfg[8]) {
   cfg[0] = c->fuse_rho ? 4 : c->engine;
   cfg[1] = fft2 ? oa::fft2_ntr(c->nz) : f.lpb;
   cfg[2] = fft2 ? oa::fft2_ntr(c->ny) : f.kc;
-  cfg[3] = fft2 ? oa::fft2_ntr(c->nx) : f.npair;
+  cfg[3] = plane ? oa::fft2_ntr(c->nx) : fft2 ? oa::fft2_nrows(c->nx) : f.npair;
   cfg[4] = fused ? f.kcp : plane ? f.cs_r : 0;
   cfg[5] = fused ? f.pcp : plane ? f.nchunk_r : 0;
   cfg[6] = (fused || fft2) ? f.cs : 0;
@@ -1979,11 +1989,14 @@ oa_status oa_psir_get(oa_ctx* c, int s, double* out) {
   HIPCHK(hipSetDevice(c->device));
   const size_t N = (size_t)c->nx * c->ny * c->nz;
   size_t off = (size_t)s * N;
-  if (c->engine == kEngPlane) {
-    // psi(r) is not kept: recompute state s from the z-pass output
+  if (c->engine == kEngPlane || c->engine == kEngFft2) {
+    // psi(r) is not kept: recompute state s from the z- or y-pass output
     FftCtx f = fctx(c);
     f.psir_state = s;
-    HIPCHK(oa::plane3_launch(2, c->nx, c->fp32, f, c->stream));
+    if (c->engine == kEngPlane)
+      HIPCHK(oa::plane3_launch(2, c->nx, c->fp32, f, c->stream));
+    else
+      HIPCHK(oa::fft2_launch(oa::FFT_XPSIR, c->nx, c->fp32, f, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     off = 0;
   }
