@@ -4,7 +4,8 @@
 
 namespace oa2 {
 #define OA_DECL(n, r1, r2) \
-  hipError_t launch_n##n(int kind, bool fp32, const oa::FftCtx& c, hipStream_t st);
+  hipError_t launch_n##n(int kind, bool fp32, const oa::FftCtx& c, hipStream_t st); \
+  hipError_t vks_n##n(int kind, const oa::VksArgs& a, hipStream_t st);
 OA_FFT2_SIZES(OA_DECL)
 #undef OA_DECL
 }  // namespace oa2
@@ -28,6 +29,18 @@ hipError_t fft2_launch(int kind, int n, bool fp32, const FftCtx& c, hipStream_t 
 #define OA_CASE(nn, r1, r2) \
   case nn:                  \
     return oa2::launch_n##nn(kind, fp32, c, st);
+    OA_FFT2_SIZES(OA_CASE)
+#undef OA_CASE
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+hipError_t vks2_launch(int kind, int n, const VksArgs& a, hipStream_t st) {
+  switch (n) {
+#define OA_CASE(nn, r1, r2) \
+  case nn:                  \
+    return oa2::vks_n##nn(kind, a, st);
     OA_FFT2_SIZES(OA_CASE)
 #undef OA_CASE
     default:
@@ -108,11 +121,13 @@ int fft2_ntr(int n) {
   }
 }
 
-int fft2_nrows(int n) {  // XRows in oa_fft2_kernels.h
+int fft2_nrows(int n) { return n > 0 && fft2_group(n) > 0 ? 4 * (64 / fft2_group(n)) : 0; }
+
+int fft2_group(int n) {
   switch (n) {
 #define OA_CASE(nn, r1, r2) \
   case nn:                  \
-    return 4 * (64 / ((r1) > (r2) ? (r1) : (r2)));
+    return (r1) > (r2) ? (r1) : (r2);
     OA_FFT2_SIZES(OA_CASE)
 #undef OA_CASE
     default:

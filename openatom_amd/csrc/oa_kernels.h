@@ -25,6 +25,26 @@ struct VPerm {
     else ((double*)p)[e] = v;
   }
 };
+// the same for points of one row
+struct VPermRow {
+  void* p;
+  size_t base;  // of element (x / x1 = 0, x % x1 = 0)
+  int st, sj, x1, inv, f32;
+  __device__ __forceinline__ VPermRow(const VPerm& v, int z, int y)
+      : p(v.p), x1(v.x1), inv(65536 / v.x1 + 1), f32(v.f32) {
+    const int h = 2 * y >= v.n ? 1 : 0, r = y - h * (v.n >> 1);
+    const int q = r / v.m, cl = r - q * v.m, nq = v.n / (2 * v.m);
+    sj = 2 * nq;
+    st = sj * x1;
+    base = (size_t)(z * v.m + cl) * (v.n / x1) * st + 2 * q + h;
+  }
+  __device__ __forceinline__ void put(int x, double v) const {
+    const int t = (x * inv) >> 16, j = x - t * x1;  // x / x1: x < 160, x1 <= 16
+    const size_t e = base + t * st + j * sj;
+    if (f32) ((float*)p)[e] = (float)v;
+    else ((double*)p)[e] = v;
+  }
+};
 // vp <- v ([nz][n][n])
 hipError_t vperm_set(const VPerm& vp, const double* v, int nz, hipStream_t st);
 // zero the rows y = ny/2 of every plane column of zbuf (pruned planes read them
@@ -85,6 +105,7 @@ struct FftCtx {
 // n is the length of the kind's axis
 hipError_t fft2_launch(int kind, int n, bool fp32, const FftCtx& c, hipStream_t st);
 int fft2_ntr(int n);  // transforms per workgroup for length n, 0 if not compiled
+int fft2_group(int n);  // threads of one transform
 int fft2_nrows(int n);  // row pairs per workgroup of kinds 2, 3 and 6
 
 // fused y+x plane passes on the two-factor engine, square planes nx == ny == n
@@ -165,16 +186,25 @@ struct VksArgs {
   const double2 *twx, *twy, *twz;  // exp(-2 pi i j / n)
   double hmati[9];
   double vol, ecut4;       // Omega; density cutoff 4 ecut_ry on |G|^2
-  const double* rho;       // [nz][ny][nx]
+  double* rho;             // [nz][ny][nx]
   double* v;               // [nz][ny][nx] out: V_KS
   VPerm vp;                // ... and in the R->G pass's order (vp.p may be null)
-  double2* hx;             // [nz][nkx][ny] after the x pass
-  double2* hl;             // [nz][nkx][nky] after the y pass
-  const double2* vloc;     // [nkx][nky][nz] V_loc(G), zero off the sphere
+  double2* hx;             // [nz][nkx][ny] after the x pass (two_factor: [nz][ny][nkx])
+  double2* hl;             // [nz][nkx][nky] after the y pass ([nz][nky][nkx])
+  const double2* vloc;     // [nkx][nky][nz] V_loc(G), zero off the sphere ([nz][nky][nkx])
   double* part_x;          // [nbx][3] exchange-correlation partial sums
   double* part_l;          // [nbl][2] Hartree and E_ext partial sums
+  int two_factor;          // oa_vks2.h: all three lengths compiled
+  // two_factor: rho as nparts > 0 partials (times inv_vol), also written to rho
+  const double* rho_part;
+  int nparts;
+  double inv_vol;
+  int nbx, nbl;            // set by vks_build
+  StepDev* res;
 };
 // workgroup counts of the x and line passes
+// one two-factor pass, n the length of its axis
+hipError_t vks2_launch(int kind, int n, const VksArgs& a, hipStream_t st);
 int vks_nbx(const VksArgs& a);
 int vks_nbl(const VksArgs& a);
 size_t vks_smem(const VksArgs& a);  // largest dynamic LDS of the passes

@@ -210,7 +210,7 @@ struct oa_ctx {
   // autotuner (opt.autotune): candidate launch shapes (buffers are sized for
   // the largest) and what was measured
   std::vector<int> tune_nchunk, tune_nchunk_r, tune_nslice_sym, tune_nslice_full;
-  std::vector<int> tune_vks;  // V_KS rows / columns / lines per workgroup
+  std::vector<int> tune_vks[3];  // V_KS rows, columns, lines per workgroup
   std::string tune_log;
   // non-local KB pseudopotential (oa_nonlocal_set): projector table, the
   // projections Z, their scaled transpose and the gram partials
@@ -631,22 +631,36 @@ oa_status alloc_vks(oa_ctx* c) {
   std::memcpy(a.hmati, c->hmati, sizeof(a.hmati));
   a.vol = c->vol;
   a.ecut4 = ecut4;
-  if (oa::vks_smem(a) > 64 * 1024)
+  a.two_factor = oa::fft2_ntr(c->nx) > 0 && oa::fft2_ntr(c->ny) > 0 && oa::fft2_ntr(c->nz) > 0;
+  if (!a.two_factor && oa::vks_smem(a) > 64 * 1024)
     return fail(c, OA_EINVAL, "V_KS pass needs more than 64 KiB of LDS");
   // autotune: row pairs (x passes), columns (y passes) and z lines per
-  // workgroup among 2, 4, 8, 16 where the LDS fits; the partial-sum arrays
-  // are sized for the most workgroups
-  int vmin = a.pr;
-  if (c->opt.autotune) {
+  // workgroup, among 2, 4, 8, 16 where the LDS fits in the Stockham passes; the
+  // partial-sum arrays are sized for the most workgroups
+  oa::VksArgs amin = a;
+  if (a.two_factor) {  // what one, two or four waves take
+    auto per = [](int v) { return std::vector<int>{v, 2 * v, 4 * v}; };
+    auto cols = [](int n) {
+      const int ntr = oa::fft2_ntr(n), g = oa::fft2_group(n);
+      return std::vector<int>{64 / g, 128 / g, ntr};
+    };
+    c->tune_vks[0] = per(64 / oa::fft2_group(c->nx));
+    c->tune_vks[1] = cols(c->ny);
+    c->tune_vks[2] = cols(c->nz);
+    amin.pr = c->tune_vks[0][0];
+    amin.lb = c->tune_vks[2][0];
+    a.pr = c->tune_vks[0][1];
+    a.cb = c->tune_vks[1][1];
+    a.lb = c->tune_vks[2][1];
+  } else if (c->opt.autotune) {
     for (int v : {2, 4, 8, 16}) {
       oa::VksArgs t = a;
       t.pr = t.cb = t.lb = v;
-      if (oa::vks_smem(t) <= 64 * 1024) c->tune_vks.push_back(v);
+      if (oa::vks_smem(t) <= 64 * 1024) c->tune_vks[0].push_back(v);
     }
-    vmin = c->tune_vks.front();
+    c->tune_vks[1] = c->tune_vks[2] = c->tune_vks[0];
+    amin.pr = amin.cb = amin.lb = c->tune_vks[0].front();
   }
-  oa::VksArgs amin = a;
-  amin.pr = amin.cb = amin.lb = vmin;
   const size_t nbox = (size_t)a.nkx * a.nky * c->nz;
   TRY(dalloc(c, &a.hx, (size_t)c->nz * a.nkx * c->ny * sizeof(double2)));
   TRY(dalloc(c, &a.hl, nbox * sizeof(double2)));
@@ -902,8 +916,17 @@ void mark(oa_ctx* c, int i) {
 
 // ---- stages (enqueue only) ----
 // V_KS[rho] into vks, and E_H, E_xc, E_ext into the step results
-oa_status st_vks(oa_ctx* c) {
+// from_parts: rho is still the partial sums of the G->R pass, which the first pass
+// adds up (where it can: else they are added up here)
+oa_status st_vks(oa_ctx* c, bool from_parts = false) {
   oa::VksArgs a = c->va;
+  if (from_parts && a.two_factor) {
+    a.rho_part = c->fc.rho_part;
+    a.nparts = c->fc.nchunk;
+    a.inv_vol = c->fc.inv_vol;
+  } else if (from_parts) {
+    HIPCHK(oa::rho_reduce(fctx(c), c->dpart, c->ndpart, c->stream, false));
+  }
   a.rho = c->rho;
   a.v = c->vks;
   a.vp = c->vperm;
@@ -924,8 +947,10 @@ oa_status st_g2r(oa_ctx* c, int ev0 = -1) {
     mk(0);
     HIPCHK(oa::plane3_launch(0, c->nx, c->fp32, fctx(c), c->stream));
     mk(1);
-    HIPCHK(oa::rho_reduce(fctx(c), c->dpart, c->ndpart, c->stream, !c->opt.vks_from_rho));
-    if (c->opt.vks_from_rho) TRY(st_vks(c));
+    if (c->opt.vks_from_rho)
+      TRY(st_vks(c, true));
+    else
+      HIPCHK(oa::rho_reduce(fctx(c), c->dpart, c->ndpart, c->stream));
     mk(2);
   } else if (c->engine == kEngFft2) {
     HIPCHK(oa::fft2_launch(oa::FFT_ZFWD, c->nz, c->fp32, fctx(c), c->stream));
@@ -933,16 +958,20 @@ oa_status st_g2r(oa_ctx* c, int ev0 = -1) {
     HIPCHK(oa::fft2_launch(oa::FFT_YFWD, c->ny, c->fp32, fctx(c), c->stream));
     mk(1);
     HIPCHK(oa::fft2_launch(oa::FFT_XC2R, c->nx, c->fp32, fctx(c), c->stream));
-    HIPCHK(oa::rho_reduce(fctx(c), c->dpart, c->ndpart, c->stream, !c->opt.vks_from_rho));
-    if (c->opt.vks_from_rho) TRY(st_vks(c));
+    if (c->opt.vks_from_rho)
+      TRY(st_vks(c, true));
+    else
+      HIPCHK(oa::rho_reduce(fctx(c), c->dpart, c->ndpart, c->stream));
     mk(2);
   } else if (c->engine == kEngFused) {
     HIPCHK(oa::fft_stage(fctx(c), c->fp32, oa::FFT_ZFWD, c->stream));
     mk(0);
     HIPCHK(oa::plane_fwd(fctx(c), c->fp32, c->stream));
     mk(1);
-    HIPCHK(oa::rho_reduce(fctx(c), c->dpart, c->ndpart, c->stream, !c->opt.vks_from_rho));
-    if (c->opt.vks_from_rho) TRY(st_vks(c));
+    if (c->opt.vks_from_rho)
+      TRY(st_vks(c, true));
+    else
+      HIPCHK(oa::rho_reduce(fctx(c), c->dpart, c->ndpart, c->stream));
     mk(2);
   } else {
     for (int s = oa::FFT_ZFWD; s <= oa::FFT_XC2R; s++) {
@@ -1369,18 +1398,18 @@ oa_status autotune(oa_ctx* c) {
         return st_gram(c, c->psi, c->psi, true, 1.0 / std::sqrt(2.0), 1.0, c->S,
                        split_on(c, kSplitS));
       });
-  if (c->opt.vks_from_rho && c->tune_vks.size() > 1) {
+  if (c->opt.vks_from_rho && c->tune_vks[0].size() > 1) {
     // V_KS from the rho of the trial passes above; the energy partials are
     // summed in workgroup order, so the choice moves E_H and E_xc by rounding
     oa::VksArgs& va = c->va;
     tune_knob(
-        c, e0, e1, "V_KS row pairs per x-pass workgroup", c->tune_vks, va.pr,
+        c, e0, e1, "V_KS row pairs per x-pass workgroup", c->tune_vks[0], va.pr,
         [&](int v) { va.pr = v; }, [&]() { return st_vks(c); });
     tune_knob(
-        c, e0, e1, "V_KS columns per y-pass workgroup", c->tune_vks, va.cb,
+        c, e0, e1, "V_KS columns per y-pass workgroup", c->tune_vks[1], va.cb,
         [&](int v) { va.cb = v; }, [&]() { return st_vks(c); });
     tune_knob(
-        c, e0, e1, "V_KS z lines per workgroup", c->tune_vks, va.lb,
+        c, e0, e1, "V_KS z lines per workgroup", c->tune_vks[2], va.lb,
         [&](int v) { va.lb = v; }, [&]() { return st_vks(c); });
   }
   tune_knob(

@@ -14,14 +14,15 @@
 //                 in the lane order of the row-class R->G pass (VPerm)
 //   k_vks_sum   : fixed-order reduction of the partial sums into StepDev
 //
-// One grid per step (not one per state), so the passes are plain batched
-// Stockham transforms on LDS: each moves ~2 x 8 MB at 100^3, well under 5% of
-// the state chain.  All arithmetic is FP64 in both precision modes.
+// These passes are plain batched Stockham transforms on LDS, for grids with a length
+// the two-factor engine is not compiled for; the others run oa_vks2.h.  All
+// arithmetic is FP64 in both precision modes.
 #include <algorithm>
 
 #include "oa_common.h"
 #include "oa_kernels.h"
 #include "oa_stockham.h"
+#include "oa_vks_point.h"
 
 namespace oa {
 namespace {
@@ -33,61 +34,54 @@ constexpr int kVW = kVT / 64;
 // a divergent branch is waited for on its own.
 constexpr int KU = 4;
 
-__device__ __forceinline__ int sfreq(int i, int n) { return i <= (n - 1) / 2 ? i : i - n; }
-
-__device__ __forceinline__ double gsq(const double* hi, int a, int b, int c) {
-  const double tpi = 6.283185307179586476925;
-  const double xk = (a * hi[0] + b * hi[1] + c * hi[2]) * tpi;
-  const double yk = (a * hi[3] + b * hi[4] + c * hi[5]) * tpi;
-  const double zk = (a * hi[6] + b * hi[7] + c * hi[8]) * tpi;
-  return xk * xk + yk * yk + zk * zk;
-}
-
-// Perdew-Zunger 1981 LDA per point: exchange factor xf, correlation energy
-// factor cf and potential factor mf (cp_pz_lda.C:48-54, 114-138).  One cube
-// root serves both powers: rs = (3/(4 pi))^(1/3) / rho^(1/3) and
-// xf = -(3/pi)^(1/3) rho^(1/3).
-__device__ __forceinline__ void pz_lda(double r, double& xf, double& cf, double& mf) {
-  const double gamma = -0.14230, beta1 = 1.05290, beta2 = 0.33340;
-  const double au = 0.03110, bu = -0.0480, cu = 0.00200, du = -0.01160;
-  const double power = 1.0 / 3.0;
-  const double rat1 = (7.0 / 6.0) * beta1, rat2 = (4.0 / 3.0) * beta2;
-  const double c_rs = 0.62035049089940001667;  // (3/(4 pi))^(1/3)
-  const double c_x = 0.98474502184269654118;   // (3/pi)^(1/3)
-  const double cr = cbrt(r);
-  const double rs = c_rs / cr;
-  const double sq = sqrt(rs);
-  xf = -c_x * cr;
-  if (rs >= 1.0) {
-    const double c1 = 1.0 + beta1 * sq + beta2 * rs;
-    const double c2 = 1.0 + rat1 * sq + rat2 * rs;
-    cf = gamma / c1;
-    mf = cf * (c2 / c1);
-  } else {
-    const double l = log(rs);
-    cf = au * l + bu + cu * rs * l + du * rs;
-    mf = au * l + (bu - power * au) + 2.0 * power * cu * rs * l + power * (2.0 * du - cu) * rs;
-  }
-}
-
-// sum of NV values over the workgroup (fixed order); result valid on thread 0
-template <int NV>
-__device__ __forceinline__ void block_sum(double (&v)[NV], double* sh) {
+// rho from the partials of the G->R pass (or as it is), V_xc and the energy sums,
+// for the two-factor passes.  Bound by the 200 or so FP64 instructions of a point and
+// by the partials: the lanes of an x pass, of which there are too few to hide either,
+// took 10 us longer at 100^3.
+__global__ __launch_bounds__(kVT) void k_rho_xc(VksArgs a) {
+  __shared__ double red[kVW * 3];
+  const size_t n = (size_t)a.nx * a.ny * a.nz, stride = (size_t)gridDim.x * kVT;
+  double acc[3] = {0.0, 0.0, 0.0};
+  for (size_t i0 = (size_t)blockIdx.x * kVT + threadIdx.x; i0 < n; i0 += 2 * stride) {
+    const size_t i[2] = {i0, i0 + stride < n ? i0 + stride : i0};
+    double r[2] = {0.0, 0.0};
+    if (a.nparts == 0) {
+      r[0] = a.rho[i[0]];
+      r[1] = a.rho[i[1]];
+    } else {
+      int c = 0;
+      for (; c + 4 <= a.nparts; c += 4) {
+        double v[4][2];
 #pragma unroll
-  for (int k = 0; k < NV; k++)
-    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0)
+        for (int u = 0; u < 4; u++)
 #pragma unroll
-    for (int k = 0; k < NV; k++) sh[w * NV + k] = v[k];
-  __syncthreads();
-  if (threadIdx.x == 0)
+          for (int h = 0; h < 2; h++) v[u][h] = a.rho_part[(size_t)(c + u) * n + i[h]];
 #pragma unroll
-    for (int k = 0; k < NV; k++) {
-      double acc = 0.0;
-      for (int i = 0; i < kVW; i++) acc += sh[i * NV + k];
-      v[k] = acc;
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+          for (int h = 0; h < 2; h++) r[h] += v[u][h];
+      }
+      for (; c < a.nparts; c++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) r[h] += a.rho_part[(size_t)c * n + i[h]];
+#pragma unroll
+      for (int h = 0; h < 2; h++) a.rho[i[h]] = r[h] *= a.inv_vol;
     }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      double xf, cf, mf;
+      pz_lda(r[h], xf, cf, mf);
+      a.v[i[h]] = xf + mf;
+      if (h == 0 || i[1] != i[0]) {
+        acc[0] += xf * r[h];
+        acc[1] += cf * r[h];
+        acc[2] += (xf + mf) * r[h];
+      }
+    }
+  }
+  block_sum<3>(acc, red);
+  if (threadIdx.x == 0)
+    for (int k = 0; k < 3; k++) a.part_x[(size_t)blockIdx.x * 3 + k] = acc[k];
 }
 
 // x pass forward: grid (nz, ceil(npair / pr)).  LDS: tw[nx], A[pr][nx], B[pr][nx].
@@ -376,30 +370,11 @@ __global__ __launch_bounds__(kVT) void k_vks_xb(VksArgs a) {
   }
 }
 
-// fixed-order sums of the partials: E_xc = (3/4 ex + ec) Omega/N,
-// muxc = sum V_xc rho Omega/N (cp_pz_lda.C:158-167), E_H = half the sum,
-// E_ext (cp_hart_ext.C:385-387)
 __global__ __launch_bounds__(kVT) void k_vks_sum(const double* __restrict__ px, int nbx,
                                                   const double* __restrict__ pl, int nbl,
                                                   double sc, StepDev* res) {
   __shared__ double red[kVW * 5];
-  double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int i = threadIdx.x; i < nbx; i += kVT) {
-    acc[0] += px[3 * i];
-    acc[1] += px[3 * i + 1];
-    acc[2] += px[3 * i + 2];
-  }
-  for (int i = threadIdx.x; i < nbl; i += kVT) {
-    acc[3] += pl[2 * i];
-    acc[4] += pl[2 * i + 1];
-  }
-  block_sum<5>(acc, red);
-  if (threadIdx.x == 0) {
-    res->exc = (0.75 * acc[0] + acc[1]) * sc;
-    res->muxc = acc[2] * sc;
-    res->ehart = 0.5 * acc[3];
-    res->eloc = acc[4];
-  }
+  vks_sum(px, nbx, pl, nbl, sc, res, red);
 }
 
 // spline of one species at |G| = g (CP_get_vpsnow, cp_hart_ext.C:433-475)
@@ -442,14 +417,24 @@ __global__ __launch_bounds__(kVT) void k_vloc(VksArgs a, PseudoDev p, double2* v
         im -= f * s;
       }
     }
-    vloc[i] = make_double2(re / a.vol, im / a.vol);
+    vloc[a.two_factor ? ((size_t)z * a.nky + j) * a.nkx + kx : i] =
+        make_double2(re / a.vol, im / a.vol);
   }
 }
 
 }  // namespace
 
-int vks_nbx(const VksArgs& a) { return a.nz * (((a.ny + 1) / 2 + a.pr - 1) / a.pr); }
-int vks_nbl(const VksArgs& a) { return a.nkx * ((a.nky + a.lb - 1) / a.lb); }
+int vks_nbx(const VksArgs& a) {
+  if (a.two_factor) {  // of k_rho_xc, two points a thread
+    const size_t n = (size_t)a.nx * a.ny * a.nz;
+    return (int)std::min<size_t>((n + 2 * kVT - 1) / (2 * kVT), 1024);
+  }
+  return a.nz * (((a.ny + 1) / 2 + a.pr - 1) / a.pr);
+}
+int vks_nbl(const VksArgs& a) {
+  if (a.two_factor) return (a.nky * a.nkx + a.lb - 1) / a.lb;
+  return a.nkx * ((a.nky + a.lb - 1) / a.lb);
+}
 
 // x passes: tw, A and B (B also stages nkx x 2 pr half-row values)
 size_t vks_smem_x(const VksArgs& a) {
@@ -464,7 +449,18 @@ size_t vks_smem(const VksArgs& a) {
   return sizeof(double2) * std::max(sx, std::max(sy, sz));
 }
 
-hipError_t vks_build(const VksArgs& a, StepDev* res, hipStream_t st) {
+hipError_t vks_build(const VksArgs& args, StepDev* res, hipStream_t st) {
+  VksArgs a = args;
+  if (a.two_factor) {
+    a.nbx = vks_nbx(a);
+    a.nbl = vks_nbl(a);
+    a.res = res;
+    hipLaunchKernelGGL(k_rho_xc, dim3(a.nbx), dim3(kVT), 0, st, a);
+    const int axis[5] = {a.nx, a.ny, a.nz, a.ny, a.nx};
+    for (int kind = 0; kind < 5; kind++)
+      if (const hipError_t e = vks2_launch(kind, axis[kind], a, st); e != hipSuccess) return e;
+    return hipSuccess;
+  }
   const int npb = ((a.ny + 1) / 2 + a.pr - 1) / a.pr;
   const size_t shx = vks_smem_x(a);
   const size_t shy = sizeof(double2) * (size_t)a.ny * (1 + 2 * a.cb);
