@@ -105,7 +105,8 @@ typedef struct {
                           products (each FP64 operand rounded to FP32 and split exactly into
                           three BF16 terms, the six term products with i + j <= 2 summed in
                           FP32; K-slice partials summed in FP64), bit 0 (default on): the
-                          Lambda gram Re Psi^H F; bit 1: S = Psi^H Psi; bit 2: Psi T, in the
+                          Lambda gram Re Psi^H F; bit 1: S = Psi^H Psi (both FP64 up to 64
+                          states); bit 2: Psi T, in the
                           update form Psi + Psi (T - I); bit 3: the Lambda projection
                           F -= w Psi Lambda.  Bits 2 and 3 apply up to 128 states (FP64
                           above).  The ||Psi^H Psi/2 - I|| residual, Newton-Schulz and the

@@ -321,6 +321,86 @@ __global__ __launch_bounds__(256) void k_gram(GramArgs a, int nbe, int nbe_b, in
   }
 }
 
+// n, nb <= kGramSmall: a wave holds the whole output (NT x NT tiles, the upper ones
+// if SYM) for every fourth chunk of the slice, and the four waves' sums meet in LDS:
+// the tiles past n of the forms above cost 2560 cycles of one SIMD per chunk at 16
+// states, here 256.  S and Lambda of 16 states x 5,150 reals 11 -> 4.4 us each, of
+// 32 states 11 -> 6 and 7 -> 8 (more waves wait for memory at once).
+template <int NT, bool SYM>
+__global__ __launch_bounds__(256) void k_gram_small(GramArgs a, int nlo) {
+  constexpr int NF = SYM ? NT : 2 * NT, NTW = SYM ? NT * (NT + 1) / 2 : NT * NT;
+  __shared__ double sm[2][NTW * 256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
+  const int sp = blockIdx.x;
+  const GSlice s = gram_slice(a, sp, nlo);
+  int row[NF];
+#pragma unroll
+  for (int f = 0; f < NF; f++) {
+    const int r = 16 * (f % NT) + l16;
+    row[f] = r < (f < NT ? a.n : a.nb) ? r : 0;  // rows past n: outputs not stored
+  }
+  v4d acc[NTW];
+#pragma unroll
+  for (int t = 0; t < NTW; t++) acc[t] = vzero();
+  auto mfmas = [&](const double (&f)[NF][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      static_for<0, NTW>([&](auto tc) __attribute__((always_inline)) {
+        constexpr int t = decltype(tc)::value;
+        constexpr int ia = SYM ? up_i(t, NT) : t / NT, ib = SYM ? up_j(t, NT) : NT + t % NT;
+        acc[t] = mfma16(f[ia][e], f[ib][e], acc[t]);
+      });
+  };
+  Frag<NF> ring[kGramRing];
+  chunk_ring(
+      0, (s.c1 - s.c0 - wave + 3) >> 2, ring,
+      [&](int c, Frag<NF>& d) __attribute__((always_inline)) {
+        const int kk = s.base + 16 * (s.c0 + wave + 4 * c) + 4 * g;
+#pragma unroll
+        for (int f = 0; f < NF; f++) gfrag(f < NT ? a.A : a.B, a.lda, row[f], kk, d.f[f]);
+      },
+      [&](int c, const Frag<NF>& d) __attribute__((always_inline)) {
+        const int k0 = s.base + 16 * (s.c0 + wave + 4 * c);
+        if (k0 >= s.rs && k0 + 16 <= s.re) {
+          mfmas(d.f);
+        } else {
+          Frag<NF> m = d;
+#pragma unroll
+          for (int f = 0; f < NF; f++) gmask(k0 + 4 * g, s.rs, s.re, m.f[f]);
+          mfmas(m.f);
+        }
+      });
+  // waves 2, 3 -> 0, 1; wave 1 -> 0
+#pragma unroll
+  for (int half = 2; half >= 1; half--) {
+    if (wave >= half && wave < 2 * half) {
+#pragma unroll
+      for (int t = 0; t < NTW; t++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) sm[wave - half][(4 * t + v) * 64 + lane] = acc[t][v];
+    }
+    __syncthreads();
+    if (wave < half) {
+#pragma unroll
+      for (int t = 0; t < NTW; t++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[t][v] += sm[wave][(4 * t + v) * 64 + lane];
+    }
+    __syncthreads();
+  }
+  if (wave != 0) return;
+  double* part = a.part + (size_t)sp * a.n * a.nb;
+  static_for<0, NTW>([&](auto tc) __attribute__((always_inline)) {
+    constexpr int t = decltype(tc)::value;
+    constexpr int ti = SYM ? up_i(t, NT) : t / NT, tj = SYM ? up_j(t, NT) : t % NT;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int r = 16 * ti + g + 4 * v, col = 16 * tj + l16;
+      if (r < a.n && col < a.nb) part[(size_t)r * a.nb + col] = s.w * acc[t][v];
+    }
+  });
+}
+
 int gram_slices(int n, int K, int k_lo, int sym, int target) {
   const int nbe = (n + kGB - 1) / kGB;
   const int blocks = sym ? nbe * (nbe + 1) / 2 : nbe * nbe;
@@ -334,6 +414,20 @@ hipError_t gram_f64(const GramArgs& a, hipStream_t st) {
   if (a.nslice < 1 || (a.k_lo > 0 && a.k_lo < a.K && a.nslice < 2) || (a.lda & 3) ||
       a.n < 1 || a.nb < 1 || (a.sym && a.nb != a.n))
     return hipErrorInvalidValue;
+  const int edge = std::max(a.n, a.nb);
+  if (edge <= kGramSmall) {
+    void (*const fn)(GramArgs, int) =
+        a.sym ? (edge <= 16   ? k_gram_small<1, true>
+                 : edge <= 32 ? k_gram_small<2, true>
+                 : edge <= 48 ? k_gram_small<3, true>
+                              : k_gram_small<4, true>)
+              : (edge <= 16   ? k_gram_small<1, false>
+                 : edge <= 32 ? k_gram_small<2, false>
+                 : edge <= 48 ? k_gram_small<3, false>
+                              : k_gram_small<4, false>);
+    hipLaunchKernelGGL(fn, dim3(a.nslice), dim3(256), 0, st, a, gram_nlo(a));
+    return hipGetLastError();
+  }
   const int nbe = (a.n + kGB - 1) / kGB, nbe_b = (a.nb + kGB - 1) / kGB;
   const int blocks = a.sym ? nbe * (nbe + 1) / 2 : nbe * nbe_b;
   hipLaunchKernelGGL(k_gram, dim3(blocks, a.nslice), dim3(256), 0, st, a, nbe, nbe_b,
@@ -444,7 +538,9 @@ template <typename P>
 static hipError_t gram_reduce_t(const P* part, int nslice, int n, int nb, int sym, double alpha,
                                 double* C, hipStream_t st) {
   if (sym && nb != n) return hipErrorInvalidValue;
-  if (sym) {
+  // up to 64 states the product wrote whole tiles in FP64 and the plain sum reads the
+  // mirrored elements again: 4.1 us for 16 states, 7.4 by tiles
+  if (sym && !(sizeof(P) == 8 && n <= kGramSmall)) {
     const int nt = (n + 15) >> 4;
     hipLaunchKernelGGL(k_gram_reduce_sym<P>, dim3(4 * (nt * (nt + 1) / 2)), dim3(1024), 0, st,
                        part, nslice, n, alpha, C);
@@ -632,7 +728,7 @@ static RwShape rw_shape(int n) {
 }
 
 // n, ni <= 128: persistent workgroups of 8 waves (two per SIMD).  M is staged
-// once per workgroup in LDS (all 128 x 128, zero beyond ni x n, row stride 129);
+// once per workgroup in LDS (16 NCH x 128, zero beyond ni x n, row stride 129);
 // workgroup b walks the 64-column k-blocks b, b + gridDim.x, ...  Wave w
 // owns the output rows j in [32 (w & 3), +32) and the k tiles 2 (w >> 2),
 // 2 (w >> 2) + 1 of a block.  The work items are (k-block, chunk of 16 i);
@@ -645,7 +741,7 @@ constexpr int rot_ring(bool use_y, bool use_sd) { return use_y && use_sd ? 3 : 4
 constexpr int gcd_c(int a, int b) { return b == 0 ? a : gcd_c(b, a % b); }
 constexpr int kRotLd = 129;                    // LDS row stride of M
 constexpr int kRotThreads = 512;
-constexpr size_t kRotSmem = (size_t)128 * kRotLd * sizeof(double);
+constexpr size_t rot_smem(int nch) { return (size_t)16 * nch * kRotLd * sizeof(double); }
 
 struct XFrag {
   double v[4][2];  // [i step][k tile]
@@ -663,22 +759,6 @@ __global__ __launch_bounds__(kRotThreads) void k_rotate_p(RotArgs a) {
   __shared__ double red[kRotThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  {  // stage M: every load of a thread is issued before its LDS stores
-    constexpr int PER = 128 * 128 / kRotThreads;
-    double mv[PER];
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-      const int e = tid + kRotThreads * u, i = e >> 7, j = e & 127;
-      const double m = a.M[(size_t)min(i, a.ni - 1) * a.n + min(j, a.n - 1)];
-      mv[u] = (i < a.ni && j < a.n) ? m : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-      const int e = tid + kRotThreads * u, i = e >> 7, j = e & 127;
-      msm[i * kRotLd + j] = mv[u];
-    }
-  }
-  __syncthreads();
   const int jb = (wave & 3) * 32, kt0 = 2 * (wave >> 2);
   const bool wact = jb < a.n;
   // Workgroup b owns the 16-column tiles [t0, t1), an even split of all
@@ -753,15 +833,31 @@ __global__ __launch_bounds__(kRotThreads) void k_rotate_p(RotArgs a) {
           acc[x][y][v] = 0.0;
         }
   };
+  // Every load below is issued on every path (items and blocks past the
+  // workgroup's share load clamped addresses and are never stored): a
+  // load that only some paths issue makes the compiler wait for all.
   XFrag ring[RING];
+  static_for<0, RING>([&](auto dc) __attribute__((always_inline)) {
+    constexpr int d = decltype(dc)::value;
+    load(d, ring[d]);
+  });
+  {  // stage M: every load of a thread is issued before its LDS stores
+    constexpr int PER = 16 * NCH * 128 / kRotThreads;
+    double mv[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+      const int e = tid + kRotThreads * u, i = e >> 7, j = e & 127;
+      const double m = a.M[(size_t)min(i, a.ni - 1) * a.n + min(j, a.n - 1)];
+      mv[u] = (i < a.ni && j < a.n) ? m : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+      const int e = tid + kRotThreads * u, i = e >> 7, j = e & 127;
+      msm[i * kRotLd + j] = mv[u];
+    }
+  }
+  __syncthreads();
   if (nitems > 0) {
-    // Every load below is issued on every path (items and blocks past the
-    // workgroup's share load clamped addresses and are never stored): a
-    // load that only some paths issue makes the compiler wait for all.
-    static_for<0, RING>([&](auto dc) __attribute__((always_inline)) {
-      constexpr int d = decltype(dc)::value;
-      load(d, ring[d]);
-    });
     // the epilogue's operands are loaded PRE items before the block ends
     // (short register lifetime, still behind MFMAs)
     constexpr int PRE = NCH >= 3 ? NCH - 3 : 0;
@@ -828,8 +924,9 @@ hipError_t rotate_f64(const RotArgs& args, hipStream_t st) {
                    k_rotate_p<nc, false, true>, k_rotate_p<nc, true, true>
     void (*const fns[16])(RotArgs) = {OA_ROT(1), OA_ROT(2), OA_ROT(4), OA_ROT(8)};
 #undef OA_ROT
-    if (const hipError_t e = grant_lds((const void*)fns[v], kRotSmem); e != hipSuccess) return e;
-    hipLaunchKernelGGL(fns[v], dim3(rotate_pgrid(a.K)), dim3(kRotThreads), kRotSmem, st, a);
+    const size_t sm = rot_smem(1 << (v >> 2));
+    if (const hipError_t e = grant_lds((const void*)fns[v], sm); e != hipSuccess) return e;
+    hipLaunchKernelGGL(fns[v], dim3(rotate_pgrid(a.K)), dim3(kRotThreads), sm, st, a);
     return hipGetLastError();
   }
   if (a.ldx % kRK) return hipErrorInvalidValue;  // whole 64-column blocks inside a row

@@ -227,6 +227,7 @@ hipError_t vloc_build(const VksArgs& a, const PseudoDev& p, double2* vloc, hipSt
 // K slices (slices never straddle k_lo).  sym: B == A, only the 16 x 16
 // tiles with i/16 <= j/16 are computed.
 // C[i][j] = sum_k w(k) A[i][k] B[j][k], i < n, j < nb (nb == n when sym)
+constexpr int kGramSmall = 64;  // states up to which a wave takes a whole gram
 struct GramArgs {
   const double* A;
   const double* B;
@@ -344,8 +345,6 @@ struct CgDev {
 };
 
 // ---- pointwise G-space kernels (oa_pointwise.hip) ----
-// gamma of the new direction from res->fnorm2 (one thread); the state advances
-hipError_t cg_gamma(const StepDev* res, CgDev* cg, hipStream_t st);
 // cg = gamma cg + F where g2 <= ecut; psi += dtm cg (cp_min_CG.C:55-105)
 hipError_t cg_update(double2* psi, double2* cgdir, const double2* f, const double* dtm,
                      const double* g2, const int* twin, double ecut, int nst, int npts, int ld,
@@ -360,7 +359,15 @@ hipError_t sd_update(double2* psi, const double2* f, const double* dtm, const in
 hipError_t red_sync(double2* psi, const int* red, const int* partner, int nred, int nst, int ld,
                     hipStream_t st);
 // sum of parts -> res field (deterministic single-workgroup reduction)
-hipError_t reduce_to(const double* part, int n, double scale, double* out, hipStream_t st);
+// *out = scale * sum of part[n], up to three sums; cg: the first is |F|^2 of a new
+// conjugate-gradient direction, whose state advances with gamma
+struct RedJob {
+  const double* part;
+  int n;
+  double scale;
+  double* out;
+};
+hipError_t reduce_to(const RedJob* jobs, int njobs, CgDev* cg, hipStream_t st);
 // sum_r V rho partials
 hipError_t dot_parts(const double* a, const double* b, size_t n, double* part, int nparts,
                      hipStream_t st);

@@ -1,7 +1,7 @@
 // oa_pointwise.hip -- G-space pointwise kernels and small reductions of the
 // CP electronic step.
 //   k_sd       : psi += dt/m F  (CP_integrate_min_STD, cp_min_std.C:56-86)
-//   k_cg_gamma, k_cg_update : conjugate-gradient direction and update
+//   cg_gamma, k_cg_update : conjugate-gradient direction and update
 //                (CP_integrate_min_CG, cp_min_CG.C:55-105; reset rule
 //                 CP_State_GSpacePlane.C:2646-2671)
 //   k_red_sync : redundant kx=0 points <- conj(partner)
@@ -61,12 +61,11 @@ hipError_t sd_update(double2* psi, const double2* f, const double* dtm, const in
 // (:2651-2671): gamma = 0 on the first iteration, or when |F| grew by more
 // than 5% after at least five steps without a reset, or more than doubled;
 // else fovlap / fovlap_old.
-__global__ void k_cg_gamma(const StepDev* __restrict__ res, CgDev* __restrict__ cg) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__device__ __forceinline__ void cg_gamma(double fnorm2, CgDev* __restrict__ cg) {
   CgDev s = *cg;
   s.fovlap_old = s.fovlap;
   s.fmag_old = s.fmag;
-  s.fovlap = res->fnorm2;
+  s.fovlap = fnorm2;
   s.fmag = sqrt(s.fovlap);
   s.iter++;
   int reset = 0;
@@ -80,11 +79,6 @@ __global__ void k_cg_gamma(const StepDev* __restrict__ res, CgDev* __restrict__ 
   s.num_reset++;
   s.gamma = reset ? 0.0 : s.fovlap / s.fovlap_old;
   *cg = s;
-}
-
-hipError_t cg_gamma(const StepDev* res, CgDev* cg, hipStream_t st) {
-  hipLaunchKernelGGL(k_cg_gamma, dim3(1), dim3(64), 0, st, res, cg);
-  return hipGetLastError();
 }
 
 // cg = gamma cg + F where g2 <= ecut; psi += dt/m cg (cp_min_CG.C:55-105), and
@@ -161,12 +155,17 @@ hipError_t red_sync(double2* psi, const int* red, const int* partner, int nred, 
   return hipGetLastError();
 }
 
-// One workgroup; each thread's loads are issued eight at a time
-// (branch-free: index clamped, value masked) rather than one per iteration
+// One workgroup per sum; each thread's loads are issued eight at a time
+// (branch-free: index clamped, value masked) rather than one per iteration.  cg:
+// the first sum is |F|^2 of a new conjugate-gradient direction.  The sums of a step
+// (EKE, E_loc, |F|^2 and the direction's gamma) were four launches of 3 us, with as
+// much again between them.
 constexpr int kRedThreads = 1024;
-__global__ __launch_bounds__(kRedThreads) void k_reduce_to(const double* __restrict__ part, int n,
-                                                           double scale,
-                                                           double* __restrict__ out) {
+__global__ __launch_bounds__(kRedThreads) void k_reduce_to(RedJob j0, RedJob j1, RedJob j2,
+                                                           CgDev* cg) {
+  const RedJob j = blockIdx.x == 0 ? j0 : blockIdx.x == 1 ? j1 : j2;
+  const double* __restrict__ part = j.part;
+  const int n = j.n;
   double v = 0.0;
   for (int i0 = 0; i0 < n; i0 += 8 * kRedThreads) {
     double a[8];
@@ -180,12 +179,18 @@ __global__ __launch_bounds__(kRedThreads) void k_reduce_to(const double* __restr
     for (int u = 0; u < 8; u++) v += a[u];
   }
   const double t = block_sum(v);
-  if (threadIdx.x == 0) *out = t * scale;
+  if (threadIdx.x == 0) {
+    *j.out = t * j.scale;
+    if (cg && blockIdx.x == 0) cg_gamma(t * j.scale, cg);
+  }
 }
 
-hipError_t reduce_to(const double* part, int n, double scale, double* out, hipStream_t st) {
-  if (n < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(kRedThreads), 0, st, part, n, scale, out);
+hipError_t reduce_to(const RedJob* jobs, int njobs, CgDev* cg, hipStream_t st) {
+  if (njobs < 1 || njobs > 3) return hipErrorInvalidValue;
+  for (int i = 0; i < njobs; i++)
+    if (jobs[i].n < 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_reduce_to, dim3(njobs), dim3(kRedThreads), 0, st, jobs[0],
+                     jobs[std::min(1, njobs - 1)], jobs[njobs - 1], cg);
   return hipGetLastError();
 }
 

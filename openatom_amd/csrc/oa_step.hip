@@ -184,6 +184,10 @@ struct oa_ctx {
   char* pin = nullptr;
   size_t pin_slot = 0;
   hipEvent_t pin_ev[kStageRing] = {};
+  // the step's EKE and E_loc sums wait for the one of |F|^2 (energies_later)
+  bool energies_later = false;
+  int energy_jobs = 0;
+  oa::RedJob energies[2];
   int ns_kind = 0;  // Newton-Schulz form: NsArgs::coop
   int ns_seen = 0;  // iterations of the last result fetched (0: none yet)
   bool sd_fused = false;  // SD update inside the Lambda rotate (nst <= 128)
@@ -741,7 +745,7 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
           hipSuccess || ncu <= 0)
     ncu = 256;
   c->nslice_sym = oa::gram_slices(n, K, 2 * c->nkx0, 1, ncu);
-  const bool split_lam = split_on(c, kSplitLambda);
+  const bool split_lam = split_on(c, kSplitLambda) && n > oa::kGramSmall;
   c->nslice_full = split_lam ? oa::gram_bf16_slices(n, K, ncu)
                              : oa::gram_slices(n, K, 2 * c->nkx0, 0, ncu);
   int max_sym = c->nslice_sym, max_full = c->nslice_full;
@@ -987,9 +991,24 @@ oa_status st_g2r(oa_ctx* c, int ev0 = -1) {
 // The EKE and E_loc reductions at the end of the R->G transform.
 oa_status st_energies(oa_ctx* c) {
   const size_t N = (size_t)c->nx * c->ny * c->nz;
-  HIPCHK(oa::reduce_to(c->eke_part, c->nst * c->nzblk, 1.0, &c->res->eke, c->stream));
+  c->energy_jobs = 0;
+  c->energies[c->energy_jobs++] = {c->eke_part, c->nst * c->nzblk, 1.0, &c->res->eke};
   if (!c->opt.vks_from_rho)  // else E_ext came with V_KS
-    HIPCHK(oa::reduce_to(c->dpart, c->ndpart, c->vol / (double)N, &c->res->eloc, c->stream));
+    c->energies[c->energy_jobs++] = {c->dpart, c->ndpart, c->vol / (double)N, &c->res->eloc};
+  if (c->energies_later) return OA_OK;
+  HIPCHK(oa::reduce_to(c->energies, c->energy_jobs, nullptr, c->stream));
+  c->energy_jobs = 0;
+  return OA_OK;
+}
+
+// |F|^2 from np partials (cg: and the direction's gamma), with the energy sums that
+// are still due
+oa_status reduce_fnorm(oa_ctx* c, int np, oa::CgDev* cg = nullptr) {
+  oa::RedJob jobs[3] = {{c->fpart, np, 1.0, &c->res->fnorm2}};
+  int n = 1;
+  for (int i = 0; i < c->energy_jobs; i++) jobs[n++] = c->energies[i];
+  c->energy_jobs = 0;
+  HIPCHK(oa::reduce_to(jobs, n, cg, c->stream));
   return OA_OK;
 }
 
@@ -1067,7 +1086,7 @@ oa_status st_gram(oa_ctx* c, const double2* A, const double2* B, bool sym, doubl
   g.nslice = sym ? c->nslice_sym : c->nslice_full;
   g.part = c->gpart;
   g.nb = c->nst;
-  if (split) {  // FP32 partials in the same buffer
+  if (split && c->nst > oa::kGramSmall) {  // FP32 partials in the same buffer
     float* pf = reinterpret_cast<float*>(c->gpart);
     HIPCHK(oa::gram_bf16(g, pf, c->stream));
     HIPCHK(oa::gram_reduce_f32(pf, g.nslice, c->nst, c->nst, g.sym, 1.0, C, c->stream));
@@ -1134,8 +1153,7 @@ oa_status st_lambda(oa_ctx* c, bool with_sd = false) {
 // |F|^2 from the partials of the fused rotate (FP64 kernel), then the
 // redundancy sync
 oa_status st_sd_finish(oa_ctx* c) {
-  HIPCHK(oa::reduce_to(c->fpart, oa::rotate_nwg(c->nst, 2 * c->npts), 1.0, &c->res->fnorm2,
-                       c->stream));
+  TRY(reduce_fnorm(c, oa::rotate_nwg(c->nst, 2 * c->npts)));
   HIPCHK(oa::red_sync(c->psi, c->red, c->partner, c->nred, c->nst, c->ld, c->stream));
   return OA_OK;
 }
@@ -1146,8 +1164,7 @@ oa_status st_lambda_cg(oa_ctx* c) {
   TRY(st_gram(c, c->psi, c->force, false, 1.0, 1.0, c->lam, split_on(c, kSplitLambda)));
   TRY(st_rotate(c, c->psi, c->lam, c->force, 1.0, -0.5, -1.0, false, true,
                 split_on(c, kSplitProj) && split_rotate_ok(c)));
-  HIPCHK(oa::reduce_to(c->fpart, lambda_nwg(c), 1.0, &c->res->fnorm2, c->stream));
-  HIPCHK(oa::cg_gamma(c->res, c->cgs, c->stream));
+  TRY(reduce_fnorm(c, lambda_nwg(c), c->cgs));
   HIPCHK(oa::cg_update(c->psi, c->cgdir, c->force, c->dtm, c->g2, c->sd_twin, c->ecut_ry, c->nst,
                        c->npts, c->ld, c->cgs, c->stream));
   return OA_OK;
@@ -1204,7 +1221,7 @@ oa_status st_nonlocal(oa_ctx* c) {
 oa_status st_sd(oa_ctx* c) {
   HIPCHK(oa::sd_update(c->psi, c->force, c->dtm, c->sd_twin, c->nst, c->npts, c->ld, c->fpart,
                        c->nfpart, c->stream));
-  HIPCHK(oa::reduce_to(c->fpart, c->nfpart, 1.0, &c->res->fnorm2, c->stream));
+  TRY(reduce_fnorm(c, c->nfpart));
   return OA_OK;
 }
 
@@ -2066,7 +2083,8 @@ oa_status oa_vpsi_r2g_states(oa_ctx* c, int s0, int ns, double* eke) {
   HIPCHK(oa::plane3_launch(1, c->nx, c->fp32, f, c->stream));
   f.zbuf = f.zout;  // the z pass back reads the R->G plane output
   HIPCHK(oa::fft2_launch(oa::FFT_ZBWD, c->nz, c->fp32, f, c->stream));
-  HIPCHK(oa::reduce_to(f.eke_part, ns * c->nzblk, 1.0, &c->res->eke, c->stream));
+  const oa::RedJob job = {f.eke_part, ns * c->nzblk, 1.0, &c->res->eke};
+  HIPCHK(oa::reduce_to(&job, 1, nullptr, c->stream));
   TRY(fetch_result(c, nullptr));
   if (eke) *eke = c->res_host->eke;
   return OA_OK;
@@ -2145,12 +2163,16 @@ oa_status enqueue_pre(oa_ctx* c, bool marks) {
   auto mk = [&](int i) {
     if (marks) mark(c, i);
   };
+  c->energies_later = true;  // their sums: with |F|^2 below
+  oa_status s = OA_OK;
   if (c->fuse_rho) {
-    TRY(st_g2r2g_rho(c, marks ? 1 : -1));  // marks 1..6, then the EKE / E_loc reductions
+    s = st_g2r2g_rho(c, marks ? 1 : -1);  // marks 1..6
   } else {
-    TRY(st_g2r(c, marks ? 1 : -1));  // marks 1..3
-    TRY(st_r2g(c, marks ? 1 : -1));  // marks 4..6, then the EKE / E_loc reductions
+    s = st_g2r(c, marks ? 1 : -1);                   // marks 1..3
+    if (s == OA_OK) s = st_r2g(c, marks ? 1 : -1);  // marks 4..6
   }
+  c->energies_later = false;
+  TRY(s);
   if (c->nl_natm > 0) TRY(st_nonlocal(c));  // timed with the Lambda stage
   if (c->opt.use_cg) {
     TRY(st_lambda_cg(c));
