@@ -4,9 +4,9 @@
 //   gram    : S = 2 Re Psi^H Psi over stored points with kx=0 halved
 //             (PairCalculator::multiplyForward, ckPairCalculator.C:682-802)
 //             and Lambda = Re Psi^H F (asymmetric PairCalculator, alpha = 1).
-//             One workgroup owns a 128 x 128 output block and one slice of
-//             the long point axis, so each slice of Psi is read once per
-//             block; the slices' partial blocks are summed in a fixed order.
+//             One workgroup owns a 64 x 64 (48 x 48) output block and one
+//             slice of the long point axis; the slices' partial blocks are
+//             summed in a fixed order.
 //   rotate  : Psi' = Psi T and F -= w Psi Lambda
 //             (bwMultiplyHelper, ckPairCalculator.C:1189-1425;
 //              unpackLambda, CP_State_GSpacePlane.C:2045-2225), optionally
@@ -28,6 +28,7 @@
 #include <hip/hip_cooperative_groups.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "oa_common.h"
@@ -45,16 +46,8 @@ __device__ __forceinline__ v4d mfma16(double a, double b, v4d c) {
 __device__ __forceinline__ v4d vzero() { return (v4d){0.0, 0.0, 0.0, 0.0}; }
 
 // ================================================================== gram
-constexpr int kGB = 128;        // output block edge
+constexpr int kGB = 128;        // rows of a skinny block
 
-// Diagonal block of the symmetric product: its 36 upper tiles (ti <= tj) in
-// four groups with few distinct row fragments per wave:
-//   wave 0: ti <= tj < 4           (10 tiles, row tiles 0-3)
-//   wave 1: ti in {0,1}, tj >= 4   ( 8 tiles, row tiles 0,1,4-7)
-//   wave 2: ti in {2,3}, tj >= 4   ( 8 tiles, row tiles 2,3,4-7)
-//   wave 3: 4 <= ti <= tj          (10 tiles, row tiles 4-7)
-// Fragment slot f of wave W holds row tile dg_rt(W, f); tile t of wave W is
-// the product of slots dg_a(W, t) and dg_b(W, t).
 __host__ __device__ constexpr int up_i(int idx, int m) {
   int i = 0;
   while (idx >= m - i) {
@@ -71,18 +64,6 @@ __host__ __device__ constexpr int up_j(int idx, int m) {
   }
   return i + idx;
 }
-__host__ __device__ constexpr int dg_nf(int W) { return (W == 0 || W == 3) ? 4 : 6; }
-__host__ __device__ constexpr int dg_nt(int W) { return (W == 0 || W == 3) ? 10 : 8; }
-__host__ __device__ constexpr int dg_rt(int W, int f) {
-  return W == 0 ? f : W == 3 ? 4 + f : W == 2 ? 2 + f : (f < 2 ? f : 2 + f);
-}
-__host__ __device__ constexpr int dg_a(int W, int t) {
-  return (W == 0 || W == 3) ? up_i(t, 4) : t / 4;
-}
-__host__ __device__ constexpr int dg_b(int W, int t) {
-  return (W == 0 || W == 3) ? up_j(t, 4) : 2 + t % 4;
-}
-
 // f[e] = X[row][kk + e]: one 32-byte load, kk a multiple of 4 inside the
 // row's allocation (chunks start on multiples of 16 below K <= lda, lda a
 // multiple of 16).  Unconditional: rows past the matrix are clamped by the
@@ -109,124 +90,6 @@ struct Frag {
   double f[NF][4];
 };
 constexpr int kGramRing = 3;
-
-// Diagonal block of the symmetric product, wave W (tile groups above); the
-// row fragments serve as both operands.
-template <int W>
-__device__ __forceinline__ void gram_diag_wave(const GramArgs& a, const GSlice& s, int sp,
-                                               int bi) {
-  constexpr int NF = dg_nf(W), NTW = dg_nt(W);
-  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
-  int row[NF];
-#pragma unroll
-  for (int f = 0; f < NF; f++) {
-    const int r = bi * kGB + 16 * dg_rt(W, f) + l16;
-    row[f] = r < a.n ? r : 0;  // rows past n: outputs not stored
-  }
-  v4d acc[NTW];
-#pragma unroll
-  for (int t = 0; t < NTW; t++) acc[t] = vzero();
-  auto mfmas = [&](const double (&f)[NF][4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-      static_for<0, NTW>([&](auto tc) __attribute__((always_inline)) {
-        constexpr int t = decltype(tc)::value;
-        constexpr int ia = dg_a(W, t), ib = dg_b(W, t);
-        acc[t] = mfma16(f[ia][e], f[ib][e], acc[t]);
-      });
-  };
-  Frag<NF> ring[kGramRing];
-  chunk_ring(
-      s.c0, s.c1, ring,
-      [&](int c, Frag<NF>& d) __attribute__((always_inline)) {
-        const int kk = s.base + 16 * c + 4 * g;
-#pragma unroll
-        for (int f = 0; f < NF; f++) gfrag(a.A, a.lda, row[f], kk, d.f[f]);
-      },
-      [&](int c, const Frag<NF>& d) __attribute__((always_inline)) {
-        const int k0 = s.base + 16 * c;
-        if (k0 >= s.rs && k0 + 16 <= s.re) {
-          mfmas(d.f);
-        } else {  // a chunk at the region's edge (both operands are these rows)
-          Frag<NF> m = d;
-#pragma unroll
-          for (int f = 0; f < NF; f++) gmask(k0 + 4 * g, s.rs, s.re, m.f[f]);
-          mfmas(m.f);
-        }
-      });
-  double* part = a.part + (size_t)sp * a.n * a.n;
-#pragma unroll
-  for (int t = 0; t < NTW; t++) {
-    const int r0 = bi * kGB + 16 * dg_rt(W, dg_a(W, t));
-    const int c0 = bi * kGB + 16 * dg_rt(W, dg_b(W, t));
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int r = r0 + g + 4 * v, col = c0 + l16;
-      if (r < a.n && col < a.n) part[(size_t)r * a.n + col] = s.w * acc[t][v];
-    }
-  }
-}
-
-// Full block: wave (wr, wc) owns the 64 x 64 quadrant (4 x 4 tiles).
-__device__ __forceinline__ void gram_full_wave(const GramArgs& a, const double* __restrict__ B,
-                                               const GSlice& s, int sp, int bi, int bj) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
-  const int wr = wave >> 1, wc = wave & 1;
-  const int rbase = bi * kGB + wr * 64, cbase = bj * kGB + wc * 64;
-  if (rbase >= a.n || cbase >= a.nb) return;
-  int ra[4], rb[4];
-#pragma unroll
-  for (int x = 0; x < 4; x++) {  // rows past the matrices: outputs not stored
-    const int r = rbase + 16 * x + l16, q = cbase + 16 * x + l16;
-    ra[x] = r < a.n ? r : 0;
-    rb[x] = q < a.nb ? q : 0;
-  }
-  v4d acc[4][4];
-#pragma unroll
-  for (int x = 0; x < 4; x++)
-#pragma unroll
-    for (int y = 0; y < 4; y++) acc[x][y] = vzero();
-  auto mfmas = [&](const double (&f)[8][4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-#pragma unroll
-      for (int x = 0; x < 4; x++)
-#pragma unroll
-        for (int y = 0; y < 4; y++) acc[x][y] = mfma16(f[x][e], f[4 + y][e], acc[x][y]);
-  };
-  Frag<8> ring[kGramRing];  // fragments 0-3: rows of A, 4-7: rows of B
-  chunk_ring(
-      s.c0, s.c1, ring,
-      [&](int c, Frag<8>& d) __attribute__((always_inline)) {
-        const int kk = s.base + 16 * c + 4 * g;
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-          gfrag(a.A, a.lda, ra[x], kk, d.f[x]);
-          gfrag(B, a.lda, rb[x], kk, d.f[4 + x]);
-        }
-      },
-      [&](int c, const Frag<8>& d) __attribute__((always_inline)) {
-        const int k0 = s.base + 16 * c;
-        if (k0 >= s.rs && k0 + 16 <= s.re) {
-          mfmas(d.f);
-        } else {  // a chunk at the region's edge (padding past K may hold anything)
-          Frag<8> m = d;
-#pragma unroll
-          for (int x = 0; x < 8; x++) gmask(k0 + 4 * g, s.rs, s.re, m.f[x]);
-          mfmas(m.f);
-        }
-      });
-  double* part = a.part + (size_t)sp * a.n * a.nb;
-#pragma unroll
-  for (int x = 0; x < 4; x++)
-#pragma unroll
-    for (int y = 0; y < 4; y++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int r = rbase + 16 * x + g + 4 * v, col = cbase + 16 * y + l16;
-        if (r < a.n && col < a.nb) part[(size_t)r * a.nb + col] = s.w * acc[x][y][v];
-      }
-}
 
 // Skinny block (nb <= 32 columns, e.g. the non-local projections of one
 // atom set): wave w owns rows [32 w, 32 w + 32) of the 128-row block and
@@ -290,54 +153,26 @@ __device__ __forceinline__ void gram_skinny_wave(const GramArgs& a, const double
       }
 }
 
-// grid (output blocks, K slices); nbe = row blocks (blocks per edge when
-// symmetric), nbe_b = column blocks, nlo = slices of the kx=0 region
-__global__ __launch_bounds__(256) void k_gram(GramArgs a, int nbe, int nbe_b, int nlo) {
-  int bi, bj, b = blockIdx.x;
-  if (a.sym) {
-    bi = 0;
-    while (b >= nbe - bi) {
-      b -= nbe - bi;
-      bi++;
-    }
-    bj = bi + b;
-  } else {
-    bi = b / nbe_b;
-    bj = b - bi * nbe_b;
-  }
-  const int sp = blockIdx.y;
-  const GSlice s = gram_slice(a, sp, nlo);
-  if (a.sym && bi == bj) {
-    switch (threadIdx.x >> 6) {
-      case 0: gram_diag_wave<0>(a, s, sp, bi); break;
-      case 1: gram_diag_wave<1>(a, s, sp, bi); break;
-      case 2: gram_diag_wave<2>(a, s, sp, bi); break;
-      default: gram_diag_wave<3>(a, s, sp, bi); break;
-    }
-  } else if (!a.sym && a.nb <= 32) {
-    gram_skinny_wave(a, a.B, s, sp, bi);
-  } else {
-    gram_full_wave(a, a.sym ? a.A : a.B, s, sp, bi, bj);
-  }
+// nb <= 32 < n: grid (row blocks, K slices)
+__global__ __launch_bounds__(256) void k_gram_skinny(GramArgs a, int nlo) {
+  gram_skinny_wave(a, a.B, gram_slice(a, blockIdx.y, nlo), blockIdx.y, blockIdx.x);
 }
 
-// n, nb <= kGramSmall: a wave holds the whole output (NT x NT tiles, the upper ones
-// if SYM) for every fourth chunk of the slice, and the four waves' sums meet in LDS:
-// the tiles past n of the forms above cost 2560 cycles of one SIMD per chunk at 16
-// states, here 256.  S and Lambda of 16 states x 5,150 reals 11 -> 4.4 us each, of
-// 32 states 11 -> 6 and 7 -> 8 (more waves wait for memory at once).
-template <int NT, bool SYM>
-__global__ __launch_bounds__(256) void k_gram_small(GramArgs a, int nlo) {
-  constexpr int NF = SYM ? NT : 2 * NT, NTW = SYM ? NT * (NT + 1) / 2 : NT * NT;
-  __shared__ double sm[2][NTW * 256];
+// Output block of MT x NT tiles from tile (ti0, tj0) (DIAG: the upper ones of a
+// diagonal block of a symmetric product): each wave holds all of it for every fourth
+// chunk of the slice, and the four waves' sums meet in LDS (2 x SM doubles).
+template <int MT, int NT, bool DIAG, int SM>
+__device__ __forceinline__ void gram_block(const GramArgs& a, const double* __restrict__ B,
+                                           const GSlice& s, int sp, int ti0, int tj0,
+                                           double (*sm)[SM]) {
+  constexpr int NF = DIAG ? NT : MT + NT, NTW = DIAG ? NT * (NT + 1) / 2 : MT * NT;
+  static_assert(NTW * 256 <= SM && (!DIAG || MT == NT), "");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
-  const int sp = blockIdx.x;
-  const GSlice s = gram_slice(a, sp, nlo);
   int row[NF];
 #pragma unroll
   for (int f = 0; f < NF; f++) {
-    const int r = 16 * (f % NT) + l16;
-    row[f] = r < (f < NT ? a.n : a.nb) ? r : 0;  // rows past n: outputs not stored
+    const int r = 16 * (f < MT ? ti0 + f : tj0 + f - MT) + l16;
+    row[f] = r < (f < MT ? a.n : a.nb) ? r : 0;  // rows past n: outputs not stored
   }
   v4d acc[NTW];
 #pragma unroll
@@ -347,7 +182,7 @@ __global__ __launch_bounds__(256) void k_gram_small(GramArgs a, int nlo) {
     for (int e = 0; e < 4; e++)
       static_for<0, NTW>([&](auto tc) __attribute__((always_inline)) {
         constexpr int t = decltype(tc)::value;
-        constexpr int ia = SYM ? up_i(t, NT) : t / NT, ib = SYM ? up_j(t, NT) : NT + t % NT;
+        constexpr int ia = DIAG ? up_i(t, NT) : t / NT, ib = DIAG ? up_j(t, NT) : MT + t % NT;
         acc[t] = mfma16(f[ia][e], f[ib][e], acc[t]);
       });
   };
@@ -357,13 +192,13 @@ __global__ __launch_bounds__(256) void k_gram_small(GramArgs a, int nlo) {
       [&](int c, Frag<NF>& d) __attribute__((always_inline)) {
         const int kk = s.base + 16 * (s.c0 + wave + 4 * c) + 4 * g;
 #pragma unroll
-        for (int f = 0; f < NF; f++) gfrag(f < NT ? a.A : a.B, a.lda, row[f], kk, d.f[f]);
+        for (int f = 0; f < NF; f++) gfrag(f < MT ? a.A : B, a.lda, row[f], kk, d.f[f]);
       },
       [&](int c, const Frag<NF>& d) __attribute__((always_inline)) {
         const int k0 = s.base + 16 * (s.c0 + wave + 4 * c);
         if (k0 >= s.rs && k0 + 16 <= s.re) {
           mfmas(d.f);
-        } else {
+        } else {  // a chunk at the region's edge (padding past K may hold anything)
           Frag<NF> m = d;
 #pragma unroll
           for (int f = 0; f < NF; f++) gmask(k0 + 4 * g, s.rs, s.re, m.f[f]);
@@ -392,46 +227,113 @@ __global__ __launch_bounds__(256) void k_gram_small(GramArgs a, int nlo) {
   double* part = a.part + (size_t)sp * a.n * a.nb;
   static_for<0, NTW>([&](auto tc) __attribute__((always_inline)) {
     constexpr int t = decltype(tc)::value;
-    constexpr int ti = SYM ? up_i(t, NT) : t / NT, tj = SYM ? up_j(t, NT) : t % NT;
+    constexpr int ti = DIAG ? up_i(t, NT) : t / NT, tj = DIAG ? up_j(t, NT) : t % NT;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      const int r = 16 * ti + g + 4 * v, col = 16 * tj + l16;
+      const int r = 16 * (ti0 + ti) + g + 4 * v, col = 16 * (tj0 + tj) + l16;
       if (r < a.n && col < a.nb) part[(size_t)r * a.nb + col] = s.w * acc[t][v];
     }
   });
 }
 
-int gram_slices(int n, int K, int k_lo, int sym, int target) {
-  const int nbe = (n + kGB - 1) / kGB;
-  const int blocks = sym ? nbe * (nbe + 1) / 2 : nbe * nbe;
-  int ns = std::max(2, target / std::max(1, blocks));
-  ns = std::min(ns, std::max(2, K / 64));  // at least four chunks per slice
-  (void)k_lo;
-  return ns;
+// One-dimensional grid of (K slice, output block), blocks fastest, a contiguous
+// range of it for each XCD: the blocks of a slice read the same rows at about the
+// same time through one L2.  With the sums of the slices, in us (before: 128 x 128
+// blocks of four different waves, idle where n is not a multiple of 128): S of 84 states
+// x 30,024 reals 23 (26), 128 x 58,400 37 (38), 132 46 (103), 180 x 73,412 82 (130),
+// 256 x 121,214 194 (220), 512 x 236,230 1071 (1277); full products 25 (32), 45 (51), 57
+// (140), 98 (174), 254 (287), 1839 (2012).  Bound by the matrix pipe, 61 to 66 TFLOP/s
+// from 256 states up, and by the start and end of a slice below.
+template <int NT>
+__global__ __launch_bounds__(256) void k_gram(GramArgs a, int nbe, int nbe_b, int nblk, int nlo) {
+  __shared__ double sm[2][NT * NT * 256];
+  const int total = gridDim.x, xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
+  const int q = total >> 3, r = total & 7;
+  const int logical = xcd * q + min(xcd, r) + k;
+  const int sp = logical / nblk;
+  int b = logical - sp * nblk, bi, bj;
+  const GSlice s = gram_slice(a, sp, nlo);
+  if (a.sym && NT == 4 && nblk == 4) {  // GramShape: two diagonal blocks, two halves
+    if (b < 2)
+      gram_block<NT, NT, true>(a, a.A, s, sp, NT * b, NT * b, sm);
+    else
+      gram_block<(NT + 1) / 2, NT, false>(a, a.A, s, sp, NT / 2 * (b - 2), NT, sm);
+    return;
+  }
+  if (a.sym) {
+    bi = 0;
+    while (b >= nbe - bi) {
+      b -= nbe - bi;
+      bi++;
+    }
+    bj = bi + b;
+    if (bi == bj) {
+      gram_block<NT, NT, true>(a, a.A, s, sp, NT * bi, NT * bi, sm);
+      return;
+    }
+  } else {
+    bi = b / nbe_b;
+    bj = b - bi * nbe_b;
+  }
+  gram_block<NT, NT, false>(a, a.sym ? a.A : a.B, s, sp, NT * bi, NT * bj, sm);
+}
+
+// Tiles per block edge and blocks of the output: a single block up to 64 rows and
+// columns, else blocks of 3 or 4 tiles, whichever computes fewer tiles (9 tiles an
+// edge: 45 instead of 78 for the symmetric product), 4 where they are equal (more
+// products per loaded row).  With two blocks an edge of 4 tiles the one off the
+// diagonal of a symmetric product is cut in two, so that no workgroup has more than 10
+// tiles (no other symmetric product has 4 blocks): 128 states 43 -> 37 us.
+struct GramShape {
+  int nt, nbe, nbe_b, blocks;
+};
+static GramShape gram_shape(int n, int nb, int sym) {
+  auto shape = [&](int nt) {
+    const int w = 16 * nt, e = (n + w - 1) / w, f = (nb + w - 1) / w;
+    return GramShape{nt, e, f, sym ? e * (e + 1) / 2 : e * f};
+  };
+  auto tiles = [&](const GramShape& s) {
+    const int full = s.nt * s.nt, diag = s.nt * (s.nt + 1) / 2;
+    return sym ? s.nbe * diag + (s.blocks - s.nbe) * full : s.blocks * full;
+  };
+  const int edge = std::max(n, nb);
+  if (edge <= kGramSmall) return shape((edge + 15) / 16);
+  const GramShape s3 = shape(3);
+  GramShape s4 = shape(4);
+  if (tiles(s3) < tiles(s4)) return s3;
+  if (sym && s4.nbe == 2) s4.blocks = 4;
+  return s4;
+}
+
+static bool gram_skinny(int n, int nb, int sym) { return !sym && nb <= 32 && n > kGramSmall; }
+
+int gram_slices(int n, int nb, int K, int sym, int ncu) {
+  const int blocks = gram_skinny(n, nb, sym) ? (n + kGB - 1) / kGB : gram_shape(n, nb, sym).blocks;
+  // whole rounds of a workgroup per CU, the more the longer (about 200 chunks a wave):
+  // then the lighter blocks on the diagonal even out (512 states: 7 slices 1.15 ms, 14
+  // 1.07; but 128 states: 64 slices 37 us, 128 47)
+  const double rounds = (double)(K / 64) / 200.0 * blocks / ncu;
+  const int ns = std::max(1, (int)std::ceil(rounds - 0.25)) * ncu / blocks;
+  return std::min(std::max(2, ns), std::max(2, K / 64));  // four chunks or more each
 }
 
 hipError_t gram_f64(const GramArgs& a, hipStream_t st) {
   if (a.nslice < 1 || (a.k_lo > 0 && a.k_lo < a.K && a.nslice < 2) || (a.lda & 3) ||
       a.n < 1 || a.nb < 1 || (a.sym && a.nb != a.n))
     return hipErrorInvalidValue;
-  const int edge = std::max(a.n, a.nb);
-  if (edge <= kGramSmall) {
-    void (*const fn)(GramArgs, int) =
-        a.sym ? (edge <= 16   ? k_gram_small<1, true>
-                 : edge <= 32 ? k_gram_small<2, true>
-                 : edge <= 48 ? k_gram_small<3, true>
-                              : k_gram_small<4, true>)
-              : (edge <= 16   ? k_gram_small<1, false>
-                 : edge <= 32 ? k_gram_small<2, false>
-                 : edge <= 48 ? k_gram_small<3, false>
-                              : k_gram_small<4, false>);
-    hipLaunchKernelGGL(fn, dim3(a.nslice), dim3(256), 0, st, a, gram_nlo(a));
+  const int nlo = gram_nlo(a);
+  if (gram_skinny(a.n, a.nb, a.sym)) {
+    hipLaunchKernelGGL(k_gram_skinny, dim3((a.n + kGB - 1) / kGB, a.nslice), dim3(256), 0, st, a,
+                       nlo);
     return hipGetLastError();
   }
-  const int nbe = (a.n + kGB - 1) / kGB, nbe_b = (a.nb + kGB - 1) / kGB;
-  const int blocks = a.sym ? nbe * (nbe + 1) / 2 : nbe * nbe_b;
-  hipLaunchKernelGGL(k_gram, dim3(blocks, a.nslice), dim3(256), 0, st, a, nbe, nbe_b,
-                     gram_nlo(a));
+  const GramShape s = gram_shape(a.n, a.nb, a.sym);
+  void (*const fn)(GramArgs, int, int, int, int) = s.nt == 1   ? k_gram<1>
+                                                   : s.nt == 2 ? k_gram<2>
+                                                   : s.nt == 3 ? k_gram<3>
+                                                               : k_gram<4>;
+  hipLaunchKernelGGL(fn, dim3(s.blocks * a.nslice), dim3(256), 0, st, a, s.nbe, s.nbe_b, s.blocks,
+                     nlo);
   return hipGetLastError();
 }
 

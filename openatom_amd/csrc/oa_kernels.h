@@ -238,8 +238,8 @@ struct GramArgs {
   double* part;  // [nslice][n][nb]
   int nb;        // rows of B
 };
-// K slices per output block for about `target` workgroups in all
-int gram_slices(int n, int K, int k_lo, int sym, int target);
+// K slices of C[n][nb] for ncu CUs
+int gram_slices(int n, int nb, int K, int sym, int ncu);
 hipError_t gram_f64(const GramArgs& a, hipStream_t st);
 // C = alpha * sum_sp part[sp]; mirrored from the computed tiles if sym
 hipError_t gram_reduce(const double* part, int nslice, int n, int nb, int sym, double alpha,

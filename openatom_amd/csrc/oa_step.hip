@@ -744,10 +744,10 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) !=
           hipSuccess || ncu <= 0)
     ncu = 256;
-  c->nslice_sym = oa::gram_slices(n, K, 2 * c->nkx0, 1, ncu);
+  c->nslice_sym = oa::gram_slices(n, n, K, 1, ncu);
   const bool split_lam = split_on(c, kSplitLambda) && n > oa::kGramSmall;
   c->nslice_full = split_lam ? oa::gram_bf16_slices(n, K, ncu)
-                             : oa::gram_slices(n, K, 2 * c->nkx0, 0, ncu);
+                             : oa::gram_slices(n, n, K, 0, ncu);
   int max_sym = c->nslice_sym, max_full = c->nslice_full;
   if (c->opt.autotune) {
     // K slices: half, the heuristic and twice it (at least 2, at most K/64)
@@ -1920,7 +1920,7 @@ oa_status oa_nonlocal_set(oa_ctx* c, const oa_nonlocal* nl) {
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) !=
             hipSuccess || ncu <= 0)
       ncu = 256;
-    const int ns = oa::gram_slices(std::max(c->nst, 4 * na), 2 * c->npts, 2 * c->nkx0, 0, ncu);
+    const int ns = oa::gram_slices(c->nst, 4 * na, 2 * c->npts, 0, ncu);
     TRY(dalloc(c, &c->nl_sf, (size_t)4 * na * ldr * sizeof(double)));
     TRY(dalloc(c, &c->nl_z, (size_t)c->nst * 4 * na * sizeof(double)));
     TRY(dalloc(c, &c->nl_mt, (size_t)na * c->nst * sizeof(double)));
