@@ -50,11 +50,17 @@ __device__ __forceinline__ void xcd_block(int& bx, int& by) {
 // ------------------------------------------------------------------ z passes
 
 // PR: every stored |kz| <= (N - 1) / 4 (pruned pass 1, Sph in oa_fft2.h)
+// FP32: 512 threads, so that a workgroup's stores to one z are as long as the FP64
+// ones; LD: the lanes across lines meet every bank with an odd stride, one with 128 or
+// 160.  Bound by the scattered runs of zbuf: 512 states of 160^3, 2.7 GB, 970 -> 864 us
+// (940 with the stride alone); 100^3 and 108^3 as before.
+template <typename T>
+constexpr int kZThreads = sizeof(T) == 4 ? 512 : 256;
 template <typename T, int R1, int R2, bool PR>
-__global__ __launch_bounds__(kThreads) void k2_zfwd(FftCtx c) {
+__global__ __launch_bounds__(kZThreads<T>) void k2_zfwd(FftCtx c) {
   using Sh = Shape<R1, R2>;
-  constexpr int N = Sh::N, G = Sh::G, NTR = Sh::NTR;
-  __shared__ cpx<T> ex[NTR * N];
+  constexpr int N = Sh::N, G = Sh::G, NTR = kZThreads<T> / G, LD = N | 1;
+  __shared__ cpx<T> ex[NTR * LD];
   int bx, s;
   xcd_block(bx, s);
   const int l0 = bx * NTR;
@@ -84,7 +90,7 @@ __global__ __launch_bounds__(kThreads) void k2_zfwd(FftCtx c) {
       }
       Dft<T, R1, -1>::run(v);
 #pragma unroll
-      for (int t = 0; t < R1; t++) ex[tr * N + j * R1 + t] = v[t];
+      for (int t = 0; t < R1; t++) ex[tr * LD + j * R1 + t] = v[t];
     }
   }
   __syncthreads();
@@ -93,7 +99,7 @@ __global__ __launch_bounds__(kThreads) void k2_zfwd(FftCtx c) {
     if (tr < nl && j < R1) {
       cpx<T> u[R2];
 #pragma unroll
-      for (int t = 0; t < R2; t++) u[t] = ex[tr * N + j + t * R1];
+      for (int t = 0; t < R2; t++) u[t] = ex[tr * LD + j + t * R1];
 #pragma unroll
       for (int t = 1; t < R2; t++) u[t] = cm(u[t], twiddle<T, -1>(c.twz, t * j));
       Dft<T, R2, -1>::run(u);
@@ -551,16 +557,17 @@ enum Kind { ZFWD = 0, YFWD, XC2R, XR2C, YBWD, ZBWD, XPSIR };
 
 template <typename T, int R1, int R2>
 hipError_t launch(int kind, const FftCtx& c, hipStream_t st) {
+  constexpr int NZ = kZThreads<T> / Shape<R1, R2>::G;
   constexpr int NTR = Shape<R1, R2>::NTR, NX = XRows<T, R1, R2>::NTR;
   const Geom& g = c.g;
   switch (kind) {
     case ZFWD:
       if (c.prune_z)
-        hipLaunchKernelGGL((k2_zfwd<T, R1, R2, true>), dim3((g.nlines + NTR - 1) / NTR, g.nst),
-                           dim3(kThreads), 0, st, c);
+        hipLaunchKernelGGL((k2_zfwd<T, R1, R2, true>), dim3((g.nlines + NZ - 1) / NZ, g.nst),
+                           dim3(kZThreads<T>), 0, st, c);
       else
-        hipLaunchKernelGGL((k2_zfwd<T, R1, R2, false>), dim3((g.nlines + NTR - 1) / NTR, g.nst),
-                           dim3(kThreads), 0, st, c);
+        hipLaunchKernelGGL((k2_zfwd<T, R1, R2, false>), dim3((g.nlines + NZ - 1) / NZ, g.nst),
+                           dim3(kZThreads<T>), 0, st, c);
       break;
     case ZBWD:
       if (c.prune_z)
