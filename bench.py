@@ -710,14 +710,18 @@ def traffic_from_counters(dirs, out_path, precision_of):
 
 def STAGE_OF_KERNEL(name):
     """The bench stage a kernel's bytes belong to (the roofline's names).
-    k3_r2g's eighth template argument is RHO: true in the fixed-V step's
-    R->G pass, which also accumulates the density."""
+    k3_r2g's eighth template argument, and the second after the shape of
+    k4_r2g, is RHO: true in the fixed-V step's R->G pass, which also
+    accumulates the density."""
     if "k2_zfwd" in name:
         return "k_zfwd"
     if "k2_zbwd" in name:
         return "k_zbwd"
-    if "k3_g2r" in name:
+    if "k3_g2r" in name or "k4_g2r" in name:
         return "k_plane_g2r"
+    if "k4_r2g" in name:
+        targs = name[name.index(">, ") + 3:].split(", ")
+        return "k_plane_r2g_rho" if targs[1] == "true" else "k_plane_r2g"
     if "k3_r2g" in name:
         targs = name[name.index("<") + 1:].split(", ")
         return "k_plane_r2g_rho" if targs[7] == "true" else "k_plane_r2g"

@@ -14,10 +14,10 @@
 //             psi += dt/m F (CP_integrate_min_STD, cp_min_std.C:56-86).
 //   ns      : Newton-Schulz iteration for (S/2)^{-1/2}
 //             (Ortho::do_iteration/step_2/step_3/tolerance_check,
-//              ortho.C:862-985; serial twin cp_lowdin.C:180-265): one
-//             cooperative launch that loops on the device with grid
-//             barriers, operand panels staged in LDS; fallback: two launches
-//             per iteration with a device-side early exit.
+//              ortho.C:862-985; serial twin cp_lowdin.C:180-265): plain
+//             launches with a device-side early exit (one workgroup up to 64
+//             states, small tiles above); on request one cooperative launch
+//             that loops on the device with grid barriers.
 //
 // MFMA operand layout (measured on gfx950): lane l supplies A[l%16][l/16]
 // and B[l/16][l%16] and receives D[l/16 + 4v][l%16] in element v.  Within
@@ -46,7 +46,6 @@ __device__ __forceinline__ v4d mfma16(double a, double b, v4d c) {
 __device__ __forceinline__ v4d vzero() { return (v4d){0.0, 0.0, 0.0, 0.0}; }
 
 // ================================================================== gram
-constexpr int kGB = 128;        // rows of a skinny block
 
 __host__ __device__ constexpr int up_i(int idx, int m) {
   int i = 0;
@@ -90,73 +89,6 @@ struct Frag {
   double f[NF][4];
 };
 constexpr int kGramRing = 3;
-
-// Skinny block (nb <= 32 columns, e.g. the non-local projections of one
-// atom set): wave w owns rows [32 w, 32 w + 32) of the 128-row block and
-// both 16-column tiles, so no wave idles on absent columns.
-__device__ __forceinline__ void gram_skinny_wave(const GramArgs& a, const double* __restrict__ B,
-                                                 const GSlice& s, int sp, int bi) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
-  const int rbase = bi * kGB + wave * 32;
-  if (rbase >= a.n) return;
-  int ra[2], rb[2];
-#pragma unroll
-  for (int x = 0; x < 2; x++) {  // rows past the matrices: outputs not stored
-    const int r = rbase + 16 * x + l16, q = 16 * x + l16;
-    ra[x] = r < a.n ? r : 0;
-    rb[x] = q < a.nb ? q : 0;
-  }
-  v4d acc[2][2];
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++) acc[x][y] = vzero();
-  auto mfmas = [&](const double (&f)[4][4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-#pragma unroll
-      for (int x = 0; x < 2; x++)
-#pragma unroll
-        for (int y = 0; y < 2; y++) acc[x][y] = mfma16(f[x][e], f[2 + y][e], acc[x][y]);
-  };
-  Frag<4> ring[kGramRing];  // fragments 0-1: rows of A, 2-3: rows of B
-  chunk_ring(
-      s.c0, s.c1, ring,
-      [&](int c, Frag<4>& d) __attribute__((always_inline)) {
-        const int kk = s.base + 16 * c + 4 * g;
-#pragma unroll
-        for (int x = 0; x < 2; x++) {
-          gfrag(a.A, a.lda, ra[x], kk, d.f[x]);
-          gfrag(B, a.lda, rb[x], kk, d.f[2 + x]);
-        }
-      },
-      [&](int c, const Frag<4>& d) __attribute__((always_inline)) {
-        const int k0 = s.base + 16 * c;
-        if (k0 >= s.rs && k0 + 16 <= s.re) {
-          mfmas(d.f);
-        } else {  // a chunk at the region's edge (padding past K may hold anything)
-          Frag<4> m = d;
-#pragma unroll
-          for (int x = 0; x < 4; x++) gmask(k0 + 4 * g, s.rs, s.re, m.f[x]);
-          mfmas(m.f);
-        }
-      });
-  double* part = a.part + (size_t)sp * a.n * a.nb;
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int r = rbase + 16 * x + g + 4 * v, col = 16 * y + l16;
-        if (r < a.n && col < a.nb) part[(size_t)r * a.nb + col] = s.w * acc[x][y][v];
-      }
-}
-
-// nb <= 32 < n: grid (row blocks, K slices)
-__global__ __launch_bounds__(256) void k_gram_skinny(GramArgs a, int nlo) {
-  gram_skinny_wave(a, a.B, gram_slice(a, blockIdx.y, nlo), blockIdx.y, blockIdx.x);
-}
 
 // Output block of MT x NT tiles from tile (ti0, tj0) (DIAG: the upper ones of a
 // diagonal block of a symmetric product): each wave holds all of it for every fourth
@@ -278,6 +210,16 @@ __global__ __launch_bounds__(256) void k_gram(GramArgs a, int nbe, int nbe_b, in
   gram_block<NT, NT, false>(a, a.sym ? a.A : a.B, s, sp, NT * bi, NT * bj, sm);
 }
 
+// nb <= 32 < n (the non-local projections of few atoms): blocks of 64 rows and all
+// columns, the rest as in k_gram.  128 states x 32 atoms x 65,922 reals 61 -> 32 us;
+// before, a wave of a 128-row block had 32 rows for all of K, and too little in flight.
+template <int NT>
+__global__ __launch_bounds__(256) void k_gram_nb(GramArgs a, int nblk, int nlo) {
+  __shared__ double sm[2][4 * NT * 256];
+  const int sp = blockIdx.x / nblk, b = blockIdx.x - sp * nblk;
+  gram_block<4, NT, false>(a, a.B, gram_slice(a, sp, nlo), sp, 4 * b, 0, sm);
+}
+
 // Tiles per block edge and blocks of the output: a single block up to 64 rows and
 // columns, else blocks of 3 or 4 tiles, whichever computes fewer tiles (9 tiles an
 // edge: 45 instead of 78 for the symmetric product), 4 where they are equal (more
@@ -308,7 +250,7 @@ static GramShape gram_shape(int n, int nb, int sym) {
 static bool gram_skinny(int n, int nb, int sym) { return !sym && nb <= 32 && n > kGramSmall; }
 
 int gram_slices(int n, int nb, int K, int sym, int ncu) {
-  const int blocks = gram_skinny(n, nb, sym) ? (n + kGB - 1) / kGB : gram_shape(n, nb, sym).blocks;
+  const int blocks = gram_skinny(n, nb, sym) ? (n + 63) / 64 : gram_shape(n, nb, sym).blocks;
   // whole rounds of a workgroup per CU, the more the longer (about 200 chunks a wave):
   // then the lighter blocks on the diagonal even out (512 states: 7 slices 1.15 ms, 14
   // 1.07; but 128 states: 64 slices 37 us, 128 47)
@@ -323,8 +265,9 @@ hipError_t gram_f64(const GramArgs& a, hipStream_t st) {
     return hipErrorInvalidValue;
   const int nlo = gram_nlo(a);
   if (gram_skinny(a.n, a.nb, a.sym)) {
-    hipLaunchKernelGGL(k_gram_skinny, dim3((a.n + kGB - 1) / kGB, a.nslice), dim3(256), 0, st, a,
-                       nlo);
+    const int nblk = (a.n + 63) / 64;
+    hipLaunchKernelGGL(a.nb <= 16 ? k_gram_nb<1> : k_gram_nb<2>, dim3(nblk * a.nslice), dim3(256),
+                       0, st, a, nblk, nlo);
     return hipGetLastError();
   }
   const GramShape s = gram_shape(a.n, a.nb, a.sym);
@@ -1912,11 +1855,15 @@ __global__ __launch_bounds__(kNlThreads) void k_nl_tail(NsArgs a, int launched, 
     es = 0.0;
     for (int w = 0; w < kNlThreads / 64; w++) es += part[w];
     const double err = sqrt(es / ((double)a.n * a.n));
-    if (err <= a.tol || it >= a.max_iter) {
+    const bool lost = !(err < __builtin_huge_val());  // S, or a product, not finite
+    if (err <= a.tol || it >= a.max_iter || lost) {
       if (tid == 0) {
         a.res->ns_iter = err <= a.tol ? it : -a.max_iter;
         a.res->ns_err = err;
       }
+      if (lost && it < a.max_iter)  // where the iterations left would have ended
+        for (size_t e = tid; e < (size_t)a.n * a.n; e += kNlThreads)
+          a.Tout[e] = __builtin_nan("");
       return;
     }
     for (int w = 0; w < nwg; w++) nl_tile<R, kNlC>(a, it + 1, w / nt, w % nt, nt, false, nl_smem);

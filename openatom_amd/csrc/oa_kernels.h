@@ -223,7 +223,7 @@ hipError_t vloc_build(const VksArgs& a, const PseudoDev& p, double2* vloc, hipSt
 // ---- dense linear algebra (oa_gemm.hip) ----
 // part[sp][i][j] = sum_{k in slice sp} w(k) A[i][k] B[j][k]; A, B are [n][lda]
 // rows of K reals (lda a multiple of 4, rows 32-byte aligned); w(k) = w_lo
-// for k < k_lo else w_hi.  Every 128 x 128 output block is split into nslice
+// for k < k_lo else w_hi.  Every output block is split into nslice
 // K slices (slices never straddle k_lo).  sym: B == A, only the 16 x 16
 // tiles with i/16 <= j/16 are computed.
 // C[i][j] = sum_k w(k) A[i][k] B[j][k], i < n, j < nb (nb == n when sym)

@@ -59,3 +59,19 @@ def test_iterations_past_the_expected_count(gpu, n):
     assert ok and ok2 and it == it2 and it > 5
     assert np.array_equal(s, s2) and np.array_equal(t, t2)
     assert err < 1e-11
+
+
+@pytest.mark.parametrize("n", [40, 65, 272])
+def test_a_value_that_is_not_finite_is_reported(gpu, n):
+    """Also with more iterations allowed than are launched: no convergence, T lost."""
+    hmat = np.diag([9.0, 9.0, 9.3]).reshape(9)
+    ecut = (2.0 * np.pi * 6.4 / 9.0) ** 2
+    k = _lib.kvecs(ecut, hmat)
+    rng = np.random.default_rng(n)
+    psi = rng.normal(size=(n, len(k[0]))) + 1j * rng.normal(size=(n, len(k[0])))
+    psi[n // 2, 7] = np.nan
+    with CPContext((27, 27, 30), hmat, ecut, n, *k, ns_mode=6) as c:
+        c.set_psi(psi)
+        c.overlap()
+        t, it, err, ok = c.ortho_ns(1e-15, 30)
+    assert not ok and it == 30 and np.isnan(err) and np.isnan(t).all()
