@@ -1673,6 +1673,18 @@ constexpr int kNlThreads = 512;
 constexpr int kNlLaunch = 10;
 enum { kNlC, kNlXT, kNlFirst };
 
+// What the launches of one run tell each other, in the unused error partials of
+// iteration 0.  The workgroups of a launch start at different times, so a launch
+// reads only what earlier launches wrote: the C launches read res->ns_iter and write
+// this, the others read this and write res->ns_iter.
+struct NlRun {
+  int conv;    // the iteration that met the tolerance, 0: none yet
+  double err;  // its change of T
+};
+__device__ __forceinline__ NlRun* nl_run(const NsArgs& a) {
+  return reinterpret_cast<NlRun*>(a.errpart);
+}
+
 struct NlBuf {
   const double *To, *Xo;
   double *Tw, *Xw;
@@ -1748,10 +1760,19 @@ __device__ __forceinline__ void nl_tile(const NsArgs& a, int it, int ti, int tj,
   const int n = a.n, nwg = nt * nt, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const NlBuf q = nl_buf(a, it);
   const int m = tid / TP;  // which product's elements this thread finishes
-  int done = 0;
   double es = 0.0;
-  if (MODE != kNlFirst && check) done = *(const volatile int*)&a.res->ns_iter;
-  if (done != 0) return;  // one more wait, but idle launches take 1.2 us
+  // the same in every workgroup (NlRun); one more wait, but idle launches take 1.2 us
+  if (MODE == kNlC && check && a.res->ns_iter != 0) return;
+  if (MODE == kNlXT && check) {
+    const NlRun r = *nl_run(a);
+    if (r.conv != 0) {
+      if (ti == 0 && tj == 0 && tid == 0) {
+        a.res->ns_iter = r.conv;
+        a.res->ns_err = r.err;
+      }
+      return;
+    }
+  }
   if (MODE == kNlC && check)
     for (int i = tid; i < nwg; i += kNlThreads) es += a.errpart[(size_t)(it - 1) * nwg + i];
   int row[NE], col[NE];
@@ -1781,10 +1802,7 @@ __device__ __forceinline__ void nl_tile(const NsArgs& a, int it, int ti, int tj,
     for (int w = 0; w < 8; w++) s += red[w];
     const double err = sqrt(s / ((double)n * n));
     if (err <= a.tol) {
-      if (ti == 0 && tj == 0 && tid == 0) {
-        a.res->ns_iter = it - 1;
-        a.res->ns_err = err;
-      }
+      if (ti == 0 && tj == 0 && tid == 0) *nl_run(a) = {it - 1, err};
       return;
     }
   }
@@ -1826,6 +1844,7 @@ __device__ __forceinline__ void nl_tile(const NsArgs& a, int it, int ti, int tj,
     if (MODE == kNlFirst && ti == 0 && tj == 0 && tid == 0) {
       a.res->ns_iter = 0;
       a.res->ns_err = 0.0;
+      *nl_run(a) = {0, 0.0};
     }
   }
   if (!check) __syncthreads();
@@ -1844,7 +1863,7 @@ __global__ __launch_bounds__(kNlThreads) void k_nl_tail(NsArgs a, int launched, 
   extern __shared__ __align__(16) double nl_smem[];
   __shared__ double part[kNlThreads / 64];
   const int nwg = nt * nt, tid = threadIdx.x;
-  if (*(const volatile int*)&a.res->ns_iter != 0) return;  // the same in every thread
+  if (nl_run(a)->conv != 0) return;  // recorded by the last launch
   for (int it = launched;; it++) {
     double es = 0.0;
     for (int i = tid; i < nwg; i += kNlThreads) es += a.errpart[(size_t)it * nwg + i];
