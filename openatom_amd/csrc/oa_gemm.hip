@@ -980,8 +980,9 @@ __global__ __launch_bounds__(256) void k_ns_coop(NsArgs a) {
 
 // One workgroup for the whole iteration, a plain launch (n <= kNsOneMax): X, T
 // and C stay in LDS (zero past n, odd row stride), a wave computes 16 x 16 tiles;
-// the new X = C X / 2 and T = C T / 2 (X, T and C commute, so C X = X C up to
-// rounding) wait in registers until every wave has read the old ones.  Bound by
+// the new X = X C / 2 and T = C T / 2 wait in registers until every wave has read the
+// old ones.  (C X / 2 is the same matrix, but with C = 3I - T X an error of X then
+// grows by up to half the square root of S's eigenvalue ratio in every iteration.)  Bound by
 // the matrix pipe of one CU at n = 64 and by the dependent products and three
 // barriers per iteration below; no operand leaves the CU.  The stage of a step
 // (4 to 5 iterations) takes 15 us at 16 states, and 64 states 37; the cooperative
@@ -1035,8 +1036,7 @@ __global__ __launch_bounds__(1024) void k_ns_one(NsArgs a) {
       const int q = wave + i * nw, t = q < nt * nt ? q : q - nt * nt;
       if (q >= 2 * nt * nt) continue;
       const int ti = t / nt, tj = t - ti * nt;
-      const double* D = q < nt * nt ? X : T;
-      p[i] = product(C, D, ti, tj) * 0.5;
+      p[i] = (q < nt * nt ? product(X, C, ti, tj) : product(C, T, ti, tj)) * 0.5;
       if (q >= nt * nt)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
@@ -1654,7 +1654,7 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
 //
 // A launch boundary takes the place of the grid barrier: about 3 us against 30 us
 // for entering a cooperative launch and 8 us per barrier.  C = 3I - T X in one
-// launch, X' = C X / 2 and T' = C T / 2 in the next; a workgroup computes one
+// launch, X' = X C / 2 and T' = C T / 2 in the next; a workgroup computes one
 // tile of 16 R rows and columns, its eight waves sharing the sum over k (four to
 // a product where there are two), all loads of a wave in flight at once: these
 // products are bound by the latency of reading what the last launch wrote
@@ -1791,7 +1791,8 @@ __device__ __forceinline__ void nl_tile(const NsArgs& a, int it, int ti, int tj,
   else if constexpr (MODE == kNlC)
     nl_product<R, false>(q.To, q.Xo, n, ti, tj, wave, KS, part + wave * E);
   else
-    nl_product<R, false>(a.C, wave < KS ? q.Xo : q.To, n, ti, tj, wave % KS, KS, part + wave * E);
+    nl_product<R, false>(wave < KS ? q.Xo : a.C, wave < KS ? a.C : q.To, n, ti, tj, wave % KS, KS,
+                         part + wave * E);
   if (MODE == kNlC && check) {
     for (int off = 32; off > 0; off >>= 1) es += __shfl_down(es, off, 64);
     if (lane == 0) red[wave] = es;
