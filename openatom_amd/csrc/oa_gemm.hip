@@ -1416,15 +1416,16 @@ hipError_t ns_run_mixed(const NsArgs& a, const Ns32Bufs& b, hipStream_t st) {
 // ---- block-row variant: one grid barrier per iteration
 //
 // Workgroup (b, h) owns rows R = [16b, 16b + 16) and the 16-column tiles
-// ct = h, h + split, h + 2 split, ... of X and T (split = gridDim.y).  X, T
-// and C are polynomials in S and commute, so the new X = X C / 2 of the
-// recurrence equals C X / 2 (up to rounding), and the new tiles
-//   X'[R,ct] = C[R,:] X[:,ct] / 2,  T'[R,ct] = C[R,:] T[:,ct] / 2
-// need only C[R,:] = 3I - T[R,:] X, which every workgroup of the row block
-// computes whole, and the previous X and T.  C[R,:] and T[R,:] sit in LDS;
+// ct = h, h + split, h + 2 split, ... of X and T (split = gridDim.y).  With
+// C = 3I - T X the new X = X C / 2 of the recurrence is D X / 2, D = 3I - X T,
+// and the new tiles
+//   T'[R,ct] = C[R,:] T[:,ct] / 2,  X'[R,ct] = D[R,:] X[:,ct] / 2
+// need only rows of C and D, which every workgroup of the row block computes
+// whole, one after the other in the same LDS rows, and the previous X and T.
+// (C X / 2, which would need no D, multiplies rounding errors: see k_ns_one.)
 // X and T go through global memory (double buffered) for the other
 // workgroups.  Iteration 1 starts from T0 = I and X0 = S/2 (ortho.C:236-239):
-// there C = 3I - S/2 and T1 = C/2 need no products, so no barrier precedes
+// there C = D = 3I - S/2 and T1 = C/2 need no products, so no barrier precedes
 // it.  After each barrier the next iteration's operands are loaded before
 // the convergence test reads the error partials, so the two latencies
 // overlap.  MFMA operands: A from LDS, B from global memory in batches of KB
@@ -1514,12 +1515,11 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
   const int wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int pr = tid >> 5, pk = tid & 31;  // A panel staging: row, first column
   constexpr int nthr = kNrWaves * 64;
-  double bc[KB], bx[KB], ap[4];
+  double bc[KB], bx[KB], ap[2][4];  // ap: rows R of T and X, columns pk + 32 q
   {
     const int n = a.n, ld = nr_ld(n);
-    double* Tr = nr_smem;  // [16][ld]: rows R of T (previous iteration, then own tiles new)
-    double* Cr = Tr + 16 * ld;  // [16][ld]: rows R of C
-    nr_load<KB>(bx, nr_rsrc(a.S, n), (h + split * (wave >> 1)) * 16 + l16, n, 0, 0.5);  // X0 = S/2
+    double* Tr = nr_smem;       // [16][ld]: rows R of the previous T, then of X
+    double* Cr = Tr + 16 * ld;  // [16][ld]: rows R of C, then of D
     // iteration 1: T0 = I, C = 3I - S/2; LDS zero past n in both directions
     for (int e = tid; e < 16 * ld; e += nthr) {
       const int r = e / ld, k = e - r * ld, row = r0 + r;
@@ -1541,26 +1541,24 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
     double* Tr = nr_smem;
     double* Cr = Tr + 16 * ld;
     // X_k and T_k live in buffer k & 1
-    const double* To = (it & 1) ? a.T0 : a.T1;
+    const double *To = (it & 1) ? a.T0 : a.T1, *Xo = (it & 1) ? a.X0 : a.X1;
     double* Xw = (it & 1) ? a.X1 : a.X0;
     double* Tw = (it & 1) ? a.T1 : a.T0;
-    const rsrc_t rXo = nr_rsrc((it & 1) ? a.X0 : a.X1, n), rTo = nr_rsrc(To, n);
-    if (it > 1) {
-      if (split > 1) {  // rows R of T_{it-1}: the other tiles come from other workgroups
-        const bool rin = r0 + pr < n;
+    const rsrc_t rXo = nr_rsrc(Xo, n), rTo = nr_rsrc(To, n);
+    // Cr = 3I - (rows R of P) Q; the first batch of Q is in bc where `ready`
+    auto rows = [&](const double* P, const double (&pre)[4], rsrc_t Q, bool ready) {
+      const bool rin = r0 + pr < n;
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (rin && pk + 32 * q < n) Tr[pr * ld + pk + 32 * q] = ap[q];
-        for (int k = pk + 128; k < n; k += 32)
-          if (rin) Tr[pr * ld + k] = To[(size_t)(r0 + pr) * n + k];
-      }
+      for (int q = 0; q < 4; q++)
+        if (rin && pk + 32 * q < n) Tr[pr * ld + pk + 32 * q] = pre[q];
+      for (int k = pk + 128; k < n; k += 32)
+        if (rin) Tr[pr * ld + k] = P[(size_t)(r0 + pr) * n + k];
       __syncthreads();
-      // C[R,:] = 3I - T[R,:] X
 #pragma nounroll
       for (int ct = wave, i = 0; ct < nct; ct += kNrWaves, i++) {
         const int col = ct * 16 + l16;
-        if (i > 0) nr_load<KB>(bc, rXo, col, n, 0, 1.0);
-        const v4d acc = nr_product<KB>(Tr, ld, bc, rXo, col, n, 1.0);
+        if (i > 0 || !ready) nr_load<KB>(bc, Q, col, n, 0, 1.0);
+        const v4d acc = nr_product<KB>(Tr, ld, bc, Q, col, n, 1.0);
 #pragma unroll
         for (int v = 0; v < 4; v++) {
           const int r = g + 4 * v, row = r0 + r;
@@ -1568,36 +1566,47 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
         }
       }
       __syncthreads();
-    }
-    // own tiles: X'[R,ct] = C[R,:] X[:,ct] / 2, T'[R,ct] = C[R,:] T[:,ct] / 2,
-    // and the change of T
+    };
+    if (it > 1) rows(To, ap[0], rXo, true);
+    // own tiles of T' = C T / 2, and the change of T
     double e = 0.0;
 #pragma nounroll
-    for (int q = wave, i = 0; q < 2 * nown; q += kNrWaves, i++) {
-      const int m = q & 1, col = (h + split * (q >> 1)) * 16 + l16;
+    for (int q = wave, i = 0; q < nown; q += kNrWaves, i++) {
+      const int col = (h + split * q) * 16 + l16;
       v4d acc;
-      if (it == 1 && m) {  // T0 = I: C T0 = C
+      if (it == 1) {  // T0 = I: C T0 = C
 #pragma unroll
         for (int v = 0; v < 4; v++) acc[v] = Cr[(g + 4 * v) * ld + min(col, ld - 1)];
       } else {
-        const rsrc_t B = it == 1 ? nr_rsrc(a.S, n) : (m ? rTo : rXo);
-        const double scale = it == 1 ? 0.5 : 1.0;
-        if (i > 0) nr_load<KB>(bx, B, col, n, 0, scale);
-        acc = nr_product<KB>(Cr, ld, bx, B, col, n, scale);
+        if (i > 0) nr_load<KB>(bx, rTo, col, n, 0, 1.0);
+        acc = nr_product<KB>(Cr, ld, bx, rTo, col, n, 1.0);
       }
-      double* D = m ? Tw : Xw;
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int r = g + 4 * v, row = r0 + r;
         if (row < n && col < n) {
-          const double nv = 0.5 * acc[v];
-          D[(unsigned)(row * n + col)] = nv;
-          if (m) {
-            const double d = Tr[r * ld + col] - nv;
-            e += d * d;
-            Tr[r * ld + col] = nv;  // this thread's element only: read before written
-          }
+          const double nv = 0.5 * acc[v], d = Tr[r * ld + col] - nv;
+          Tw[(unsigned)(row * n + col)] = nv;
+          e += d * d;
         }
+      }
+    }
+    if (it > 1) {
+      __syncthreads();  // every wave has read the rows of C and T
+      rows(Xo, ap[1], rTo, false);
+    }
+    // own tiles of X' = D X / 2
+#pragma nounroll
+    for (int q = wave; q < nown; q += kNrWaves) {
+      const int col = (h + split * q) * 16 + l16;
+      const rsrc_t B = it == 1 ? nr_rsrc(a.S, n) : rXo;
+      const double scale = it == 1 ? 0.5 : 1.0;  // X0 = S/2
+      nr_load<KB>(bx, B, col, n, 0, scale);
+      const v4d acc = nr_product<KB>(Cr, ld, bx, B, col, n, scale);
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int row = r0 + g + 4 * v;
+        if (row < n && col < n) Xw[(unsigned)(row * n + col)] = 0.5 * acc[v];
       }
     }
     {  // workgroup sum in a fixed order
@@ -1613,15 +1622,14 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
     grid.sync();
     // the next iteration's first operands, then the error partials
     if (it < a.max_iter) {
-      if (split > 1) {
-        const double* p = Tw + (size_t)min(r0 + pr, n - 1) * n;
+      const size_t row = (size_t)min(r0 + pr, n - 1) * n;
 #pragma unroll
-        for (int q = 0; q < 4; q++) ap[q] = p[min(pk + 32 * q, n - 1)];
+      for (int q = 0; q < 4; q++) {
+        ap[0][q] = Tw[row + min(pk + 32 * q, n - 1)];
+        ap[1][q] = Xw[row + min(pk + 32 * q, n - 1)];
       }
-      const rsrc_t rXw = nr_rsrc(Xw, n);
-      nr_load<KB>(bc, rXw, wave * 16 + l16, n, 0, 1.0);
-      nr_load<KB>(bx, (wave & 1) ? nr_rsrc(Tw, n) : rXw, (h + split * (wave >> 1)) * 16 + l16, n,
-                  0, 1.0);
+      nr_load<KB>(bc, nr_rsrc(Xw, n), wave * 16 + l16, n, 0, 1.0);
+      nr_load<KB>(bx, nr_rsrc(Tw, n), (h + split * wave) * 16 + l16, n, 0, 1.0);
     }
     for (int i = tid; i < nwg; i += nthr) epart[i] = a.errpart[(size_t)it * nwg + i];
     __syncthreads();
@@ -1641,12 +1649,13 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
     a.res->ns_iter = conv ? conv : -a.max_iter;
     a.res->ns_err = err;
   }
-  // T of the last iteration: this workgroup's tiles are in its LDS rows
-  const int n = a.n, ld = nr_ld(n), nct = (n + 15) >> 4, nown = (nct - h + split - 1) / split;
+  // this workgroup's tiles of the last iteration's T
+  const double* Tl = ((conv ? conv : a.max_iter) & 1) ? a.T1 : a.T0;
+  const int n = a.n, nct = (n + 15) >> 4, nown = (nct - h + split - 1) / split;
   for (int e = tid; e < 16 * nown * 16; e += nthr) {
     const int r = e / (16 * nown), t = e - r * 16 * nown;
     const int row = r0 + r, col = (h + split * (t >> 4)) * 16 + (t & 15);
-    if (row < n && col < n) a.Tout[(size_t)row * n + col] = nr_smem[r * ld + col];
+    if (row < n && col < n) a.Tout[(size_t)row * n + col] = Tl[(size_t)row * n + col];
   }
 }
 
