@@ -1515,7 +1515,7 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
   const int wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int pr = tid >> 5, pk = tid & 31;  // A panel staging: row, first column
   constexpr int nthr = kNrWaves * 64;
-  double bc[KB], bx[KB], ap[2][4];  // ap: rows R of T and X, columns pk + 32 q
+  double bc[KB], bx[KB], ap[4];  // ap: rows R of T, columns pk + 32 q
   {
     const int n = a.n, ld = nr_ld(n);
     double* Tr = nr_smem;       // [16][ld]: rows R of the previous T, then of X
@@ -1544,69 +1544,62 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
     const double *To = (it & 1) ? a.T0 : a.T1, *Xo = (it & 1) ? a.X0 : a.X1;
     double* Xw = (it & 1) ? a.X1 : a.X0;
     double* Tw = (it & 1) ? a.T1 : a.T0;
-    const rsrc_t rXo = nr_rsrc(Xo, n), rTo = nr_rsrc(To, n);
-    // Cr = 3I - (rows R of P) Q; the first batch of Q is in bc where `ready`
-    auto rows = [&](const double* P, const double (&pre)[4], rsrc_t Q, bool ready) {
-      const bool rin = r0 + pr < n;
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (rin && pk + 32 * q < n) Tr[pr * ld + pk + 32 * q] = pre[q];
-      for (int k = pk + 128; k < n; k += 32)
-        if (rin) Tr[pr * ld + k] = P[(size_t)(r0 + pr) * n + k];
-      __syncthreads();
+    double e = 0.0;
+    // m = 0: C = 3I - T X and the own tiles of T' = C T / 2, m = 1: D = 3I - X T and
+    // X' = D X / 2
 #pragma nounroll
-      for (int ct = wave, i = 0; ct < nct; ct += kNrWaves, i++) {
-        const int col = ct * 16 + l16;
-        if (i > 0 || !ready) nr_load<KB>(bc, Q, col, n, 0, 1.0);
-        const v4d acc = nr_product<KB>(Tr, ld, bc, Q, col, n, 1.0);
+    for (int m = 0; m < 2; m++) {
+      const rsrc_t rO = nr_rsrc(m ? Xo : To, n);
+      if (it > 1) {
+        if (m) __syncthreads();  // every wave has read the rows of C and T
+        const bool rin = r0 + pr < n;
+        const double* P = (m ? Xo : To) + (size_t)min(r0 + pr, n - 1) * n;
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          if (rin && pk + 32 * q < n) Tr[pr * ld + pk + 32 * q] = m ? P[pk + 32 * q] : ap[q];
+        for (int k = pk + 128; k < n; k += 32)
+          if (rin) Tr[pr * ld + k] = P[k];
+        __syncthreads();
+        const rsrc_t rQ = nr_rsrc(m ? To : Xo, n);
+#pragma nounroll
+        for (int ct = wave, i = 0; ct < nct; ct += kNrWaves, i++) {
+          const int col = ct * 16 + l16;
+          if (i > 0 || m) nr_load<KB>(bc, rQ, col, n, 0, 1.0);
+          const v4d acc = nr_product<KB>(Tr, ld, bc, rQ, col, n, 1.0);
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            const int r = g + 4 * v, row = r0 + r;
+            if (col < n) Cr[r * ld + col] = (row < n ? (row == col ? 3.0 : 0.0) - acc[v] : 0.0);
+          }
+        }
+        __syncthreads();
+      }
+#pragma nounroll
+      for (int q = wave, i = 0; q < nown; q += kNrWaves, i++) {
+        const int col = (h + split * q) * 16 + l16;
+        v4d acc;
+        if (it == 1 && m == 0) {  // T0 = I: C T0 = C
+#pragma unroll
+          for (int v = 0; v < 4; v++) acc[v] = Cr[(g + 4 * v) * ld + min(col, ld - 1)];
+        } else {
+          const rsrc_t B = it == 1 ? nr_rsrc(a.S, n) : rO;  // X0 = S/2
+          const double scale = it == 1 ? 0.5 : 1.0;
+          if (i > 0 || m) nr_load<KB>(bx, B, col, n, 0, scale);
+          acc = nr_product<KB>(Cr, ld, bx, B, col, n, scale);
+        }
+        double* D = m ? Xw : Tw;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
           const int r = g + 4 * v, row = r0 + r;
-          if (col < n) Cr[r * ld + col] = (row < n ? (row == col ? 3.0 : 0.0) - acc[v] : 0.0);
+          if (row < n && col < n) {
+            const double nv = 0.5 * acc[v];
+            D[(unsigned)(row * n + col)] = nv;
+            if (m == 0) {  // Tr holds the previous T
+              const double d = Tr[r * ld + col] - nv;
+              e += d * d;
+            }
+          }
         }
-      }
-      __syncthreads();
-    };
-    if (it > 1) rows(To, ap[0], rXo, true);
-    // own tiles of T' = C T / 2, and the change of T
-    double e = 0.0;
-#pragma nounroll
-    for (int q = wave, i = 0; q < nown; q += kNrWaves, i++) {
-      const int col = (h + split * q) * 16 + l16;
-      v4d acc;
-      if (it == 1) {  // T0 = I: C T0 = C
-#pragma unroll
-        for (int v = 0; v < 4; v++) acc[v] = Cr[(g + 4 * v) * ld + min(col, ld - 1)];
-      } else {
-        if (i > 0) nr_load<KB>(bx, rTo, col, n, 0, 1.0);
-        acc = nr_product<KB>(Cr, ld, bx, rTo, col, n, 1.0);
-      }
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int r = g + 4 * v, row = r0 + r;
-        if (row < n && col < n) {
-          const double nv = 0.5 * acc[v], d = Tr[r * ld + col] - nv;
-          Tw[(unsigned)(row * n + col)] = nv;
-          e += d * d;
-        }
-      }
-    }
-    if (it > 1) {
-      __syncthreads();  // every wave has read the rows of C and T
-      rows(Xo, ap[1], rTo, false);
-    }
-    // own tiles of X' = D X / 2
-#pragma nounroll
-    for (int q = wave; q < nown; q += kNrWaves) {
-      const int col = (h + split * q) * 16 + l16;
-      const rsrc_t B = it == 1 ? nr_rsrc(a.S, n) : rXo;
-      const double scale = it == 1 ? 0.5 : 1.0;  // X0 = S/2
-      nr_load<KB>(bx, B, col, n, 0, scale);
-      const v4d acc = nr_product<KB>(Cr, ld, bx, B, col, n, scale);
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int row = r0 + g + 4 * v;
-        if (row < n && col < n) Xw[(unsigned)(row * n + col)] = 0.5 * acc[v];
       }
     }
     {  // workgroup sum in a fixed order
@@ -1622,12 +1615,9 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
     grid.sync();
     // the next iteration's first operands, then the error partials
     if (it < a.max_iter) {
-      const size_t row = (size_t)min(r0 + pr, n - 1) * n;
+      const double* p = Tw + (size_t)min(r0 + pr, n - 1) * n;
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        ap[0][q] = Tw[row + min(pk + 32 * q, n - 1)];
-        ap[1][q] = Xw[row + min(pk + 32 * q, n - 1)];
-      }
+      for (int q = 0; q < 4; q++) ap[q] = p[min(pk + 32 * q, n - 1)];
       nr_load<KB>(bc, nr_rsrc(Xw, n), wave * 16 + l16, n, 0, 1.0);
       nr_load<KB>(bx, nr_rsrc(Tw, n), (h + split * wave) * 16 + l16, n, 0, 1.0);
     }
@@ -1766,7 +1756,8 @@ __device__ __forceinline__ void nl_tile(const NsArgs& a, int it, int ti, int tj,
   __shared__ double red[8];
   constexpr int NP = MODE == kNlXT ? 2 : 1, KS = 8 / NP, E = 256 * R * R, TP = kNlThreads / NP;
   constexpr int NE = (E + TP - 1) / TP;
-  const int n = a.n, nwg = nt * nt, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int n = a.n, nwg = nt * nt, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: so are its matrices
   const NlBuf q = nl_buf(a, it);
   const int m = tid / TP;  // which product's elements this thread finishes
   double es = 0.0;
