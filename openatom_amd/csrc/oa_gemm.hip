@@ -1662,7 +1662,7 @@ __global__ __launch_bounds__(kNrWaves * 64) void k_ns_rows(NsArgs a) {
 // iteration's partials, summed in the same order by every workgroup) overlaps
 // the product, and only the stores depend on it.  Iterations after convergence
 // return at once; where the last call's count is known one more than that is
-// launched, and k_nl_tail, one workgroup, runs any others by the same code in the
+// launched, and k_nl_tail runs any others by the same code in the
 // same order, so the result does not depend on how many were launched.  T goes to
 // Tout in every iteration.  The stage takes 70 us at 84, 128 and 180 states, 95 at
 // 256 and 174 at 512 (4 to 6 iterations); the cooperative forms took 103, 91, 186,
@@ -1677,8 +1677,9 @@ enum { kNlC, kNlXT, kNlFirst };
 // reads only what earlier launches wrote: the C launches read res->ns_iter and write
 // this, the others read this and write res->ns_iter.
 struct NlRun {
-  int conv;    // the iteration that met the tolerance, 0: none yet
-  double err;  // its change of T
+  int conv;             // the iteration that met the tolerance, 0: none yet
+  double err;           // its change of T
+  unsigned next, done;  // k_nl_tail: tiles handed out, tiles finished
 };
 __device__ __forceinline__ NlRun* nl_run(const NsArgs& a) {
   return reinterpret_cast<NlRun*>(a.errpart);
@@ -1803,7 +1804,7 @@ __device__ __forceinline__ void nl_tile(const NsArgs& a, int it, int ti, int tj,
     for (int w = 0; w < 8; w++) s += red[w];
     const double err = sqrt(s / ((double)n * n));
     if (err <= a.tol) {
-      if (ti == 0 && tj == 0 && tid == 0) *nl_run(a) = {it - 1, err};
+      if (ti == 0 && tj == 0 && tid == 0) *nl_run(a) = {it - 1, err, 0, 0};
       return;
     }
   }
@@ -1845,7 +1846,7 @@ __device__ __forceinline__ void nl_tile(const NsArgs& a, int it, int ti, int tj,
     if (MODE == kNlFirst && ti == 0 && tj == 0 && tid == 0) {
       a.res->ns_iter = 0;
       a.res->ns_err = 0.0;
-      *nl_run(a) = {0, 0.0};
+      *nl_run(a) = {0, 0.0, 0, 0};
     }
   }
   if (!check) __syncthreads();
@@ -1858,25 +1859,36 @@ __global__ __launch_bounds__(kNlThreads) void k_nl(NsArgs a, int it) {
 }
 
 // After `launched` iterations: records convergence of the last one, or runs the
-// rest, up to max_iter, in one workgroup
+// rest, up to max_iter.  The tiles of all C and X', T' phases are handed out in order;
+// a workgroup waits for the phases before its tile's.  Those tiles have all been taken
+// by workgroups that run, so every wait ends however few of them are resident: this
+// needs no cooperative launch, and where nothing is left to do all return at once.  At
+// most as many workgroups as tiles: each takes one tile of the phase that finds the
+// end, none of a later one.  An iteration of 512 states takes 75 us here (35 launched
+// by itself; 8 ms in the one workgroup that this kernel once was).
+constexpr int kNlSpin = 1 << 22;  // polls of a wait: seconds, where a tile takes microseconds
 template <int R>
 __global__ __launch_bounds__(kNlThreads) void k_nl_tail(NsArgs a, int launched, int nt) {
   extern __shared__ __align__(16) double nl_smem[];
   __shared__ double part[kNlThreads / 64];
+  __shared__ int ticket;  // -1: the wait did not end
   const int nwg = nt * nt, tid = threadIdx.x;
-  if (nl_run(a)->conv != 0) return;  // recorded by the last launch
-  for (int it = launched;; it++) {
+  NlRun* run = nl_run(a);
+  if (run->conv != 0) return;  // recorded by the last launch
+  // the same in every workgroup: true at the end of the iteration, recorded by one
+  auto ended = [&](int it, bool record) {
     double es = 0.0;
     for (int i = tid; i < nwg; i += kNlThreads) es += a.errpart[(size_t)it * nwg + i];
     for (int off = 32; off > 0; off >>= 1) es += __shfl_down(es, off, 64);
-    __syncthreads();
     if ((tid & 63) == 0) part[tid >> 6] = es;
     __syncthreads();
     es = 0.0;
     for (int w = 0; w < kNlThreads / 64; w++) es += part[w];
+    __syncthreads();
     const double err = sqrt(es / ((double)a.n * a.n));
     const bool lost = !(err < __builtin_huge_val());  // S, or a product, not finite
-    if (err <= a.tol || it >= a.max_iter || lost) {
+    if (!(err <= a.tol || it >= a.max_iter || lost)) return false;
+    if (record) {
       if (tid == 0) {
         a.res->ns_iter = err <= a.tol ? it : -a.max_iter;
         a.res->ns_err = err;
@@ -1884,14 +1896,45 @@ __global__ __launch_bounds__(kNlThreads) void k_nl_tail(NsArgs a, int launched, 
       if (lost && it < a.max_iter)  // where the iterations left would have ended
         for (size_t e = tid; e < (size_t)a.n * a.n; e += kNlThreads)
           a.Tout[e] = __builtin_nan("");
+    }
+    return true;
+  };
+  if (ended(launched, blockIdx.x == 0)) return;
+  // Thread 0 finishes a tile and takes the next one in one place, and the ways through
+  // the loop meet at a barrier before it: with a branch for thread 0 at the end too the
+  // compiler made loops of their own for it and for the other lanes of its wave.
+  const int rounds = 2 * nwg * (a.max_iter - launched) + 1;  // all tickets, and the end
+  for (int round = 0; round < rounds; round++) {
+    if (tid == 0) {
+      if (round > 0) {  // nl_tile has ended with a barrier: every store of the tile is done
+        __threadfence();
+        __hip_atomic_fetch_add(&run->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      const unsigned t =
+          __hip_atomic_fetch_add(&run->next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned before = t / nwg * nwg;  // tiles of the earlier phases
+      int left = kNlSpin;
+      while (__hip_atomic_load(&run->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < before &&
+             --left > 0)
+        __builtin_amdgcn_s_sleep(8);
+      __threadfence();
+      ticket = left > 0 ? (int)t : -1;
+    }
+    __syncthreads();
+    const int t = __builtin_amdgcn_readfirstlane(ticket), phase = t / nwg, w = t - phase * nwg, it = launched + 1 + phase / 2;
+    if (t < 0) {
+      if (tid == 0) {
+        a.res->ns_iter = -a.max_iter;
+        a.res->ns_err = __builtin_nan("");
+      }
       return;
     }
-    for (int w = 0; w < nwg; w++) nl_tile<R, kNlC>(a, it + 1, w / nt, w % nt, nt, false, nl_smem);
-    __threadfence();
-    __syncthreads();
-    for (int w = 0; w < nwg; w++) nl_tile<R, kNlXT>(a, it + 1, w / nt, w % nt, nt, false, nl_smem);
-    __threadfence();
-    __syncthreads();
+    if (phase & 1) {
+      nl_tile<R, kNlXT>(a, it, w / nt, w % nt, nt, false, nl_smem);
+    } else {
+      if (phase > 0 && ended(it - 1, w == 0)) return;
+      nl_tile<R, kNlC>(a, it, w / nt, w % nt, nt, false, nl_smem);
+    }
   }
 }
 
@@ -1909,7 +1952,7 @@ static hipError_t ns_steps_r(const NsArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((k_nl<R, kNlC>), grid, thr, sm, st, a, it);
     hipLaunchKernelGGL((k_nl<R, kNlXT>), grid, thr, sm, st, a, it);
   }
-  hipLaunchKernelGGL(k_nl_tail<R>, dim3(1), thr, sm, st, a, count, nt);
+  hipLaunchKernelGGL(k_nl_tail<R>, dim3(std::min(nt * nt, cu_count())), thr, sm, st, a, count, nt);
   return hipGetLastError();
 }
 static hipError_t ns_run_steps(const NsArgs& a, hipStream_t st) {
