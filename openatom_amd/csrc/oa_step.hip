@@ -163,7 +163,8 @@ struct oa_ctx {
   double* eke_part = nullptr;
   int nblk = 0;
   double *S = nullptr, *T = nullptr, *lam = nullptr, *gpart = nullptr, *S2 = nullptr;
-  int nslice_sym = 0, nslice_full = 0;  // gram K slices (symmetric S, full Lambda)
+  // gram K slices: symmetric FP64 products (S, residual), S as a split product, Lambda
+  int nslice_sym = 0, nslice_split = 0, nslice_full = 0;
   double *nsX0 = nullptr, *nsX1 = nullptr, *nsT0 = nullptr, *nsT1 = nullptr, *nsC = nullptr,
          *errpart = nullptr;
   oa::Ns32Bufs ns32{};  // FP32 Newton-Schulz work space (mixed contexts with ns_fp32)
@@ -213,7 +214,7 @@ struct oa_ctx {
   double2* vloc = nullptr;
   // autotuner (opt.autotune): candidate launch shapes (buffers are sized for
   // the largest) and what was measured
-  std::vector<int> tune_nchunk, tune_nchunk_r, tune_nslice_sym, tune_nslice_full;
+  std::vector<int> tune_nchunk, tune_nchunk_r, tune_nslice_sym, tune_nslice_full;  // sym: of S
   std::vector<int> tune_vks[3];  // V_KS rows, columns, lines per workgroup
   std::string tune_log;
   // non-local KB pseudopotential (oa_nonlocal_set): projector table, the
@@ -748,7 +749,9 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
   const bool split_lam = split_on(c, kSplitLambda) && n > oa::kGramSmall;
   c->nslice_full = split_lam ? oa::gram_bf16_slices(n, K, ncu)
                              : oa::gram_slices(n, n, K, 0, ncu);
-  int max_sym = c->nslice_sym, max_full = c->nslice_full;
+  const bool split_s = split_on(c, kSplitS) && n > oa::kGramSmall;
+  if (split_s) c->nslice_split = oa::gram_bf16_slices(n, K, ncu);
+  int max_sym = c->nslice_sym, max_split = c->nslice_split, max_full = c->nslice_full;
   if (c->opt.autotune) {
     // K slices: half, the heuristic and twice it (at least 2, at most K/64)
     auto cands = [&](int h) {
@@ -758,15 +761,16 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
       if (v.empty()) v.push_back(h);
       return v;
     };
-    c->tune_nslice_sym = cands(c->nslice_sym);
+    c->tune_nslice_sym = cands(split_s ? c->nslice_split : c->nslice_sym);
     c->tune_nslice_full = cands(c->nslice_full);
-    max_sym = std::max(max_sym, c->tune_nslice_sym.back());
+    int& max_s = split_s ? max_split : max_sym;
+    max_s = std::max(max_s, c->tune_nslice_sym.back());
     max_full = std::max(max_full, c->tune_nslice_full.back());
   }
-  // the split product's partials are FP32
+  // the split products' partials are FP32
   TRY(dalloc(c, &c->gpart,
-             nn * std::max(max_sym * sizeof(double),
-                           max_full * (split_lam ? sizeof(float) : sizeof(double)))));
+             nn * std::max({max_sym * sizeof(double), max_split * sizeof(float),
+                            max_full * (split_lam ? sizeof(float) : sizeof(double))})));
   TRY(dalloc(c, &c->nsX0, nn * sizeof(double)));
   TRY(dalloc(c, &c->nsX1, nn * sizeof(double)));
   TRY(dalloc(c, &c->nsT0, nn * sizeof(double)));
@@ -1087,6 +1091,7 @@ oa_status st_gram(oa_ctx* c, const double2* A, const double2* B, bool sym, doubl
   g.part = c->gpart;
   g.nb = c->nst;
   if (split && c->nst > oa::kGramSmall) {  // FP32 partials in the same buffer
+    if (sym) g.nslice = c->nslice_split;
     float* pf = reinterpret_cast<float*>(c->gpart);
     HIPCHK(oa::gram_bf16(g, pf, c->stream));
     HIPCHK(oa::gram_reduce_f32(pf, g.nslice, c->nst, c->nst, g.sym, 1.0, C, c->stream));
@@ -1408,9 +1413,9 @@ oa_status autotune(oa_ctx* c) {
       if (t_fused >= 0.0 && t_sep >= 0.0 && t_sep < t_fused) c->fuse_rho = false;
     }
   }
+  int& nslice_s = c->nslice_split > 0 ? c->nslice_split : c->nslice_sym;
   tune_knob(
-      c, e0, e1, "S K slices", c->tune_nslice_sym, c->nslice_sym,
-      [&](int v) { c->nslice_sym = v; },
+      c, e0, e1, "S K slices", c->tune_nslice_sym, nslice_s, [&](int v) { nslice_s = v; },
       [&]() {
         return st_gram(c, c->psi, c->psi, true, 1.0 / std::sqrt(2.0), 1.0, c->S,
                        split_on(c, kSplitS));
