@@ -225,7 +225,13 @@ oa_status oa_get_config(const oa_ctx *ctx, int cfg[8]);
 /* the stored k-vectors in use */
 oa_status oa_get_kvecs(const oa_ctx *ctx, int *kx, int *ky, int *kz);
 
-/* coefficients in/out, [nstates][npts] complex (GStateSlab::packedPlaneData) */
+/* coefficients in/out, [nstates][npts] complex (GStateSlab::packedPlaneData).
+ * The calls return when the copy is done.  Out of the context (oa_psi_get,
+ * oa_force_get), from 8 MiB up and into pageable memory, the data come through
+ * pinned host memory that the first such call allocates and the context keeps
+ * (16 MiB, or four states if those are larger; not in oa_ctx_device_bytes), emptied by
+ * up to eight threads for the time of the copy; pinned and device memory are
+ * copied to directly. */
 oa_status oa_psi_set(oa_ctx *ctx, const double *psi);
 oa_status oa_psi_get(oa_ctx *ctx, double *psi);
 /* V_KS(r) in [Nz][Ny][Nx] (the VksMsg payload, CP_State_RealSpacePlane.C:530-597) */

@@ -1780,6 +1780,8 @@ static bool copy_staged(oa_ctx* c, const double2* dev, double* host, hipError_t*
   const int nthr = std::min({8, (int)std::thread::hardware_concurrency() - 1,
                              (int)(c->npts * sizeof(double2) * c->nst / kStageMin) + 1});
   if (nthr < 2 || !stage_ring(c)) return false;
+  // steps may still be queued: wait for them here, not with the threads polling
+  if ((*err = hipStreamSynchronize(c->stream)) != hipSuccess) return true;
   try {
     Stager s(c, dev, host);
     *err = s.run(nthr);
