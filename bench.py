@@ -60,19 +60,26 @@ def stage_bytes(stage, geo, csz, rsz):
     return bx
 
 
+def v_bytes(geo, csz):
+    """Bytes per point of the V that the R->G plane pass reads: by row class
+    (planes of a multiple of 4 points a side that hold 4 kmax + 1 of them) a
+    copy in the pass's own precision, else the FP64 array."""
+    n = geo["nx"]
+    return csz // 2 if n % 4 == 0 and 4 * geo["kabs"] + 1 <= n else 8
+
+
 def plane_bytes(stage, geo, csz, nst, launch):
     """HBM bytes a two-factor fused plane pass must move (psi(r) stays on
     chip): G->R reads the populated z-lines of every state (n_lines Nz c)
     and writes one rho partial (N doubles) per state chunk; R->G reads and
-    writes the z-lines and reads V (N doubles) once per chunk, and with rho
-    fused into it also writes one rho partial per chunk."""
+    writes the z-lines and reads V (N values, v_bytes each) once per chunk,
+    and with rho fused into it also writes one rho partial per chunk."""
     n = geo["nx"] * geo["ny"] * geo["nz"]
     lines = geo["nlines"] * geo["nz"] * csz
     if stage == "k_plane_g2r":
         return nst * lines + launch["nchunk"] * n * 8
-    if stage == "k_plane_r2g_rho":
-        return 2 * nst * lines + 2 * launch["pcp"] * n * 8
-    return 2 * nst * lines + launch["pcp"] * n * 8
+    v = v_bytes(geo, csz) + (8 if stage == "k_plane_r2g_rho" else 0)
+    return 2 * nst * lines + launch["pcp"] * n * v
 
 
 # options every benchmark context takes (set from the command line)
@@ -134,7 +141,8 @@ def run_precision(sysd, precision, steps, warmup, device=0, use_graph=0, vks=Tru
     last = c.result()
     tim = c.timings()
     last["resid_max"], last["resid_rms"] = c.residual()
-    geo = dict(nx=c.nx, ny=c.ny, nz=c.nz, nlines=c.nlines, nplane_x=c.nplane_x, npts=c.npts)
+    geo = dict(nx=c.nx, ny=c.ny, nz=c.nz, nlines=c.nlines, nplane_x=c.nplane_x, npts=c.npts,
+               kabs=int(max(abs(k).max() for k in (sysd["kx"], sysd["ky"]))))
     psi = c.get_psi()
     cfg = dict(c.config)
     tuning = c.tuning_log()
