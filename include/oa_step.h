@@ -132,7 +132,8 @@ typedef struct {
                           (default): the R->G pass recomputes psi(r) from the z-pass output
                           (no psi(r) buffer; measured faster on MI355X at 100^3: the extra
                           write and read of psi(r) cost more than the y-FFT and x c2r they
-                          replace).  Bit-identical results either way. */
+                          replace).  The same rho either way, forces equal to rounding (the
+                          last bit of a product's sum may be rounded otherwise). */
 } oa_options;
 
 typedef struct {
