@@ -453,8 +453,8 @@ def main():
                          "precision of --serve-precisions) and print its JSON line")
     ap.add_argument("--serve-precisions", default="fp64,mixed")
     ap.add_argument("--ns-mode", type=int, default=None,
-                    help="force the Newton-Schulz kernel (ns_mode option; default: autotuned). "
-                         "1 = one launch per product, no cooperative launch")
+                    help="force the Newton-Schulz kernel (ns_mode option; default 0: plain "
+                         "launches). 1 = one launch per product")
     ap.add_argument("--psir-keep", type=int, default=None,
                     help="psir_keep option: 1 keeps psi(r) between the plane passes, 0 "
                     "recomputes it in the R->G pass (default: the library's, 1)")

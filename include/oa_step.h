@@ -380,8 +380,9 @@ oa_status oa_step_result(oa_ctx *ctx, oa_step_out *out);
  * planes: y+x G->R), [2] x c2r + rho (fused planes: rho reduction),
  * [3] V psi + x r2c (fused planes: V psi, x and y R->G), [4] y-FFT back
  * (fused planes: empty), [5] z-FFT + pack + kinetic force,
- * [6] EKE/E_loc reductions + Lambda (for n <= 128 with the SD update in the
- * same pass), [7] SD (or its |F| reduction) + redundancy sync, [8] S,
+ * [6] Lambda (for n <= 128 with the SD update in the same pass; with use_cg
+ * the direction and update too), [7] SD, redundancy sync and the sums of EKE,
+ * E_loc and |F|^2 (use_cg: empty), [8] S,
  * [9] Newton-Schulz, [10] Psi T, [11] residual, [12] whole step.
  * Fills min(n, OA_NTIMINGS) entries.  oa_set_timing(ctx, 2) records only
  * [3] and [12] and reports 0 for the other entries: every recorded event

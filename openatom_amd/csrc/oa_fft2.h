@@ -74,7 +74,10 @@ constexpr TwTab<R> make_tw() {
 // Rounded to nearest, sqrt(1/2), cos(pi/8), sin(pi/8) and sin(pi/3) all come out
 // 1.6 to 3.1e-8 too small, and the results of every pass with them.  Here each entry
 // takes, of the floats on both sides of its parts, the pair that keeps the sum of
-// the moduli's errors so far nearest to zero.  FP32BIAS
+// the moduli's errors so far nearest to zero.  psi(r) of random coefficients against
+// FP64, cubes of 27 to 160: mean error -6.5 to +5.5e-8 -> -2.8 to +1.2e-8, rms (the mean in
+// it) 1.34 to 1.60e-7 -> 1.31 to 1.59e-7 (less at seven of nine lengths; 1.49 -> 1.55 at 90,
+// 1.50 -> 1.54 at 160), with the radix kernels as they are.
 struct Near {
   double v[2];
 };
@@ -178,7 +181,9 @@ template <typename T, int S>
 struct Dft<T, 3, S> {
   template <bool ONE>
   static __device__ __forceinline__ void run_tw(cpx<T>* v, const cpx<T>* w) {
-    // FP32: 0.866025388 three times and the next float once (see make_tw32)
+    // FP32: 0.866025388 three times and the next float once (see make_tw32).  Outputs
+    // 1 and 2 of a real input are each other's conjugates but for this ulp, 6e-8 d.x, as
+    // much as one rounding of the sum.
     const T h = (T)S * (T)0.86602540378443864676;
     const T h1 = sizeof(T) == 4 ? (T)S * (T)0.866025447845458984 : h;
     cpx<T> t1, d;

@@ -2018,7 +2018,7 @@ hipError_t ns_run(const NsArgs& a, hipStream_t st) {
   if (!a.coop) return ns_run_launches(a, st);
   if (a.coop == kNsStepsKind) return ns_run_steps(a, st);
   if (a.coop == kNsOneKind) {
-    if (a.n > kNsOneMax) return ns_run_launches(a, st);
+    if (a.n > kNsOneMax) return hipErrorInvalidValue;  // X, T and C would not fit in LDS
     const hipError_t e = grant_lds((const void*)k_ns_one, kNsOneSmem);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_ns_one, dim3(1), dim3(ns_one_threads(a.n)), kNsOneSmem, st, a);

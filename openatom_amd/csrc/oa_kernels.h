@@ -202,9 +202,9 @@ struct VksArgs {
   int nbx, nbl;            // set by vks_build
   StepDev* res;
 };
-// workgroup counts of the x and line passes
 // one two-factor pass, n the length of its axis
 hipError_t vks2_launch(int kind, int n, const VksArgs& a, hipStream_t st);
+// workgroup counts of the x and line passes (two-factor: of k_rho_xc and the lines)
 int vks_nbx(const VksArgs& a);
 int vks_nbl(const VksArgs& a);
 size_t vks_smem(const VksArgs& a);  // largest dynamic LDS of the passes
@@ -221,13 +221,13 @@ struct PseudoDev {
 hipError_t vloc_build(const VksArgs& a, const PseudoDev& p, double2* vloc, hipStream_t st);
 
 // ---- dense linear algebra (oa_gemm.hip) ----
+constexpr int kGramSmall = 64;  // states up to which a wave takes a whole gram
 // part[sp][i][j] = sum_{k in slice sp} w(k) A[i][k] B[j][k]; A, B are [n][lda]
 // rows of K reals (lda a multiple of 4, rows 32-byte aligned); w(k) = w_lo
 // for k < k_lo else w_hi.  Every output block is split into nslice
 // K slices (slices never straddle k_lo).  sym: B == A, only the 16 x 16
 // tiles with i/16 <= j/16 are computed.
 // C[i][j] = sum_k w(k) A[i][k] B[j][k], i < n, j < nb (nb == n when sym)
-constexpr int kGramSmall = 64;  // states up to which a wave takes a whole gram
 struct GramArgs {
   const double* A;
   const double* B;
@@ -302,7 +302,7 @@ struct NsArgs {
              // tiles (two grid barriers per iteration); 2, 3, 4: one cooperative launch
              // over 16-row blocks, each split over 1, 2 or 4 workgroups by column
              // tiles (one barrier per iteration); kNsOneKind: one workgroup, a plain
-             // launch, for n <= kNsOneMax (two launches per iteration above);
+             // launch, n <= kNsOneMax;
              // kNsStepsKind: two plain launches per iteration by small tiles for
              // the iterations expected, one more that runs any others
   int hint;  // kNsStepsKind: iterations the last call took, 0 if not known
@@ -358,9 +358,9 @@ hipError_t sd_update(double2* psi, const double2* f, const double* dtm, const in
 // redundant kx=0 points <- conj(partner) (CP_State_GSpacePlane.C:2862-3061)
 hipError_t red_sync(double2* psi, const int* red, const int* partner, int nred, int nst, int ld,
                     hipStream_t st);
-// sum of parts -> res field (deterministic single-workgroup reduction)
-// *out = scale * sum of part[n], up to three sums; cg: the first is |F|^2 of a new
-// conjugate-gradient direction, whose state advances with gamma
+// *out = scale * sum of part[n], up to three sums, a workgroup each, in a fixed order;
+// cg: the first is |F|^2 of a new conjugate-gradient direction, whose state advances
+// with gamma
 struct RedJob {
   const double* part;
   int n;

@@ -908,7 +908,8 @@ oa_status check_range(oa_ctx* c, int s0, int ns) {
 }
 
 // Timing marks inside oa_step: ev[0] start, ev[1..6] after each FFT stage,
-// ev[7] reductions + Lambda, ev[8] SD + sync, ev[9] S, ev[10] NS,
+// ev[7] Lambda, ev[8] SD + sync + sums of EKE, E_loc, |F|^2 (CG: all of it in ev[7]),
+// ev[9] S, ev[10] NS,
 // ev[11] Psi T, ev[12] residual (end).
 // Timing level 2 records only the step's ends and the R->G plane pass
 // (marks 0, 3, 4, 12): each recorded event costs the stream a few

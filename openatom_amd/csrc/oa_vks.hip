@@ -10,8 +10,7 @@
 //                 cp_hart_ext.C:186-330) with E_H and E_ext sums, z FFT back
 //   k_vks_y<+1> : y FFT back -> hx
 //   k_vks_xb    : Hermitian x c2r of row pairs, added to V_xc
-//                 (acceptHartVks, CP_Rho_RealSpacePlane.C:1365-1390); also
-//                 in the lane order of the row-class R->G pass (VPerm)
+//                 (acceptHartVks, CP_Rho_RealSpacePlane.C:1365-1390)
 //   k_vks_sum   : fixed-order reduction of the partial sums into StepDev
 //
 // These passes are plain batched Stockham transforms on LDS, for grids with a length
@@ -358,13 +357,8 @@ __global__ __launch_bounds__(kVT) void k_vks_xb(VksArgs a) {
       const int i = i0 + u * kVT, q = i / a.nx, y = 2 * (p0 + q);
       if (i < cnt2 && q < np) {
         const cpx<double> r = R[i];
-        const int x = i - q * a.nx;
         a.v[i0v[u]] = v0[u] + r.x;
-        if (a.vp.p) a.vp.put(z, y, x, v0[u] + r.x);
-        if (y + 1 < a.ny) {
-          a.v[i1v[u]] = v1[u] + r.y;
-          if (a.vp.p) a.vp.put(z, y + 1, x, v1[u] + r.y);
-        }
+        if (y + 1 < a.ny) a.v[i1v[u]] = v1[u] + r.y;
       }
     }
   }
