@@ -1036,7 +1036,7 @@ __global__ __launch_bounds__(1024) void k_ns_one(NsArgs a) {
       const int q = wave + i * nw, t = q < nt * nt ? q : q - nt * nt;
       if (q >= 2 * nt * nt) continue;
       const int ti = t / nt, tj = t - ti * nt;
-      p[i] = (q < nt * nt ? product(X, C, ti, tj) : product(C, T, ti, tj)) * 0.5;
+      p[i] = product(q < nt * nt ? X : C, q < nt * nt ? C : T, ti, tj) * 0.5;
       if (q >= nt * nt)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
