@@ -504,10 +504,14 @@ oa_status build_layout(oa_ctx* c) {
     c->fuse_rho = rho_ok > 0;
     const int max_r = c->fuse_rho ? std::min(c->nst, kMaxRhoChunks) : c->nst;
     // a rho partial is written and read back: 3.3 us at 100^3, where a unit of
-    // the G->R pass is about 1 us; both scale with the points of a plane
+    // the G->R pass is about 1 us; both scale with the points of a plane.  A workgroup
+    // that has a whole plane and a CU to itself takes longer (6.6 us at 150^3 in FP64,
+    // the partial 8): with the same weight as the others 48 states ran in 3 chunks,
+    // 575 us, where 5 take 520
     const double part = 3e-6 * (double)c->nx * c->ny * c->nz;
-    pick_chunks(c->nz * rowparts, std::max(1, occ_g), ncu, c->nst, kMaxRhoChunks, part, f.cs,
-                f.nchunk);
+    const bool alone = rowparts == 1 && occ_g <= 1;
+    pick_chunks(c->nz * rowparts, std::max(1, occ_g), ncu, c->nst, kMaxRhoChunks,
+                alone ? part / 8 : part, f.cs, f.nchunk);
     pick_chunks(c->nz, std::max(1, c->fuse_rho ? rho_ok : occ_r), ncu, c->nst, max_r,
                 c->fuse_rho ? part : 0.0, f.cs_r, f.nchunk_r);
     c->nzblk = (c->nlines + oa::fft2_ntr(c->nz) - 1) / oa::fft2_ntr(c->nz);
