@@ -383,9 +383,12 @@ template <typename P>
 static hipError_t gram_reduce_t(const P* part, int nslice, int n, int nb, int sym, double alpha,
                                 double* C, hipStream_t st) {
   if (sym && nb != n) return hipErrorInvalidValue;
-  // up to 64 states the product wrote whole tiles in FP64 and the plain sum reads the
-  // mirrored elements again: 4.1 us for 16 states, 7.4 by tiles
-  if (sym && !(sizeof(P) == 8 && n <= kGramSmall)) {
+  // up to 64 states the product wrote whole tiles in FP64, so the plain sum can read the
+  // mirrored elements again: 4.1 us for 16 states, 7.4 by tiles.  Beyond 32 its strided
+  // reads of them cost more than the tiles' turn through LDS: S at 10,324 reals takes
+  // 18.7 us plain and 14.7 by tiles for 40 states, 27.7 and 19.8 for 64 (62,106 reals:
+  // 36.1 and 23.4)
+  if (sym && !(sizeof(P) == 8 && n <= 32)) {
     const int nt = (n + 15) >> 4;
     hipLaunchKernelGGL(k_gram_reduce_sym<P>, dim3(4 * (nt * (nt + 1) / 2)), dim3(1024), 0, st,
                        part, nslice, n, alpha, C);
