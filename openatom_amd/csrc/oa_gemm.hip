@@ -553,22 +553,32 @@ __global__ __launch_bounds__(256, 2) void k_rotate_w(RotArgs a) {
   }
 }
 
-// Waves per workgroup and 16-row tiles per wave for n output rows: the pair
-// that computes the fewest rows past n (9 tiles: 3 x 3, 12: 4 x 3, 16: 4 x 4),
-// then the larger tile per wave; four waves before three, which leave two SIMDs
-// with half the work unless an even number of workgroups shares the CU.
+// Waves per workgroup and 16-row tiles per wave for n output rows and K columns: the
+// pair with the shortest chain of tiles on one SIMD.  ceil(workgroups / CUs) of a CU
+// spread their waves over its four SIMDs; a wave costs its jt tiles and a little for the
+// loads that it does not share (0.1), and the first and the last one of a SIMD run
+// without a neighbour (jt / 2).  Few columns then take small tiles, which leave no CU
+// without a workgroup, and many columns the tiles that compute the fewest rows past n.
+// Over 17 state counts from 129 to 512 and 10 column counts from 1,142 to 252,902 the
+// rule is within 1 % of the fastest pair on average (the fewest rows past n alone: 15 %).
+// Y = M^T X, us, 4 x 4, 4 x 3, 3 x 3, 4 x 2: 256 x 1,142 51, 51, 40, 32; 512 x 17,874
+// 203, 199, 226, 170; 384 x 62,106 380, 308, 357, 303; 144 x 252,902 306, 233, 228, 263;
+// 512 x 252,902 1,964, 2,116, 2,235, 2,064.
 struct RwShape {
   int waves, jt, blocks;
 };
-static RwShape rw_shape(int n) {
-  const int nt = (n + 15) / 16;
-  RwShape best{4, 4, (nt + 15) / 16};
-  int waste = best.blocks * 16;
-  const int cand[3][2] = {{4, 3}, {3, 3}, {4, 2}};
+static RwShape rw_shape(int n, int K) {
+  const int nt = (n + 15) / 16, ncu = cu_count();
+  RwShape best{};
+  long long low = -1;
+  const int cand[4][2] = {{4, 4}, {4, 3}, {3, 3}, {4, 2}};
   for (const auto& c : cand) {
     const int per = c[0] * c[1], blocks = (nt + per - 1) / per;
-    if (blocks * per < waste) {
-      waste = blocks * per;
+    const long long wgs = (long long)((K + kRK - 1) / kRK) * blocks;
+    const long long waves = ((wgs + ncu - 1) / ncu * c[0] + 3) / 4;  // of one SIMD
+    const long long cost = waves * (10 * c[1] + 1) + 5 * c[1];
+    if (low < 0 || cost < low) {
+      low = cost;
       best = {c[0], c[1], blocks};
     }
   }
@@ -753,7 +763,7 @@ static int rotate_pgrid(int K) {
 }
 
 int rotate_nwg(int n, int K) {
-  return n <= 128 ? rotate_pgrid(K) : ((K + kRK - 1) / kRK) * rw_shape(n).blocks;
+  return n <= 128 ? rotate_pgrid(K) : ((K + kRK - 1) / kRK) * rw_shape(n, K).blocks;
 }
 
 hipError_t rotate_f64(const RotArgs& args, hipStream_t st) {
@@ -778,7 +788,7 @@ hipError_t rotate_f64(const RotArgs& args, hipStream_t st) {
     return hipGetLastError();
   }
   if (a.ldx % kRK) return hipErrorInvalidValue;  // whole 64-column blocks inside a row
-  const RwShape sh = rw_shape(a.n);
+  const RwShape sh = rw_shape(a.n, a.K);
   const bool y = a.beta != 0.0;
   void (*const fn)(RotArgs) = sh.jt == 4   ? (y ? k_rotate_w<4, true> : k_rotate_w<4, false>)
                               : sh.jt == 3 ? (y ? k_rotate_w<3, true> : k_rotate_w<3, false>)
