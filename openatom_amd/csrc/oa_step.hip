@@ -219,12 +219,14 @@ struct oa_ctx {
   std::string tune_log;
   // non-local KB pseudopotential (oa_nonlocal_set): projector table, the
   // projections Z, their scaled transpose and the gram partials
-  int nl_natm = 0, nl_cap = 0, nl_nslice = 0;  // atoms set, atoms allocated, K slices
+  int nl_natm = 0, nl_cap = 0;                 // atoms set, atoms allocated
+  int nl_nslice[2] = {};                       // K slices of Z, of Z with its derivatives
+  size_t nl_part_len = 0;                      // doubles
   double* nl_sf = nullptr;    // [4 nl_cap][2 ld]: rows of oa::nl_sf_build
   double* nl_z = nullptr;     // [nst][4 nl_cap]
   double* nl_mt = nullptr;    // [nl_cap][nst]
   double* nl_vn = nullptr;    // [nl_cap] vnorm / Omega per atom
-  double* nl_part = nullptr;  // [nl_nslice][nst][4 nl_cap]
+  double* nl_part = nullptr;  // partial sums of either product, [slice][nst][columns]
   double* nl_fatm = nullptr;  // [nl_cap][3]
 };
 
@@ -1196,7 +1198,7 @@ oa_status st_nl_z(oa_ctx* c, bool derivs) {
   g.w_lo = 1.0;
   g.w_hi = 2.0;
   g.sym = 0;
-  g.nslice = c->nl_nslice;
+  g.nslice = c->nl_nslice[derivs];
   g.part = c->nl_part;
   HIPCHK(oa::gram_f64(g, c->stream));
   HIPCHK(oa::gram_reduce(c->nl_part, g.nslice, c->nst, g.nb, 0, 1.0, c->nl_z, c->stream));
@@ -1926,21 +1928,30 @@ oa_status oa_nonlocal_set(oa_ctx* c, const oa_nonlocal* nl) {
   HIPCHK(hipSetDevice(c->device));
   HIPCHK(hipStreamSynchronize(c->stream));
   const int na = nl->natoms;
+  int ncu = 0;
+  if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) !=
+          hipSuccess || ncu <= 0)
+    ncu = 256;
+  // Z has na columns, with its derivatives 4 na: a count of K slices each.  The wider
+  // product's count for both left CUs idle: one call for Z of 128 states x 21 atoms x
+  // 62,106 reals 81 -> 66 us, 256 x 21 131 -> 83
+  int ns[2];
+  size_t len[2];
+  for (int d = 0; d < 2; d++) {
+    ns[d] = oa::gram_slices(c->nst, d ? 4 * na : na, 2 * c->npts, 0, ncu);
+    len[d] = (size_t)c->nst * (d ? 4 * na : na);
+  }
   if (na > c->nl_cap) {  // buffers for this many atoms (kept until destroy)
     const int ldr = 2 * c->ld;
-    int ncu = 0;
-    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) !=
-            hipSuccess || ncu <= 0)
-      ncu = 256;
-    const int ns = oa::gram_slices(c->nst, 4 * na, 2 * c->npts, 0, ncu);
+    const size_t part = std::max(ns[0] * len[0], ns[1] * len[1]);
     TRY(dalloc(c, &c->nl_sf, (size_t)4 * na * ldr * sizeof(double)));
     TRY(dalloc(c, &c->nl_z, (size_t)c->nst * 4 * na * sizeof(double)));
     TRY(dalloc(c, &c->nl_mt, (size_t)na * c->nst * sizeof(double)));
     TRY(dalloc(c, &c->nl_vn, (size_t)na * sizeof(double)));
-    TRY(dalloc(c, &c->nl_part, (size_t)ns * c->nst * 4 * na * sizeof(double)));
+    TRY(dalloc(c, &c->nl_part, part * sizeof(double)));
     TRY(dalloc(c, &c->nl_fatm, (size_t)na * 3 * sizeof(double)));
     c->nl_cap = na;
-    c->nl_nslice = ns;
+    c->nl_part_len = part;
   }
   // the table of this atom set, rows [4 na][2 ld] (padding points zero)
   const size_t ldr = 2 * (size_t)c->ld;
@@ -1986,6 +1997,9 @@ oa_status oa_nonlocal_set(oa_ctx* c, const oa_nonlocal* nl) {
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   HIPCHK(e);
   c->nl_natm = na;
+  // fewer atoms than the buffers hold: as many slices as fit (two at least, as for more)
+  for (int d = 0; d < 2; d++)
+    c->nl_nslice[d] = (int)std::min<size_t>(ns[d], c->nl_part_len / len[d]);
   drop_graphs(c);  // captured steps lack (or hold the old) non-local stage
   return OA_OK;
 }
