@@ -92,7 +92,7 @@ constexpr int kGramRing = 3;
 
 // Output block of MT x NT tiles from tile (ti0, tj0) (DIAG: the upper ones of a
 // diagonal block of a symmetric product): each wave holds all of it for every fourth
-// chunk of the slice, and the four waves' sums meet in LDS (2 x SM doubles).
+// chunk of the slice, and the four waves' sums meet in LDS (4 x SM doubles).
 template <int MT, int NT, bool DIAG, int SM>
 __device__ __forceinline__ void gram_block(const GramArgs& a, const double* __restrict__ B,
                                            const GSlice& s, int sp, int ti0, int tj0,
@@ -137,33 +137,29 @@ __device__ __forceinline__ void gram_block(const GramArgs& a, const double* __re
           mfmas(m.f);
         }
       });
-  // waves 2, 3 -> 0, 1; wave 1 -> 0
-#pragma unroll
-  for (int half = 2; half >= 1; half--) {
-    if (wave >= half && wave < 2 * half) {
-#pragma unroll
-      for (int t = 0; t < NTW; t++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) sm[wave - half][(4 * t + v) * 64 + lane] = acc[t][v];
-    }
-    __syncthreads();
-    if (wave < half) {
-#pragma unroll
-      for (int t = 0; t < NTW; t++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) acc[t][v] += sm[wave][(4 * t + v) * 64 + lane];
-    }
-    __syncthreads();
-  }
-  if (wave != 0) return;
-  double* part = a.part + (size_t)sp * a.n * a.nb;
+  // Tile t is summed and stored by wave t & 3, in the order (0 + 2) + (1 + 3) whichever
+  // wave it is: one barrier.  By halves to wave 0, which then stored everything, were
+  // three more: S of 33, 64, 128, 256 states x 10,324 reals 16.2, 21.2, 23.6, 43.7 us
+  // then, 15.1, 19.7, 21.9, 41.2 now; 256 x 62,106 138 and 136
   static_for<0, NTW>([&](auto tc) __attribute__((always_inline)) {
     constexpr int t = decltype(tc)::value;
+    if (wave != (t & 3)) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) sm[wave][(4 * t + v) * 64 + lane] = acc[t][v];
+    }
+  });
+  __syncthreads();
+  double* part = a.part + (size_t)sp * a.n * a.nb;
+  static_for<0, NTW>([&](auto tc) __attribute__((always_inline)) {
+    constexpr int t = decltype(tc)::value, o = t & 3;
     constexpr int ti = DIAG ? up_i(t, NT) : t / NT, tj = DIAG ? up_j(t, NT) : t % NT;
+    if (wave != o) return;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
+      const int e = (4 * t + v) * 64 + lane;
+      const double d = (acc[t][v] + sm[o ^ 2][e]) + (sm[o ^ 1][e] + sm[o ^ 3][e]);
       const int r = 16 * (ti0 + ti) + g + 4 * v, col = 16 * (tj0 + tj) + l16;
-      if (r < a.n && col < a.nb) part[(size_t)r * a.nb + col] = s.w * acc[t][v];
+      if (r < a.n && col < a.nb) part[(size_t)r * a.nb + col] = s.w * d;
     }
   });
 }
@@ -178,7 +174,7 @@ __device__ __forceinline__ void gram_block(const GramArgs& a, const double* __re
 // from 256 states up, and by the start and end of a slice below.
 template <int NT>
 __global__ __launch_bounds__(256) void k_gram(GramArgs a, int nbe, int nbe_b, int nblk, int nlo) {
-  __shared__ double sm[2][NT * NT * 256];
+  __shared__ double sm[4][NT * NT * 256];
   const int total = gridDim.x, xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
   const int q = total >> 3, r = total & 7;
   const int logical = xcd * q + min(xcd, r) + k;
@@ -217,7 +213,7 @@ __global__ __launch_bounds__(256) void k_gram(GramArgs a, int nbe, int nbe_b, in
 // reals, one call, 66 -> 60 us).
 template <int NT>
 __global__ __launch_bounds__(256) void k_gram_nb(GramArgs a, int nblk, int nlo) {
-  __shared__ double sm[2][4 * NT * 256];
+  __shared__ double sm[4][4 * NT * 256];
   const int sp = blockIdx.x / nblk, b = blockIdx.x - sp * nblk;
   gram_block<4, NT, false>(a, a.B, gram_slice(a, sp, nlo), sp, 4 * b, 0, sm);
 }
