@@ -219,6 +219,11 @@ struct oa_ctx {
   std::string tune_log;
   // non-local KB pseudopotential (oa_nonlocal_set): projector table, the
   // projections Z, their scaled transpose and the gram partials
+  struct {  // what the state chunks of the plane passes follow
+    int units, occ_g, occ_r, ncu;
+    double part;  // weight of a rho partial
+    int max_g;    // rho partials allocated
+  } rule = {};
   int nl_natm = 0, nl_cap = 0;                 // atoms set, atoms allocated
   int nl_nslice[2] = {};                       // K slices of Z, of Z with its derivatives
   size_t nl_part_len = 0;                      // doubles
@@ -512,8 +517,10 @@ oa_status build_layout(oa_ctx* c) {
     // 575 us, where 5 take 520
     const double part = 3e-6 * (double)c->nx * c->ny * c->nz;
     const bool alone = rowparts == 1 && occ_g <= 1;
-    pick_chunks(c->nz * rowparts, std::max(1, occ_g), ncu, c->nst, kMaxRhoChunks,
-                alone ? part / 8 : part, f.cs, f.nchunk);
+    c->rule = {c->nz * rowparts, std::max(1, occ_g), std::max(1, occ_r), ncu,
+               alone ? part / 8 : part};
+    pick_chunks(c->rule.units, c->rule.occ_g, ncu, c->nst, kMaxRhoChunks, c->rule.part, f.cs,
+                f.nchunk);
     pick_chunks(c->nz, std::max(1, c->fuse_rho ? rho_ok : occ_r), ncu, c->nst, max_r,
                 c->fuse_rho ? part : 0.0, f.cs_r, f.nchunk_r);
     c->nzblk = (c->nlines + oa::fft2_ntr(c->nz) - 1) / oa::fft2_ntr(c->nz);
@@ -707,6 +714,7 @@ oa_status alloc_state(oa_ctx* c, const double* occ) {
     if (c->fuse_rho)
       np = std::max({np, c->fc.nchunk_r, c->tune_nchunk_r.empty() ? 0 : c->tune_nchunk_r.back()});
     TRY(dalloc(c, &c->fc.rho_part, (size_t)np * N * sizeof(double)));
+    c->rule.max_g = np;
   }
   if (c->engine == kEngPlane) {
     // one state's psi(r) for oa_psir_get; every state's when the passes
@@ -898,8 +906,17 @@ FftCtx range_ctx(oa_ctx* c, int s0, int ns) {
                 (c->fp32 ? 8 : 16);
   f.occ = c->occ + s0;
   f.eke_part = c->eke_part + (size_t)s0 * c->nzblk;
-  f.nchunk = (ns + f.cs - 1) / f.cs;
-  f.nchunk_r = (ns + f.cs_r - 1) / f.cs_r;
+  if (ns < c->nst) {
+    // Chunks of its own: a part of the states in chunks of all states' size leaves CUs
+    // idle.  128 states in four ranges, density and back, us: 54^3 mixed 177 -> 146 and
+    // 170 -> 153, 75^3 FP64 699 -> 344 and 705 -> 582.  68 lengths, state counts and
+    // precisions x 2, 4, 8 ranges: 7 and 15 % on average, from 0.9 (150^3 FP64, 4 states,
+    // where uneven chunks of whole planes happened to fit) to 2.9 times
+    const auto& r = c->rule;
+    pick_chunks(r.units, r.occ_g, r.ncu, ns, std::min(kMaxRhoChunks, r.max_g), r.part, f.cs,
+                f.nchunk);
+    pick_chunks(c->nz, r.occ_r, r.ncu, ns, ns, 0.0, f.cs_r, f.nchunk_r);
+  }
   return f;
 }
 
