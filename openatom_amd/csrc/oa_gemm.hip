@@ -425,7 +425,9 @@ constexpr int kRK = 64;
 // block.  Y = M^T X (and Y += ...): 512 states x 260,992 reals 68 (62) TFLOP/s,
 // 256 x 131,824 50 (47), 180 x 73,600 45 (46); 50 (50), 45 (40), 32 (32) before,
 // with 32 x 64 outputs per wave, 1.5 times the loads per MFMA and Y accessed in
-// 8-byte pieces.  A library product of the first two shapes reaches 71 and 49.
+// 8-byte pieces.  A library product of the first two shapes reaches 71 and 49.  With the
+// tiles of rw_shape, Y = M^T X as a step's stage: 512 x 241,238 67, 256 x 134,952 57,
+// 180 x 75,332 50.
 constexpr int kRwRing = 3;
 
 template <int JT>
