@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256) void k_gram(GramArgs a, int nbe, int nbe_b, in
 }
 
 // nb <= 32 < n (the non-local projections of few atoms): blocks of 64 rows and all
-// columns, the rest as in k_gram.  128 states x 32 atoms x 65,922 reals 61 -> 32 us;
+// columns, the rest as in k_gram.  128 states x 32 atoms x 65,922 reals 61 -> 22 us;
 // before, a wave of a 128-row block had 32 rows for all of K, and too little in flight.
 // From 33 rows: whole blocks of 64 x 64 are 16 tiles for 4 or 8 (64 x 8 atoms x 62,106
 // reals, one call, 66 -> 60 us).
